@@ -40,6 +40,54 @@ __device__ __forceinline__ void st_stream(f32x4* p, f32x4 v) {
 }
 __device__ __forceinline__ f32x4 ld_cached(const f32x4* p) { return *p; }
 
+// Rows of any length and alignment as float4: a dwordx4 access needs dword
+// alignment only, so a row that starts anywhere is read and written 16 bytes
+// a lane like an aligned one, and only its last n % 4 floats go one by one.
+// f: float4 index in a row of n floats.  Past the end loads give 0 and stores
+// nothing.  Ragged = false: rows are whole, 16-byte aligned float4.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool Ragged, bool Stream = true>
+__device__ __forceinline__ f32x4 ld_row4(const float* row, uint32_t f, uint32_t n) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (!Ragged) {
+        if (4 * f < n) {
+            const f32x4* p = reinterpret_cast<const f32x4*>(row) + f;
+            v = Stream ? ld_stream(p) : *p;
+        }
+        return v;
+    }
+    if (4 * f + 4 <= n) {
+        const f32x4_a4* p = reinterpret_cast<const f32x4_a4*>(row + 4 * f);
+        v = Stream ? (f32x4)__builtin_nontemporal_load(p) : (f32x4)*p;
+    } else if (4 * f < n) {
+        v.x = row[4 * f];
+        if (4 * f + 1 < n) v.y = row[4 * f + 1];
+        if (4 * f + 2 < n) v.z = row[4 * f + 2];
+    }
+    return v;
+}
+template <bool Ragged, bool Stream = true>
+__device__ __forceinline__ void st_row4(float* row, uint32_t f, uint32_t n, f32x4 v) {
+    if (!Ragged) {
+        f32x4* p = reinterpret_cast<f32x4*>(row) + f;
+        if (4 * f < n) {
+            if (Stream) st_stream(p, v);
+            else *p = v;
+        }
+        return;
+    }
+    if (4 * f + 4 <= n) {
+        f32x4_a4* p = reinterpret_cast<f32x4_a4*>(row + 4 * f);
+        if (Stream) __builtin_nontemporal_store((f32x4_a4)v, p);
+        else *p = v;
+    } else if (4 * f < n) {
+        row[4 * f] = v.x;
+        if (4 * f + 1 < n) row[4 * f + 1] = v.y;
+        if (4 * f + 2 < n) row[4 * f + 2] = v.z;
+    }
+}
+
 // Exact wave-wide max.  max is order-free, so any reduction tree gives the
 // same bits; NaN operands are dropped like Rust's f32::max.
 __device__ __forceinline__ float wave_max(float v) {

@@ -15,19 +15,24 @@
 // 2 * P * cols * 4 bytes (P = the workgroup count, ~512 for large batches:
 // 2% of the traffic at 16384 x 2048).
 //
-// Vector path (cols % 4 == 0, 16-byte aligned, cols <= 4096):
-//   1. rms_bwd_rows_kernel: a row is split over S = 1, 2 or 4 waves (at
-//      most 4 float4 columns per wave and operand); a workgroup of 4 waves
-//      runs up to 16 row iterations with the next row's loads in flight;
-//      gamma is staged in LDS; each wave's dgamma partial stays in
-//      registers; the row slots' partials are added in a fixed order through
-//      LDS and written as workspace row p = the block index.
-//   2. rms_bwd_reduce_kernel: 8 float4 columns x 64 row slots per block;
-//      every slot adds its partial rows in order (16 loads in flight), then
-//      a fixed-shape tree adds the slots -> dgamma (deterministic).
-// Generic path (any shape): one workgroup per row writes dx and inv[r] to the
-// workspace; then one thread per column folds its dgamma over the rows in
-// the reference's order.
+// Row pass (rms_bwd_rows_kernel, cols <= 16384, any alignment): a row is split
+// over S = 1, 2, 4, 8 or 16 waves (at most 4 float4 columns per wave and
+// operand); a workgroup runs several row iterations with the next row's loads
+// in flight; gamma is staged in LDS; each wave's dgamma partial stays in
+// registers; the row slots' partials are added in a fixed order through LDS
+// and written as partial row p = the block index.  Column pass: 8 float4
+// columns x 64 row slots per block; every slot adds its partial rows in order
+// (16 loads in flight), then a fixed-shape tree adds the slots -> dgamma
+// (deterministic).
+//   * 16-byte aligned rows of whole float4, cols <= 4096: workgroups of 4
+//     waves, up to 16 row iterations, the partial rows in the workspace
+//     (rms_bwd_reduce_kernel).
+//   * other rows: their workspace is one float per row, so the partial rows
+//     wait in the last P rows of dx, and the column pass computes those rows'
+//     dx after it has added them (rms_bwd_finish_kernel).
+// Generic path (longer rows, a single row): one workgroup per row writes dx
+// and inv[r] to the workspace; then one thread per column folds its dgamma
+// over the rows in the reference's order.
 #include <mutex>
 
 #include "common.hpp"
@@ -44,8 +49,10 @@ struct BwArgs {
     const float* g;
     float* dx;
     float* dgamma;
-    float* ws;
+    float* ws;    // caller's or library's scratch
+    float* part;  // P partial dgamma rows of cols floats
     uint64_t rows;
+    uint64_t dx_rows;  // the row pass writes dx for rows r < dx_rows
     uint64_t cols;
     float eps;
     uint32_t rpw;       // row iterations per workgroup (vector path)
@@ -55,31 +62,40 @@ struct BwArgs {
 __device__ __forceinline__ float sum4(f32x4 a) { return (a.x + a.y) + (a.z + a.w); }
 
 // A row is split over S waves (wave w: row slot j = w / S, column part
-// q = w % S, float4 columns (q*NCHW + k)*64 + lane, k < NCHW), so a wave holds
-// at most 4 float4 per operand.  Iteration it of workgroup b takes row
-// (it * P + b) * (4/S) + j (P = the grid size), so each iteration of the grid
+// q = w % S, NCHW chunks of 64 float4), so a wave holds at most 4 float4 per
+// operand.  Long and ragged rows deal the chunks out in turn (k*S + q), so that
+// the waves' shares differ by one chunk at most.  Iteration it of workgroup b takes row
+// (it * P + b) * kSlots + j (P = the grid size), so each iteration of the grid
 // sweeps one contiguous band of rows (measured 89 -> 80 us at 16384 x 2048
-// against giving each workgroup a contiguous block of rows).  Per row, the S waves' partial sums meet in LDS (slot
-// parity double-buffered, one barrier per iteration) and are added in q
-// order.  Each wave keeps its dgamma partial in registers; at the end the
-// row slots' partials are added in j order through LDS and written as
-// workspace row b.
-template <int NCHW, int S>
-__global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) void rms_bwd_rows_kernel(BwArgs a) {
-    constexpr int kSlots = kBwWaves / S;
-    extern __shared__ f32x4 part[];  // [cols4] dgamma combine, then [cols4] gamma
-    f32x4* gam = part + (a.cols >> 2);
-    __shared__ float red[2][kBwWaves][2];
+// against giving each workgroup a contiguous block of rows).  Per row, the S
+// waves' partial sums meet in LDS (slot parity double-buffered, one barrier
+// per iteration) and are added in q order.  Each wave keeps its dgamma partial
+// in registers; at the end the row slots' partials are added in j order
+// through LDS and written as partial row b.  Rows from dx_rows on leave their
+// inv and coeff in ws instead of writing dx.
+// Ragged: rows of any length and alignment (see ld_row4).
+template <int NCHW, int S, int kWaves, bool Ragged>
+__global__ __launch_bounds__(kWave * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
+void rms_bwd_rows_kernel(BwArgs a) {
+    constexpr bool kLong = kWaves != kBwWaves;
+    constexpr int kThreads = kWaves * kWave;
+    constexpr int kSlots = kWaves / S;
+    extern __shared__ f32x4 gam[];  // [cols4]: gamma, then the dgamma combine
+    __shared__ float red[2][kWaves][2];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    // a scalar, so that row addresses live in SGPRs
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int j = wave / S, q = wave % S;
-    const uint32_t cols4 = (uint32_t)(a.cols >> 2);
+    const uint32_t cols = (uint32_t)a.cols;
+    const uint32_t cols4 = (cols + 3) >> 2;
     const float fcols = (float)a.cols;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     // iteration it of block b: row (it * P + b) * slots + j -- the grid sweeps
     // one contiguous band of rows per iteration.
     const uint64_t rstride = (uint64_t)gridDim.x * kSlots;
     const uint64_t rbase = (uint64_t)blockIdx.x * kSlots;
+
+    auto col4 = [&](int k) { return (uint32_t)(kLong ? k * S + q : q * NCHW + k) * kWave + lane; };
 
     f32x4 acc[NCHW];
 #pragma unroll
@@ -91,20 +107,20 @@ __global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) v
         const uint64_t r = rbase + (uint64_t)it * rstride + j;
         const bool live = it < a.rpw && r < a.rows;
         const uint64_t rr = live ? r : 0;
-        const f32x4* xr = reinterpret_cast<const f32x4*>(a.x) + rr * cols4;
-        const f32x4* dr = reinterpret_cast<const f32x4*>(a.dy) + rr * cols4;
+        const float* xr = a.x + rr * cols;
+        const float* dr = a.dy + rr * cols;
 #pragma unroll
         for (int k = 0; k < NCHW; ++k) {
-            const uint32_t f = (uint32_t)(q * NCHW + k) * kWave + lane;
-            xo[k] = (live && f < cols4) ? ld_stream(xr + f) : zero;
-            dout[k] = (live && f < cols4) ? ld_stream(dr + f) : zero;
+            const uint32_t f = col4(k);
+            xo[k] = live ? ld_row4<Ragged>(xr, f, cols) : zero;
+            dout[k] = live ? ld_row4<Ragged>(dr, f, cols) : zero;
         }
     };
     load_row(0, xv, dv);
     // gamma lives in LDS for the whole sweep: its reads are LDS operations,
     // so they neither hold registers nor make a wait for them also wait for
     // the prefetched row.
-    for (uint32_t f = threadIdx.x; f < cols4; f += kBwBlock) gam[f] = reinterpret_cast<const f32x4*>(a.g)[f];
+    for (uint32_t f = threadIdx.x; f < cols4; f += kThreads) gam[f] = ld_row4<Ragged, false>(a.g, f, cols);
     __syncthreads();
     for (uint32_t it = 0; it < a.rpw; ++it) {
         const uint64_t r = rbase + (uint64_t)it * rstride + j;
@@ -114,7 +130,7 @@ __global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) v
         float ss = 0.0f, dot = 0.0f;
 #pragma unroll
         for (int k = 0; k < NCHW; ++k) {
-            const uint32_t f = (uint32_t)(q * NCHW + k) * kWave + lane;
+            const uint32_t f = col4(k);
             ss += sum4(xv[k] * xv[k]);
             dot += sum4((xv[k] * dv[k]) * gam[f < cols4 ? f : 0]);
         }
@@ -138,12 +154,20 @@ __global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) v
         const float inv = 1.0f / sqrtf(ss / fcols + a.eps);
         const float coeff = (dot * inv) / (ss + a.eps * fcols);
         if (live) {
-            f32x4* orow = reinterpret_cast<f32x4*>(a.dx) + r * cols4;
+#pragma unroll
+            for (int k = 0; k < NCHW; ++k) acc[k] = acc[k] + (dv[k] * xv[k]) * inv;
+        }
+        if (kLong && live && r >= a.dx_rows) {  // dx from rms_bwd_finish_kernel
+            if (q == 0 && lane == 0) {
+                a.ws[r - a.dx_rows] = inv;
+                a.ws[r - a.dx_rows + (a.rows - a.dx_rows)] = coeff;
+            }
+        } else if (live) {
+            float* orow = a.dx + r * cols;
 #pragma unroll
             for (int k = 0; k < NCHW; ++k) {
-                const uint32_t f = (uint32_t)(q * NCHW + k) * kWave + lane;
-                if (f < cols4) st_stream(orow + f, (gam[f] * inv) * dv[k] - coeff * xv[k]);
-                acc[k] = acc[k] + (dv[k] * xv[k]) * inv;
+                const uint32_t f = col4(k);
+                if (f < cols4) st_row4<Ragged>(orow, f, cols, (gam[f] * inv) * dv[k] - coeff * xv[k]);
             }
         }
 #pragma unroll
@@ -152,20 +176,22 @@ __global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) v
             dv[k] = dn[k];
         }
     }
-    // Row slots' partials added in j order through LDS, then one partial row.
+    // Row slots' partials added in j order through LDS (gamma is done with),
+    // then one partial row.
+    __syncthreads();
 #pragma unroll 1
     for (int jj = 0; jj < kSlots; ++jj) {
         if (j == jj) {
 #pragma unroll
             for (int k = 0; k < NCHW; ++k) {
-                const uint32_t f = (uint32_t)(q * NCHW + k) * kWave + lane;
-                if (f < cols4) part[f] = (jj == 0) ? acc[k] : part[f] + acc[k];
+                const uint32_t f = col4(k);
+                if (f < cols4) gam[f] = (jj == 0) ? acc[k] : gam[f] + acc[k];
             }
         }
         __syncthreads();
     }
-    f32x4* wrow = reinterpret_cast<f32x4*>(a.ws) + (uint64_t)blockIdx.x * cols4;
-    for (uint32_t f = threadIdx.x; f < cols4; f += kBwBlock) wrow[f] = part[f];
+    float* prow = a.part + (uint64_t)blockIdx.x * cols;
+    for (uint32_t f = threadIdx.x; f < cols4; f += kThreads) st_row4<Ragged, false>(prow, f, cols, gam[f]);
 }
 
 // dgamma = sum of the P partial rows, deterministic: block = 8 float4
@@ -176,13 +202,10 @@ __global__ __launch_bounds__(kBwBlock) __attribute__((amdgpu_waves_per_eu(4))) v
 constexpr int kRedCols = 8;
 constexpr int kRedSlots = 64;
 constexpr int kRedBatch = 16;
-__global__ __launch_bounds__(kRedCols * kRedSlots) void rms_bwd_reduce_kernel(BwArgs a) {
+template <bool Ragged>
+__device__ __forceinline__ void reduce_partials(const BwArgs& a, int c, int slot, uint64_t col) {
     __shared__ f32x4 red[kRedSlots][kRedCols];
-    const uint64_t cols4 = a.cols >> 2;
-    const int c = threadIdx.x % kRedCols;
-    const int slot = threadIdx.x / kRedCols;
-    const uint64_t col = (uint64_t)blockIdx.x * kRedCols + c;
-    const f32x4* w4 = reinterpret_cast<const f32x4*>(a.ws);
+    const uint64_t cols4 = (a.cols + 3) >> 2;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 t = zero;
     if (col < cols4) {
@@ -191,7 +214,9 @@ __global__ __launch_bounds__(kRedCols * kRedSlots) void rms_bwd_reduce_kernel(Bw
 #pragma unroll
             for (int u = 0; u < kRedBatch; ++u) {
                 const uint64_t p = p0 + (uint64_t)u * kRedSlots;
-                v[u] = p < a.partials ? w4[p * cols4 + col] : zero;
+                v[u] = p < a.partials
+                           ? ld_row4<Ragged, false>(a.part + p * a.cols, (uint32_t)col, (uint32_t)a.cols)
+                           : zero;
             }
 #pragma unroll
             for (int u = 0; u < kRedBatch; ++u) {
@@ -206,7 +231,46 @@ __global__ __launch_bounds__(kRedCols * kRedSlots) void rms_bwd_reduce_kernel(Bw
         if (slot < w) red[slot][c] = red[slot][c] + red[slot + w][c];
         __syncthreads();
     }
-    if (slot == 0 && col < cols4) reinterpret_cast<f32x4*>(a.dgamma)[col] = red[0][c];
+    if (slot == 0 && col < cols4)
+        st_row4<Ragged, false>(a.dgamma, (uint32_t)col, (uint32_t)a.cols, red[0][c]);
+}
+
+__global__ __launch_bounds__(kRedCols * kRedSlots) void rms_bwd_reduce_kernel(BwArgs a) {
+    const int c = threadIdx.x % kRedCols, slot = threadIdx.x / kRedCols;
+    reduce_partials<false>(a, c, slot, (uint64_t)blockIdx.x * kRedCols + c);
+}
+
+// The same, and then dx of the last rows, which held the partials: a block
+// owns its columns of all of them, so after the reduction's barriers nothing
+// reads what it overwrites.  inv and coeff of those rows come from ws.
+constexpr int kFinBatch = 4;  // rows a thread has in flight
+template <bool Ragged>
+__global__ __launch_bounds__(kRedCols * kRedSlots) void rms_bwd_finish_kernel(BwArgs a) {
+    const int c = threadIdx.x % kRedCols, slot = threadIdx.x / kRedCols;
+    const uint64_t col = (uint64_t)blockIdx.x * kRedCols + c;
+    const uint32_t cols = (uint32_t)a.cols;
+    // gamma before dgamma is written: the two may be the same buffer
+    const f32x4 g = ld_row4<Ragged, false>(a.g, (uint32_t)col, cols);
+    reduce_partials<Ragged>(a, c, slot, col);
+    if (4 * col >= a.cols) return;
+    const uint64_t tail = a.rows - a.dx_rows;
+    for (uint64_t p0 = slot; p0 < tail; p0 += kFinBatch * kRedSlots) {
+        f32x4 x[kFinBatch], d[kFinBatch];
+#pragma unroll
+        for (int u = 0; u < kFinBatch; ++u) {
+            const uint64_t p = p0 + (uint64_t)u * kRedSlots;
+            if (p >= tail) continue;
+            x[u] = ld_row4<Ragged>(a.x + (a.dx_rows + p) * cols, (uint32_t)col, cols);
+            d[u] = ld_row4<Ragged>(a.dy + (a.dx_rows + p) * cols, (uint32_t)col, cols);
+        }
+#pragma unroll
+        for (int u = 0; u < kFinBatch; ++u) {
+            const uint64_t p = p0 + (uint64_t)u * kRedSlots;
+            if (p >= tail) continue;
+            const float inv = a.ws[p], coeff = a.ws[p + tail];
+            st_row4<Ragged>(a.dx + (a.dx_rows + p) * cols, (uint32_t)col, cols, (g * inv) * d[u] - coeff * x[u]);
+        }
+    }
 }
 
 // ---- generic path
@@ -259,20 +323,17 @@ __global__ __launch_bounds__(kBwBlock) void fill_zero_kernel(float* p, uint64_t 
     if (i < n) p[i] = 0.0f;
 }
 
-static bool bwd_vec(uint64_t cols) { return cols % 4 == 0 && cols / 4 <= 1024; }
-
-// Waves per row for the vector path: each wave holds <= 4 float4 columns.
+// Waves per row: each wave holds <= 4 float4 columns.
 static uint32_t bwd_split(uint64_t cols) {
-    const uint64_t c4 = cols / 4;
-    return c4 <= 256 ? 1u : (c4 <= 512 ? 2u : 4u);
+    const uint64_t c4 = (cols + 3) / 4;
+    return c4 <= 256 ? 1u : (c4 <= 512 ? 2u : (c4 <= 1024 ? 4u : (c4 <= 2048 ? 8u : 16u)));
 }
 
-
-// Row iterations per workgroup: ~512 workgroups (4 waves each, two per SIMD,
-// with the next row's loads in flight) -- measured against 256, 384, 768 and
-// 1024 at 16384 x 2048: fewer partial rows to reduce, and enough waves to keep
-// HBM busy (70.0 vs 72.7 us at 1024); at most 16 iterations so that large
-// batches keep few partial rows.
+// Row iterations per workgroup, up to 4096 columns: ~512 workgroups (4 waves
+// each, two per SIMD, with the next row's loads in flight) -- measured against
+// 256, 384, 768 and 1024 at 16384 x 2048: fewer partial rows to reduce, and
+// enough waves to keep HBM busy (70.0 vs 72.7 us at 1024); at most 16
+// iterations so that large batches keep few partial rows.
 static uint32_t bwd_iters(uint64_t rows, uint32_t split) {
     const uint64_t per_iter = kBwWaves / split;
     uint64_t it = (rows + 512 * per_iter - 1) / (512 * per_iter);
@@ -281,22 +342,45 @@ static uint32_t bwd_iters(uint64_t rows, uint32_t split) {
     return (uint32_t)it;
 }
 
-// Workspace floats for the vector and generic plans (the larger is required).
-static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols, uint64_t* partials, uint32_t* iters) {
+// Workspace floats: the partial rows for whole float4 rows of up to 4096
+// columns, else one float per row.
+static bool bwd_ws_plan(uint64_t cols) { return cols % 4 == 0 && cols / 4 <= 1024; }
+static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols) {
+    if (!bwd_ws_plan(cols)) return rows;
     const uint32_t split = bwd_split(cols);
-    const uint32_t it = bwd_iters(rows, split);
-    const uint64_t rpb = (uint64_t)it * (kBwWaves / split);  // rows per block = per partial row
-    const uint64_t p = (rows + rpb - 1) / rpb;
-    if (partials) *partials = p;
-    if (iters) *iters = it;
-    const uint64_t vec = bwd_vec(cols) ? p * cols : 0;
+    const uint64_t rpb = (uint64_t)bwd_iters(rows, split) * (kBwWaves / split);  // rows per block = per partial row
+    const uint64_t vec = (rows + rpb - 1) / rpb * cols;
     return vec > rows ? vec : rows;
 }
 
 template <int NCHW, int S>
 static void launch_rows(const BwArgs& a, hipStream_t s) {
-    const size_t lds = 2 * (a.cols / 4) * sizeof(f32x4);
-    hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S>), dim3((uint32_t)a.partials), dim3(kBwBlock), lds, s, a);
+    const size_t lds = a.cols / 4 * sizeof(f32x4);
+    hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwWaves, false>), dim3((uint32_t)a.partials), dim3(kBwBlock), lds,
+                       s, a);
+}
+
+// Long and ragged rows (up to 16384 columns): workgroups of 16 waves, one per
+// CU, so that the fewest partial rows (whose rows of dx are read and written
+// again at the end) keep every SIMD at four waves.  Measured, rows x columns:
+// 4096 x 8192 85.5 us (4.7 TB/s; one workgroup per row and one thread per
+// dgamma column before: 1740), 4096 x 8191 108 (1753), 8000 x 2049 57 (2770),
+// 2048 x 14336 82 (966); with 512 workgroups of 8 waves 90, 110, 62 and 96,
+// 256 of 8 86, 117, 67 and 82, 128 of 16 110, 134, 76 and 96.  Rows of whole
+// float4 up to 4096 columns keep the workspace plan (8192 x 4096 74 us, 5.4
+// TB/s: no row is done twice).
+constexpr int kBwLongWaves = 16;
+constexpr uint64_t kBwLongBlocks = 256;
+
+template <int NCHW, int S>
+static void launch_long(const BwArgs& a, bool ragged, hipStream_t s) {
+    constexpr int W = S > kBwLongWaves ? S : kBwLongWaves;
+    const size_t lds = (a.cols + 3) / 4 * sizeof(f32x4);
+    const dim3 grid((uint32_t)a.partials), block(W * kWave);
+    if (ragged)
+        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, true>), grid, block, lds, s, a);
+    else
+        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, false>), grid, block, lds, s, a);
 }
 
 // Library-held scratch for the allocation-free entry point: the dgamma
@@ -347,7 +431,7 @@ extern "C" uint64_t kore_hip_rms_norm_backward_workspace_bytes(uint64_t rows, ui
     if (rows == 0 || cols == 0) return 0;
     uint64_t elems;
     if (!mul_ok(rows, cols, &elems) || elems > kMaxElements) return 0;
-    return bwd_ws_floats(rows, cols, nullptr, nullptr) * sizeof(float);
+    return bwd_ws_floats(rows, cols) * sizeof(float);
 }
 
 // The whole entry point once the workspace is known.  ws == nullptr asks for
@@ -368,8 +452,8 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
     if (!grad_out || !x || !grad_x || (!own_scratch && !workspace)) return KORE_HIP_ERR_NULL_PTR;
     uint64_t elems;
     if (!mul_ok(rows, cols, &elems) || elems > kMaxElements || rows > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-    BwArgs a{grad_out, x, gamma, grad_x, grad_gamma, workspace, rows, cols, eps, 0, 0};
-    const uint64_t need = bwd_ws_floats(rows, cols, &a.partials, &a.rpw) * sizeof(float);
+    BwArgs a{grad_out, x, gamma, grad_x, grad_gamma, workspace, nullptr, rows, rows, cols, eps, 0, 0};
+    const uint64_t need = bwd_ws_floats(rows, cols) * sizeof(float);
     if (own_scratch) {
         if (need > kBwScratchBytes) return KORE_HIP_ERR_SCRATCH;
         workspace_bytes = kBwScratchBytes;
@@ -388,10 +472,15 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         if (st != KORE_HIP_OK) return st;
         workspace = a.ws;
     }
-    const bool vec = bwd_vec(cols) && aligned16(grad_out) && aligned16(x) && aligned16(gamma) &&
-                     aligned16(grad_x) && aligned16(grad_gamma) && aligned16(workspace);
-    if (vec) {
-        const uint64_t cols4 = cols / 4;
+    const uint64_t cols4 = (cols + 3) / 4;
+    const bool aligned = cols % 4 == 0 && aligned16(grad_out) && aligned16(x) && aligned16(gamma) &&
+                         aligned16(grad_x) && aligned16(grad_gamma) && aligned16(workspace);
+    const uint32_t split = bwd_split(cols);
+    if (aligned && bwd_ws_plan(cols)) {
+        a.rpw = bwd_iters(rows, split);
+        const uint64_t rpb = (uint64_t)a.rpw * (kBwWaves / split);
+        a.partials = (rows + rpb - 1) / rpb;
+        a.part = a.ws;
         if (cols4 <= 64) launch_rows<1, 1>(a, s);
         else if (cols4 <= 128) launch_rows<2, 1>(a, s);
         else if (cols4 <= 256) launch_rows<4, 1>(a, s);
@@ -399,6 +488,35 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         else launch_rows<4, 4>(a, s);
         hipLaunchKernelGGL(rms_bwd_reduce_kernel, dim3((uint32_t)((cols4 + kRedCols - 1) / kRedCols)),
                            dim3(kRedCols * kRedSlots), 0, s, a);
+    } else if (cols <= 16384 && rows > 1) {
+        // The workspace of these shapes holds one float per row, so the P
+        // partial rows wait in dx's last P rows until the second launch has
+        // reduced them and computes those rows' dx; 2 P <= rows, the inv and
+        // coeff it needs being the workspace's first 2 P floats.
+        const uint64_t slots = split > (uint32_t)kBwLongWaves ? 1 : (uint32_t)kBwLongWaves / split;
+        uint64_t rpb = (rows + kBwLongBlocks - 1) / kBwLongBlocks;
+        if (rpb < 2) rpb = 2;
+        rpb = (rpb + slots - 1) / slots * slots;
+        a.rpw = (uint32_t)(rpb / slots);
+        a.partials = (rows + rpb - 1) / rpb;
+        if (2 * a.partials > rows) a.partials = rows / 2;  // one row more for some workgroup
+        while (a.partials * rpb < rows) a.rpw += 1, rpb += slots;
+        a.dx_rows = rows - a.partials;
+        a.part = grad_x + a.dx_rows * cols;
+        if (cols4 <= 64) launch_long<1, 1>(a, !aligned, s);
+        else if (cols4 <= 128) launch_long<2, 1>(a, !aligned, s);
+        else if (cols4 <= 256) launch_long<4, 1>(a, !aligned, s);
+        else if (cols4 <= 512) launch_long<4, 2>(a, !aligned, s);
+        else if (cols4 <= 1024) launch_long<4, 4>(a, !aligned, s);
+        else if (cols4 <= 1536) launch_long<3, 8>(a, !aligned, s);
+        else if (cols4 <= 2048) launch_long<4, 8>(a, !aligned, s);
+        else if (cols4 <= 3072) launch_long<3, 16>(a, !aligned, s);
+        else launch_long<4, 16>(a, !aligned, s);
+        const dim3 grid((uint32_t)((cols4 + kRedCols - 1) / kRedCols)), block(kRedCols * kRedSlots);
+        if (aligned)
+            hipLaunchKernelGGL(rms_bwd_finish_kernel<false>, grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL(rms_bwd_finish_kernel<true>, grid, block, 0, s, a);
     } else {
         hipLaunchKernelGGL(rms_bwd_row_generic_kernel, dim3((uint32_t)rows), dim3(kBwBlock), 0, s, a);
         hipLaunchKernelGGL(rms_bwd_col_generic_kernel, dim3((uint32_t)((cols + kBwBlock - 1) / kBwBlock)),

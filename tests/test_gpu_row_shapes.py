@@ -1,0 +1,79 @@
+"""Row kernels on long and ragged rows: lengths around each change of plan,
+views at every 4-byte offset, against the oracle (bit-exact where the entry
+point is) with the tolerances of test_gpu_parity.py."""
+import numpy as np
+import pytest
+
+import oracle
+from inputs import assert_close_scaled, normal, rmsnorm_inputs
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from kore_amd import rocm  # noqa: E402
+from kore_amd.rocm import HipBuffer  # noqa: E402
+
+DEV = 0
+U32 = 2.0 ** -24
+
+
+def at(arr: np.ndarray, offset: int) -> HipBuffer:
+    """arr on the device, starting `offset` floats past a 16-byte boundary."""
+    flat = np.ascontiguousarray(arr).reshape(-1)
+    t = torch.empty(flat.size + 8, dtype=torch.from_numpy(flat).dtype, device="cuda:0")
+    v = t[offset:offset + flat.size]
+    v.copy_(torch.from_numpy(flat))
+    return HipBuffer.from_tensor(v)
+
+
+def room(n: int, offset: int):
+    """A NaN-filled buffer of n floats at `offset`, and the whole allocation, whose guards must stay NaN."""
+    t = torch.full((n + 16,), float("nan"), device="cuda:0")
+    return HipBuffer.from_tensor(t[8 + offset - 4:8 + offset - 4 + n]), t, 8 + offset - 4
+
+
+def inside(t, start: int, n: int) -> np.ndarray:
+    h = t.cpu().numpy()
+    assert np.isnan(h[:start]).all() and np.isnan(h[start + n:]).all(), "written outside the output"
+    return h[start:start + n]
+
+
+# One float4 per lane and wave more or less around 256, 512, 1024, 4096, 6144, 8192, 12288 and 16384 columns; 16385 is
+# the generic path's.  Rows: fewer than, and not a multiple of, a workgroup's.
+@pytest.mark.parametrize("rows,cols,offset", [
+    (1, 1, 0), (3, 5, 1), (9, 255, 2), (601, 258, 3), (7, 513, 0), (5, 1021, 1), (513, 1030, 2), (3, 2049, 0),
+    (6, 3071, 3), (1100, 4095, 1), (4, 4096, 1), (3, 4097, 0), (2, 4100, 0), (515, 6143, 2), (2, 6144, 0), (3, 6145, 1),
+    (520, 8192, 0), (2, 8191, 0), (3, 8193, 3), (2, 12288, 0), (2, 12291, 1), (259, 16384, 0), (2, 16383, 2),
+    (2, 16385, 0)])
+def test_rms_norm_backward_long_and_ragged(rows, cols, offset):
+    print(f"rms_norm_backward rows={rows} cols={cols} offset={offset}", flush=True)
+    x, g = rmsnorm_inputs(rows, cols, seed=rows + cols)
+    dy = normal((rows, cols), rows * 3 + cols)
+    dx, dx_all, dx_at = room(rows * cols, offset)
+    dg, dg_all, dg_at = room(cols, offset)
+    ws, ws_all, ws_at = room(rocm.rocm_rms_norm_backward_workspace_bytes(rows, cols) // 4, offset)
+    rocm.rocm_rms_norm_backward_f32(DEV, at(dy, offset), at(x, offset), at(g, offset), rows, cols, 1e-5, ws, dx, dg)
+    torch.cuda.synchronize()
+    inside(ws_all, ws_at, ws.nbytes // 4)
+    dx_w, dg_w = oracle.rms_norm_backward(dy, x, g, 1e-5)
+    x64, dy64, g64 = (a.astype(np.float64) for a in (x, dy, g))
+    inv = 1.0 / np.sqrt((x64 * x64).mean(1, keepdims=True) + 1e-5)
+    terms = np.abs(x64 * dy64 * g64).sum(1, keepdims=True) * inv ** 3 / cols
+    # dx is a difference of two terms, each with a sum of cols (rows for dgamma) roundings on either side
+    assert_close_scaled(inside(dx_all, dx_at, rows * cols).reshape(rows, cols), dx_w,
+                        np.abs(g64 * inv * dy64) + terms * np.abs(x64), rtol=1e-5 + cols * U32, what="dx")
+    assert_close_scaled(inside(dg_all, dg_at, cols), dg_w, np.abs(dy64 * x64 * inv).sum(0), rtol=1e-5 + rows * U32,
+                        what="dgamma")
+
+
+@pytest.mark.parametrize("rows,cols", [(700, 8192), (65, 1001)])
+def test_rms_norm_backward_dgamma_over_gamma(rows, cols):
+    """grad_gamma may be gamma's buffer; every row of dx uses the old gamma."""
+    x, g = rmsnorm_inputs(rows, cols, seed=3)
+    dy = normal((rows, cols), 4)
+    want = rocm.rocm_rms_norm_backward_f32(DEV, at(dy, 0), at(x, 0), at(g, 0), rows, cols, 1e-5)
+    gb = at(g, 0)
+    dx, dg = rocm.rocm_rms_norm_backward_f32(DEV, at(dy, 0), at(x, 0), gb, rows, cols, 1e-5, grad_gamma=gb)
+    torch.cuda.synchronize()
+    assert dx.to_host().tobytes() == want[0].to_host().tobytes()
+    assert dg.to_host()[:cols * 4].tobytes() == want[1].to_host()[:cols * 4].tobytes()

@@ -26,10 +26,13 @@
 // Shapes: a row of up to 1024 floats, or of 2049-4096, is held in one wave's
 // registers (one wave per row, 4 rows per workgroup); 1025-2048 floats and
 // up to 16384 in one workgroup's (256 threads; 512 for the 1025-2048
-// backward); longer rows (vocab-sized) stream through a workgroup in three
-// passes.  Unaligned views and cols % 4 != 0 use the looped kernel with
-// scalar accesses.  Every kernel reads a row fully before writing it, so out
-// may alias an input.
+// backward); up to 135168 (vocabularies) in the registers and LDS of a CU
+// (forward and cross-entropy); still longer rows, and the backward's from
+// 16385, stream through a workgroup in three passes (two).  Rows of any length
+// and alignment take the same kernels, their last cols % 4 floats one by one.
+// Every kernel reads a row fully before writing it, so out may alias an input.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kore_hip_internal.hpp"
 
@@ -100,29 +103,30 @@ __device__ __forceinline__ float block_combine(float v, float* red) {
 // Row in registers.  Wave mode (Block = false): one wave per row, element f4
 // index = c*64 + lane, 4 rows per 256-thread workgroup.  Block mode: one
 // workgroup of BS threads per row, index = c*BS + tid.
-template <SmKind K, int NCH, bool Block, int BS = kSmBlock>
+// Ragged: rows of any length and alignment (ld_row4).  Causal rows read only
+// the float4 that hold a column they keep.
+template <SmKind K, int NCH, bool Block, bool Ragged, int BS = kSmBlock>
 __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
     constexpr int kWavesB = BS / kWave;
     __shared__ float red[kWavesB];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const uint64_t row = Block ? (uint64_t)blockIdx.x : (uint64_t)blockIdx.x * kSmWaves + wave;
     if (!Block && row >= a.rows) return;  // uniform per wave; no block barrier in wave mode
     const int step = Block ? BS : kWave;
     const int me = Block ? (int)threadIdx.x : lane;
-    const uint32_t cols4 = (uint32_t)(a.cols >> 2);      // <= 4096 here
+    const uint32_t cols = (uint32_t)a.cols;               // <= 16384 here
     const uint32_t lim = (uint32_t)row_limit<K>(a, row);  // <= cols
-    const f32x4* ar = reinterpret_cast<const f32x4*>(a.a) + row * cols4;
-    const f32x4* br = reinterpret_cast<const f32x4*>(a.b) + row * cols4;
-    f32x4* orow = reinterpret_cast<f32x4*>(a.out) + row * cols4;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const float* ar = a.a + row * cols;
+    const float* br = a.b + row * cols;
+    float* orow = a.out + row * cols;
 
     f32x4 v[NCH], g[NCH];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const uint32_t f = (uint32_t)(c * step + me);
-        v[c] = f < cols4 ? ld_stream(ar + f) : zero;
-        if (K == SmKind::Bwd) g[c] = f < cols4 ? ld_stream(br + f) : zero;
+        v[c] = ld_row4<Ragged>(ar, f, K == SmKind::Causal && !Ragged ? (lim + 3u) & ~3u : (K == SmKind::Causal ? lim : cols));
+        if (K == SmKind::Bwd) g[c] = ld_row4<Ragged>(br, f, cols);
     }
 
     if (K == SmKind::Bwd) {
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const uint32_t f = (uint32_t)(c * step + me);
-            if (f < cols4) st_stream(orow + f, v[c] * (g[c] - dot));
+            st_row4<Ragged>(orow, f, cols, v[c] * (g[c] - dot));
         }
         return;
     }
@@ -182,15 +186,176 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 if ((uint64_t)(4 * f + k) == t) f4_set(o, k, f4_get(o, k) - inv_batch);
-            if (f < cols4) st_stream(orow + f, o);
+            st_row4<Ragged>(orow, f, cols, o);
         }
         return;
     }
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const uint32_t f = (uint32_t)(c * step + me);
-        if (f < cols4) st_stream(orow + f, v[c] * inv);
+        st_row4<Ragged>(orow, f, cols, v[c] * inv);
     }
+}
+
+// Rows of 16385 to kLongCols floats (vocabularies): one workgroup of 1024
+// threads holds the row, R float4 a thread in registers and the rest in LDS,
+// and reads it once.  A CU's registers and LDS hold one such row, so its own
+// arithmetic has to hide behind its own traffic: while the loads arrive a
+// thread keeps a running max m and s = sum e^(x - m) (rescaled when a group of
+// float4 raises m), and the values are exponentiated a second time, against
+// the row's max, between the stores.  Thread i's float4 c is c * 1024 + i of
+// the row; chunks past R go to LDS, and are loaded first, through the
+// registers that the first chunks' loads then take over.
+// Bound by HBM: 8 bytes a float.  2048 x 128256: 767 us in the loop kernel's
+// three passes, 382 here (5.5 TB/s); x 50257 421 -> 157, x 20000 98 -> 56; 64 x
+// 128256 103 -> 19.  Ragged 16368 x 1023 in the wave kernel 60.5 -> 25.8 us,
+// its backward 49.4 -> 38.4 (whole float4, 16384 x 1024: 22.7 and 31.3).
+constexpr int kLongThreads = 1024;
+constexpr int kLongRegs = 24;   // float4 a thread: 96 of the 128 VGPRs that 16 waves leave
+constexpr int kLongLds = 9;     // float4 a thread: 144 of the 160 KB
+constexpr uint64_t kLongCols = 4ull * kLongThreads * (kLongRegs + kLongLds);
+
+// Running max and sum of a thread's values; columns that take no part are -inf
+// (they add 0).  A thread that has met nothing above -inf keeps s = 0 or NaN:
+// the row's own max decides then.
+struct Online {
+    float m = -__builtin_inff();
+    float s = 0.0f;
+    // N float4; those with in[c] false repeat a value of the row and only leave
+    // the max as it is.
+    template <int N>
+    __device__ __forceinline__ void add(const f32x4* v, const bool* in) {
+        float mn = m;
+#pragma unroll
+        for (int c = 0; c < N; ++c) mn = fmaxf(fmaxf(mn, fmaxf(v[c].x, v[c].y)), fmaxf(v[c].z, v[c].w));
+        s *= m == -__builtin_inff() ? 1.0f : exp_diff(m - mn);
+        m = mn;
+        const float base = mn == -__builtin_inff() ? 0.0f : mn;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            const float t = (exp_diff(v[c].x - base) + exp_diff(v[c].y - base)) +
+                            (exp_diff(v[c].z - base) + exp_diff(v[c].w - base));
+            s += in[c] ? t : 0.0f;
+        }
+        // Used only past the block's barriers: the compiler would sink the
+        // sums there and keep every term in a register until then.
+        asm volatile("" : "+v"(m), "+v"(s));
+    }
+};
+
+template <SmKind K, int R, bool Lds, bool Ragged>
+__global__ __launch_bounds__(kLongThreads) void softmax_long_kernel(SmArgs a) {
+    constexpr int kWavesB = kLongThreads / kWave;
+    constexpr int kPre = Lds ? kLongLds : 0;  // LDS chunks, through v[0 .. kPre)
+    constexpr int kGrp = 4;                   // float4 a rescaling
+    constexpr uint32_t kChunk = 4 * kLongThreads;
+    extern __shared__ f32x4 keep[];  // [LDS chunks][thread]
+    __shared__ float red[kWavesB];
+    const float ninf = -__builtin_inff();
+    const uint32_t tid = threadIdx.x;
+    const uint64_t row = blockIdx.x;
+    const uint32_t cols = (uint32_t)a.cols;
+    const uint32_t lim = (uint32_t)row_limit<K>(a, row);
+    const uint32_t whole = cols & ~3u;  // columns in whole float4; a ragged row's last ones are one thread's `tail`
+    const uint32_t need = K == SmKind::Causal && ((lim + 3u) & ~3u) < whole ? (lim + 3u) & ~3u : whole;
+    const float* ar = a.a + row * cols;
+    float* orow = a.out + row * cols;
+    Online o;
+
+    // Float4 past the ones to read repeat the last of them, so that no load is
+    // conditional (a branch per load costs the registers this kernel lives on).
+    const uint32_t last4 = (need >> 2) - 1u;
+    auto load = [&](uint32_t c) {
+        const uint32_t f = c * kLongThreads + tid;
+        const uint32_t off = 16u * (f < last4 ? f : last4);
+        const f32x4 r = __builtin_nontemporal_load(
+            reinterpret_cast<const f32x4_a4*>(reinterpret_cast<const char*>(ar) + off));
+        __builtin_amdgcn_sched_barrier(0);
+        return r;
+    };
+    auto add = [&](auto N_, uint32_t c, f32x4* v) {
+        constexpr int N = decltype(N_)::value;
+        bool in[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const uint32_t f = (c + u) * kLongThreads + tid;
+            in[u] = f <= last4;
+            if (K == SmKind::Causal) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) f4_set(v[u], k, 4 * f + k < lim ? f4_get(v[u], k) : ninf);
+            }
+        }
+        o.add<N>(v, in);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // The target's logit, read before any store: out may be the logits.
+    const uint64_t t = (K == SmKind::CeBwd) ? target_index(a.b[row], a.cols) : ~0ull;
+    const float xt = t < cols ? ar[t] : 0.0f;
+    f32x4 v[R];
+#pragma unroll
+    for (int c = 0; c < R; ++c) v[c] = load(c < kPre ? R + c : c);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < kPre; ++c) {
+        if ((uint32_t)(R + c) * kChunk < cols) keep[(uint32_t)c * kLongThreads + tid] = v[c];  // uniform
+        add(std::integral_constant<int, 1>(), R + c, &v[c]);
+        v[c] = load(c);
+    }
+    static_assert(R % kGrp == 0, "whole groups");
+#pragma unroll
+    for (int g = 0; g < R / kGrp; ++g) {
+        // the chunks that were loaded first come first
+        constexpr int kFirst = (kPre + kGrp - 1) / kGrp;
+        const int c = (g + kFirst) % (R / kGrp) * kGrp;
+        add(std::integral_constant<int, kGrp>(), c, &v[c]);
+    }
+    f32x4 tail = {ninf, ninf, ninf, ninf};
+    if (Ragged) {
+        if (tid == 0) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (whole + k < lim) f4_set(tail, k, ar[whole + k]);
+        }
+        const bool in = true;
+        o.add<1>(&tail, &in);
+    }
+    const float m = block_combine<true, kWavesB>(wave_max(o.m), red);
+    o.s *= o.m == ninf ? 1.0f : exp_diff(o.m - m);
+    const float s = block_combine<false, kWavesB>(wave_sum(o.s), red);
+    const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
+    const float inv_batch = 1.0f / (float)a.rows;
+    const float scale = (K == SmKind::CeBwd) ? inv * inv_batch : inv;
+    auto value = [&](uint32_t f, f32x4 x) {  // outputs of float4 f
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float e = exp_diff(f4_get(x, k) - m) * scale;
+            f4_set(x, k, K != SmKind::Causal || 4 * f + k < lim ? e : 0.0f * scale);
+        }
+        return x;
+    };
+    auto store = [&](uint32_t c, f32x4 x) {
+        const uint32_t first = c * kChunk;
+        const uint32_t n4 = whole > first ? (whole - first) >> 2 : 0u;
+        x = value(c * kLongThreads + tid, x);
+        if (tid < n4) __builtin_nontemporal_store((f32x4_a4)x, reinterpret_cast<f32x4_a4*>(orow + first) + tid);
+    };
+#pragma unroll
+    for (int c = 0; c < R; ++c) {
+        store(c, v[c]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (Lds) {
+        for (uint32_t c = R; c * kChunk < whole; ++c) store(c, keep[(c - R) * kLongThreads + tid]);
+    }
+    if (Ragged && tid == 0) {
+        tail = value(whole >> 2, tail);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (whole + k < cols) orow[whole + k] = f4_get(tail, k);
+    }
+    // The thread that stored the target's column stores it once more.
+    if (K == SmKind::CeBwd && t < cols && tid == (t < whole ? (uint32_t)(t >> 2) % kLongThreads : 0u))
+        orow[t] = exp_diff(xt - m) * scale - inv_batch;
 }
 
 // Any row length and alignment: one workgroup per row, the row streamed
@@ -274,10 +439,52 @@ __global__ __launch_bounds__(kSmBlock) void softmax_loop_kernel(SmArgs a) {
     }
 }
 
-template <SmKind K, int NCH>
+template <SmKind K, int NCH, bool Ragged>
 static void launch_wave(const SmArgs& a, hipStream_t s) {
     const uint64_t blocks = (a.rows + kSmWaves - 1) / kSmWaves;
-    hipLaunchKernelGGL((softmax_reg_kernel<K, NCH, false>), dim3((uint32_t)blocks), dim3(kSmBlock), 0, s, a);
+    hipLaunchKernelGGL((softmax_reg_kernel<K, NCH, false, Ragged>), dim3((uint32_t)blocks), dim3(kSmBlock), 0, s, a);
+}
+
+template <SmKind K, int R, bool Ragged>
+static void launch_long(const SmArgs& a, hipStream_t s) {
+    constexpr bool kLds = R == kLongRegs;
+    const uint64_t chunks = ((a.cols + 3) / 4 + kLongThreads - 1) / kLongThreads;
+    const size_t lds = chunks > (uint64_t)R ? (chunks - R) * kLongThreads * sizeof(f32x4) : 0;
+    hipLaunchKernelGGL((softmax_long_kernel<K, R, kLds, Ragged>), dim3((uint32_t)a.rows), dim3(kLongThreads), lds, s, a);
+}
+
+// The kernel for the row length.
+template <SmKind K, bool Ragged>
+static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
+    const uint64_t cols4 = (a.cols + 3) / 4;
+    const dim3 grid((uint32_t)a.rows);
+    if (cols4 <= 64) launch_wave<K, 1, Ragged>(a, s);
+    else if (cols4 <= 128) launch_wave<K, 2, Ragged>(a, s);
+    else if (cols4 <= 256) launch_wave<K, 4, Ragged>(a, s);
+    else if (cols4 <= 512) {
+        // 1025-2048 columns: one workgroup per row streams faster than one
+        // wave per row (measured at 32768 x 2048: forward 85.8 -> 83.3 us
+        // with 256 threads x 2 float4, backward 129.3 -> 121.7 us with 512
+        // threads x 1 float4 each of y and dy)
+        if (K == SmKind::Bwd)
+            hipLaunchKernelGGL((softmax_reg_kernel<K, 1, true, Ragged, 512>), grid, dim3(512), 0, s, a);
+        else
+            hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    }
+    else if (cols4 <= 1024) launch_wave<K, 16, Ragged>(a, s);
+    else if (cols4 <= 2048)
+        hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    else if (cols4 <= 4096)
+        hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    else if (K != SmKind::Bwd && a.cols <= kLongCols) {
+        if constexpr (K != SmKind::Bwd) {
+            if (cols4 <= 8 * kLongThreads) launch_long<K, 8, Ragged>(a, s);
+            else if (cols4 <= 16 * kLongThreads) launch_long<K, 16, Ragged>(a, s);
+            else launch_long<K, kLongRegs, Ragged>(a, s);
+        }
+    }
+    else
+        hipLaunchKernelGGL((softmax_loop_kernel<K, !Ragged>), grid, dim3(kSmBlock), 0, s, a);
 }
 
 template <SmKind K>
@@ -288,31 +495,12 @@ static int softmax_launch(const SmArgs& a, hipStream_t s) {
     if (!mul_ok(a.rows, a.cols, &elems) || elems > kMaxElements || a.rows > 0x7fffffffull)
         return KORE_HIP_ERR_OVERFLOW;
     if (K == SmKind::Causal && a.seq_offset + a.rows < a.seq_offset) return KORE_HIP_ERR_OVERFLOW;
-    const bool vec = (a.cols % 4 == 0) && aligned16(a.a) && aligned16(a.out) &&
-                     (K != SmKind::Bwd || aligned16(a.b));
-    const uint64_t cols4 = a.cols / 4;
-    if (vec && cols4 <= 64) launch_wave<K, 1>(a, s);
-    else if (vec && cols4 <= 128) launch_wave<K, 2>(a, s);
-    else if (vec && cols4 <= 256) launch_wave<K, 4>(a, s);
-    else if (vec && cols4 <= 512) {
-        // 1025-2048 columns: one workgroup per row streams faster than one
-        // wave per row (measured at 32768 x 2048: forward 85.8 -> 83.3 us
-        // with 256 threads x 2 float4, backward 129.3 -> 121.7 us with 512
-        // threads x 1 float4 each of y and dy)
-        if (K == SmKind::Bwd)
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 1, true, 512>), dim3((uint32_t)a.rows), dim3(512), 0, s, a);
-        else
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
-    }
-    else if (vec && cols4 <= 1024) launch_wave<K, 16>(a, s);
-    else if (vec && cols4 <= 2048)
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
-    else if (vec && cols4 <= 4096)
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
-    else if (vec)
-        hipLaunchKernelGGL((softmax_loop_kernel<K, true>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
+    const bool aligned = (a.cols % 4 == 0) && aligned16(a.a) && aligned16(a.out) &&
+                         (K != SmKind::Bwd || aligned16(a.b));
+    if (aligned)
+        softmax_dispatch<K, false>(a, s);
     else
-        hipLaunchKernelGGL((softmax_loop_kernel<K, false>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
+        softmax_dispatch<K, true>(a, s);
     return launch_status();
 }
 

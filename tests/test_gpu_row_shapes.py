@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from inputs import assert_close_scaled, normal, rmsnorm_inputs
+from inputs import assert_close, assert_close_scaled, normal, rmsnorm_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +77,87 @@ def test_rms_norm_backward_dgamma_over_gamma(rows, cols):
     torch.cuda.synchronize()
     assert dx.to_host().tobytes() == want[0].to_host().tobytes()
     assert dg.to_host()[:cols * 4].tobytes() == want[1].to_host()[:cols * 4].tobytes()
+
+
+# ----------------------------------------------------------- softmax family
+# Tolerances as in test_gpu_parity.py: 1e-5 against 64 bits; 1e-5 plus one rounding per term that the oracle's
+# left-to-right sums take.  Lengths: each plan's first and last (wave, workgroup, the long kernel's 8, 16 and 24 float4 a
+# thread and its LDS chunks, the loop), whole and ragged, at every 4-byte offset.
+SM_LENGTHS = [(9, 3, 1), (5, 250, 2), (6, 257, 3), (7, 511, 0), (5, 1023, 1), (3, 1024, 2), (3, 2047, 0), (3, 2048, 1),
+              (2, 4093, 3), (2, 8189, 0), (2, 16383, 2), (2, 16385, 0), (2, 16388, 0), (2, 32768, 0), (2, 32769, 1),
+              (2, 65536, 0), (2, 65539, 0), (2, 98304, 3), (2, 98308, 0), (2, 131071, 0), (2, 135168, 0),
+              (2, 135169, 0)]
+
+
+def _rows_with_specials(rows, cols, seed):
+    x = normal((rows, cols), seed) * 3
+    x[0, cols // 2:] -= 40.0          # a max early in the row, and late
+    x[-1, :cols // 2] -= 40.0
+    x[0, 0::7] = -np.inf              # threads that meet nothing but -inf
+    return x
+
+
+def _soft64(x):
+    e = np.exp(x.astype(np.float64) - x.max(-1, keepdims=True).astype(np.float64))
+    return e / e.sum(-1, keepdims=True)
+
+
+@pytest.mark.parametrize("rows,cols,offset", SM_LENGTHS)
+def test_softmax_family_long_and_ragged(rows, cols, offset):
+    print(f"softmax family rows={rows} cols={cols} offset={offset}", flush=True)
+    x = _rows_with_specials(rows, cols, cols)
+    n = rows * cols
+
+    def out_of(call):
+        b, t, start = room(n, offset)
+        call(b)
+        torch.cuda.synchronize()
+        return inside(t, start, n).reshape(rows, cols)
+
+    want = _soft64(x)
+    got = out_of(lambda b: rocm.rocm_softmax_f32(DEV, at(x, offset), rows, cols, b))
+    assert_close(got, want, what="softmax vs f64")
+    assert_close(got, oracle.softmax(x), rtol=1e-5 + cols * U32, what="softmax vs oracle")
+
+    back = cols // 3  # row r keeps back + r + 1 columns
+    got = out_of(lambda b: rocm.rocm_softmax_causal_f32(DEV, at(x, offset), rows, cols, back, b))
+    want_c = np.zeros((rows, cols))
+    for r in range(rows):
+        keep = min(back + r + 1, cols)
+        if np.isfinite(x[r, :keep]).any():
+            want_c[r, :keep] = _soft64(x[r:r + 1, :keep])[0]
+        else:
+            want_c[r, :keep] = np.nan
+        assert (got[r, keep:] == 0.0).all()
+    assert_close(got, want_c, what="causal vs f64")
+
+    y, dy = oracle.softmax(x), normal((rows, cols), cols + 1)
+    got = out_of(lambda b: rocm.rocm_softmax_backward_f32(DEV, at(dy, offset), at(y, offset), rows, cols, b))
+    y64, dy64 = y.astype(np.float64), dy.astype(np.float64)
+    scale = np.abs(y64) * (np.abs(dy64) + np.abs(y64 * dy64).sum(-1, keepdims=True))
+    assert_close_scaled(got, oracle.softmax_backward(dy, y), scale, rtol=1e-5 + cols * U32, what="backward")
+
+    t = np.array([(cols - 1 - 5 * r) % cols for r in range(rows)], np.float32)  # the last columns, a ragged tail's too
+    ref = want.copy()
+    ref[np.arange(rows), t.astype(np.int64)] -= 1.0
+    got = out_of(lambda b: rocm.rocm_cross_entropy_backward_f32(DEV, at(x, offset), at(t, 0), rows, cols, b))
+    assert_close(got, ref / rows, what="cross entropy vs f64")
+    b = at(x, offset)  # in place
+    rocm.rocm_cross_entropy_backward_f32(DEV, b, at(t, 0), rows, cols, b)
+    assert b.to_host(np.float32).tobytes() == got.tobytes()
+
+
+@pytest.mark.parametrize("cols", [1001, 20000, 70001])
+def test_softmax_long_and_ragged_nonfinite_rows(cols):
+    x = normal((6, cols), cols) * 2
+    x[0, 5] = np.nan
+    x[1, :] = -np.inf
+    x[2, cols - 1] = np.inf
+    x[3, :-1] = -np.inf
+    x[4] = -3e38
+    x[5, 0] = 3e38
+    for got, want in ((rocm.rocm_softmax_f32(DEV, at(x, 1), 6, cols), oracle.softmax(x)),
+                      (rocm.rocm_softmax_causal_f32(DEV, at(x, 1), 6, cols, cols), oracle.softmax_causal(x, cols)),
+                      (rocm.rocm_softmax_causal_f32(DEV, at(x, 0), 6, cols, 3), oracle.softmax_causal(x, 3))):
+        got = got.to_host(np.float32).reshape(6, cols)
+        assert_close(got, want, rtol=1e-5 + cols * U32, what="nonfinite rows")

@@ -33,7 +33,8 @@
 // checked against the plain fold on adversarial rows by the CPU test suite
 // (tests/csrc/check_segmented_fold.c restates this kernel in scalar C).
 //
-// Data movement per wave (one row per wave, four waves per workgroup):
+// Data movement per wave (one row per wave to 3072 columns, then two waves a
+// row and, from 4097, four):
 //   * the row is loaded with wave-wide global_load_dwordx4 (coalesced, 1 KiB
 //     per instruction), all in flight before first use, and kept in VGPRs
 //     for the epilogue: one HBM read per byte;
@@ -51,8 +52,10 @@
 //     v_readlane, jumps whole runs, and when a segment falls back the owning
 //     lane's fold of its own registers is broadcast.  No LDS, no re-read of
 //     global memory.
-// A wave's LDS traffic never crosses waves, so there are no barriers: LDS
-// operations from one wave complete in issue order.
+// One wave per row has no barriers: its LDS traffic never crosses waves, and
+// LDS operations from one wave complete in issue order.  Waves that share a row
+// meet at barriers for the estimates' sums, the running sum (handed from wave
+// to wave in the row's order) and the absmax.
 
 // Epilogue (element-parallel over all 64 lanes, coalesced layout):
 //   inv  = 1 / sqrt(ss / cols + eps)   IEEE sqrt and division (cpu_fused.rs:181-182)
@@ -93,17 +96,21 @@ struct NormArgs {
 // Transpose tile geometry.  Segment j (SL4 consecutive float4 of the row)
 // starts at float4 j*P of the tile, with an odd pitch P: 16 lanes reading
 // float4 k of 16 consecutive segments then hit 16 distinct 16-byte bank
-// groups.  For even SL4 with four waves per workgroup the tile holds half a
-// row (32 segments = SL4/2 whole load chunks) and is filled in two passes;
-// odd SL4, and one wave per workgroup (launches of few rows, where LDS is
-// plentiful and the second pass's round trip is on the row's chain), take
-// one pass.
+// groups.  A half tile (even SL4) holds 32 of a wave's 64 segments (SL4/2
+// whole load chunks) and is filled in two passes; a whole one takes one pass
+// (launches of few rows, where LDS is plentiful and the second pass's round
+// trip is on the row's chain, and odd SL4).
 __host__ __device__ constexpr int seg_pitch4(int sl4) { return (sl4 & 1) ? sl4 : sl4 + 1; }
-__host__ __device__ constexpr int tile_segs(int sl4, int wpb) { return (sl4 & 1) || wpb == 1 ? kSegs : kSegs / 2; }
-__host__ __device__ constexpr uint32_t wave_lds_f4(int sl4, int wpb) {
-    return (uint32_t)(tile_segs(sl4, wpb) * seg_pitch4(sl4));
+__host__ __device__ constexpr uint32_t wave_lds_f4(int sl4, bool half) {
+    return (uint32_t)((half ? kSegs / 2 : kSegs) * seg_pitch4(sl4));
 }
 
+// Rows a launch may hold.  Full: exactly 256 * SL4 * W columns, 16-byte
+// aligned.  Part: any whole number of float4, 16-byte aligned.  Ragged: any
+// length and 4-byte alignment (codes: any byte): dwordx4 accesses need no more
+// than dword alignment, and the row's last cols % 4 floats are one lane's.
+typedef uint32_t u32_a1 __attribute__((aligned(1)));
+enum class RowForm { Full, Part, Ragged };
 
 __device__ __forceinline__ int32_t cvt_i32_sat(float v) {
     // v_cvt_i32_f32: round toward zero, saturating, NaN -> 0.  Written as asm
@@ -258,10 +265,9 @@ __device__ __forceinline__ void auto_scan(uint32_t& a, uint32_t& b) {
     auto_scan_step<0x143, 0xc>(a, b);  // row_bcast:31 -> rows 2, 3
 }
 
-// Vector path: cols % 4 == 0, x/w/y 16-byte aligned, q 4-byte aligned,
-// ceil(cols/4 / 64) <= SL4.  Segment j covers float4 [j*SL4, (j+1)*SL4).
-// Grid: one block per WPB rows (one row per wave); dynamic LDS =
-// WPB * wave_lds_f4(SL4, WPB) float4 (the transpose tiles).
+// Vector path: up to 16384 columns, ceil(cols/4 / 64) <= SL4 * W.  Segment j of
+// a wave covers float4 [j*SL4, (j+1)*SL4) of its part of the row.  Dynamic LDS
+// = WPB * wave_lds_f4(SL4, Half) float4 (the transpose tiles).
 // silu(z) = z / (1 + e^-z) from the hardware exp2 and reciprocal (5 VALU
 // instead of ~25 for expf + IEEE division).  Error: v_exp_f32 and v_rcp_f32
 // are 1 ulp each; rounding z*log2(e) to f32 perturbs e^-z by |z|*2^-24*ln2
@@ -288,37 +294,73 @@ __device__ __forceinline__ float wave_max_nonneg(float v) {
     return read_lane(v, kWave - 1);
 }
 
-// FULL: cols == 256*SL4 exactly (every chunk and segment complete, no bounds
-// checks).  Otherwise rows are ragged: loads past the end read 0, segments
-// past the end are empty.
-template <NormOut Out, int SL4, bool FULL, int WPB>
+// W waves share a row: wave w owns float4 [64 SL4 w, 64 SL4 (w + 1)) of it as
+// 64 segments of its own, and the resolve passes the exact running sum from
+// wave to wave.  Rows past 4096 columns take W > 1, because one wave's float4
+// and squares then fill its registers (one wave a SIMD); a wave's walks and
+// folds also shorten by W.  WPB: waves per workgroup (W of one row, or W = 1
+// and WPB rows).
+template <NormOut Out, int SL4, RowForm Form, int WPB, int W, bool Half>
 __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
-    constexpr int NCH = SL4;  // 64*SL4 float4 cover the row: SL4 wave-wide chunks
+    static_assert(W == 1 || W == WPB, "a workgroup holds one row of W waves, or WPB rows of one");
+    constexpr bool FULL = Form == RowForm::Full;
+    constexpr bool RAGGED = Form == RowForm::Ragged;
+    constexpr int NCH = SL4;  // 64*SL4 float4 cover the wave's part: SL4 wave-wide chunks
     constexpr int P = seg_pitch4(SL4);
-    constexpr int TS = tile_segs(SL4, WPB);
+    constexpr int TS = Half ? kSegs / 2 : kSegs;
     constexpr int NPASS = kSegs / TS;
     constexpr int CPP = NCH / NPASS;  // load chunks per tile pass
-    constexpr uint32_t kWaveF4 = wave_lds_f4(SL4, WPB);
+    constexpr uint32_t kWaveF4 = wave_lds_f4(SL4, Half);
     extern __shared__ f32x4 lds4[];
+    __shared__ float meet[W > 1 ? 2 * W + 1 : 1];  // sums, absmaxes, the running sum
     const int lane = threadIdx.x & (kWave - 1);
     // Wave index as a scalar: row addresses then live in SGPRs and every
     // load and store takes the scalar-base form with a lane offset.
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const uint64_t row = (uint64_t)blockIdx.x * WPB + wave;
-    if (row >= args.rows) return;  // uniform per wave; no block barrier follows
-    const uint32_t cols4 = FULL ? (uint32_t)(kWave * SL4) : (args.cols >> 2);
-    const int nseg = FULL ? kSegs : (int)((cols4 + SL4 - 1) / SL4);
+    const uint64_t row = W > 1 ? (uint64_t)blockIdx.x : (uint64_t)blockIdx.x * WPB + wave;
+    if (W == 1 && row >= args.rows) return;  // uniform per wave; no block barrier follows
+    const uint32_t part0 = W > 1 ? (uint32_t)(kWave * SL4 * wave) : 0u;  // this wave's first float4
+    // float4 of the row, and whole ones
+    const uint32_t cols4 = FULL ? (uint32_t)(kWave * SL4 * W) : (args.cols + (RAGGED ? 3u : 0u)) >> 2;
+    const uint32_t whole4 = FULL ? cols4 : args.cols >> 2;
+    const int part4 = (int)cols4 - (int)part0;  // float4 from this wave's first on
+    const int nseg = FULL || part4 >= kSegs * SL4 ? kSegs : (part4 <= 0 ? 0 : (part4 + SL4 - 1) / SL4);
     f32x4* tile = lds4 + (size_t)wave * kWaveF4;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const f32x4* w4 = reinterpret_cast<const f32x4*>(args.w);
+
+    // Float4 f of a row of floats (RAGGED: f < whole4 only, the last one apart).
+    auto ld = [&](const float* r, uint32_t f) {
+        if (RAGGED) {
+            const f32x4_a4* q = reinterpret_cast<const f32x4_a4*>(r) + f;
+            return f < whole4 ? (f32x4)__builtin_nontemporal_load(q) : zero;
+        }
+        return FULL || f < cols4 ? ld_stream(reinterpret_cast<const f32x4*>(r) + f) : zero;
+    };
+    auto ld_weight = [&](uint32_t f) {
+        if (RAGGED) return f < whole4 ? (f32x4)reinterpret_cast<const f32x4_a4*>(args.w)[f] : zero;
+        return FULL || f < cols4 ? ld_cached(reinterpret_cast<const f32x4*>(args.w) + f) : zero;
+    };
+    // The row's last cols % 4 floats as a float4 (RAGGED).
+    auto ld_last = [&](const float* r) {
+        f32x4 v = zero;
+        const float* p = r + 4u * whole4;
+        const uint32_t n = args.cols & 3u;
+        if (n > 0) v.x = p[0];
+        if (n > 1) v.y = p[1];
+        if (n > 2) v.z = p[2];
+        return v;
+    };
 
     // ---- HBM reads: coalesced, chunk-major, all in flight.
-    const f32x4* xr = reinterpret_cast<const f32x4*>(args.x) + row * cols4;
+    const float* xr = args.x + row * (FULL ? (uint64_t)(4 * kWave * SL4 * W) : args.cols);
     f32x4 xv[NCH];
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        const uint32_t f = (uint32_t)c * kWave + lane;
-        xv[c] = (FULL || f < cols4) ? ld_stream(xr + f) : zero;
+    for (int c = 0; c < NCH; ++c) xv[c] = ld(xr, part0 + (uint32_t)c * kWave + lane);
+    if (RAGGED && (args.cols & 3u)) {
+        const f32x4 last = ld_last(xr);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (part0 + (uint32_t)c * kWave + lane == whole4) xv[c] = last;
     }
 
     // Wave priority rises with a row's progress (its loads issued: 1; its
@@ -332,9 +374,10 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     const int seg_id = kSegs - 1 - lane;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
-    // ---- transpose the squares through the wave's tile: float4 f of the row
-    // (segment q = f / SL4, offset f % SL4) goes to q*P + f % SL4 = f + (P -
-    // SL4)*q, minus the pass's base; segment reads use constant offsets.
+    // ---- transpose the squares through the wave's tile: float4 f of the
+    // wave's part (segment q = f / SL4, offset f % SL4) goes to q*P + f % SL4
+    // = f + (P - SL4)*q, minus the pass's base; segment reads use constant
+    // offsets.
     f32x4 seg[SL4];
 #pragma unroll
     for (int h = 0; h < NPASS; ++h) {
@@ -362,7 +405,15 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     // Estimate of the running sum at this segment's start = sum over the
     // segments before it = lanes above this one (any summation order).
     const float incl = wave_incl_scan(ssum);
-    const float est = read_lane(incl, kWave - 1) - incl;
+    float est = read_lane(incl, kWave - 1) - incl;
+    if (W > 1) {
+        if (lane == kWave - 1) meet[wave] = incl;
+        __syncthreads();
+        float before = 0.0f;
+#pragma unroll
+        for (int w = 0; w + 1 < W; ++w) before += w < wave ? meet[w] : 0.0f;
+        est += before;
+    }
 
     // Binade of the estimate (exponent field ef; ef <= 1 is the uniform grid
     // [0, 2^-125) of step 2^-149), selected branch-free.  Segment 0 folds
@@ -371,7 +422,8 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     const uint32_t ef_raw = __float_as_uint(est) >> 23;  // est >= 0
     const uint32_t ef = ef_raw < 1u ? 1u : ef_raw;
     const bool sub = ef == 1u;
-    const bool first = seg_id == 0 || empty;
+    const bool head = seg_id == 0 && wave == 0;  // the row's first segment (W == 1: every wave's)
+    const bool first = (W > 1 ? head : seg_id == 0) || empty;
     const bool bad = ef >= 255u;
     const float bot = sub ? 0.0f : __uint_as_float(ef << 23);
     const float top = __uint_as_float((ef + 1u) << 23);  // ef + 1 == 255 -> +Inf
@@ -407,7 +459,7 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     // sum, make a lighter scan but more resolve steps: measured slower at
     // every size.)  This lane's segment ends its run when the next segment
     // (lane - 1, moved here by wave_shr:1) has another key.
-    const int key_me = empty ? 1024 : (seg_id == 0 ? 1025 : (valid ? (int)ef : 2048 + seg_id));
+    const int key_me = empty ? 1024 : ((W > 1 ? head : seg_id == 0) ? 1025 : (valid ? (int)ef : 2048 + seg_id));
     const int key_next = __builtin_amdgcn_update_dpp(key_me, key_me, 0x138, 0xf, 0xf, false);
     const bool ends_here = lane == 0 || key_next != key_me;
     const uint64_t ends = __ballot(ends_here);
@@ -449,36 +501,51 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     // reads are issued before the test so that they overlap it.
     __builtin_amdgcn_s_setprio(3);
     uint32_t s = __builtin_amdgcn_readlane(__float_as_uint(w0), kWave - 1);
-    int j = 1;
-    uint32_t c0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, kSegs - 2);
-    uint32_t c1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, kSegs - 2);
-    while (j < nseg) {
-        const int nj = (int)(c1 & 0xffu);
-        const uint32_t n0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, (kSegs - 1 - nj) & (kWave - 1));
-        const uint32_t n1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, (kSegs - 1 - nj) & (kWave - 1));
-        const int32_t dp = (int32_t)(c1 << 17) >> 25;
-        const uint32_t t = s + (c0 & 0xffffffu) + ((s & 1u) ? (uint32_t)dp : 0u);
-        const uint32_t lo = (c0 >> 24) << 23;
-        const uint32_t da = s - lo, db = t - lo;
-        if ((c1 & 0x8000u) && (da > db ? da : db) < 0x800000u) {
-            s = t;
-            j = nj;
-            c0 = n0;
-            c1 = n1;
-            continue;
+    // W > 1: wave by wave, the running sum handed on through LDS.
+    auto resolve = [&](int j) {
+        uint32_t c0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, kSegs - 1 - j);
+        uint32_t c1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, kSegs - 1 - j);
+        while (j < nseg) {
+            const int nj = (int)(c1 & 0xffu);
+            const uint32_t n0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, (kSegs - 1 - nj) & (kWave - 1));
+            const uint32_t n1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, (kSegs - 1 - nj) & (kWave - 1));
+            const int32_t dp = (int32_t)(c1 << 17) >> 25;
+            const uint32_t t = s + (c0 & 0xffffffu) + ((s & 1u) ? (uint32_t)dp : 0u);
+            const uint32_t lo = (c0 >> 24) << 23;
+            const uint32_t da = s - lo, db = t - lo;
+            if ((c1 & 0x8000u) && (da > db ? da : db) < 0x800000u) {
+                s = t;
+                j = nj;
+                c0 = n0;
+                c1 = n1;
+                continue;
+            }
+            // Fold segment j alone.  The entry of segment j + 1 is read first so
+            // that its latency hides under the fold chain.  Every lane folds its
+            // own segment from s (same cost as one lane under an exec mask,
+            // without the mask changes); lane 63 - j's sum is the one kept.
+            const int L = kSegs - 1 - j;
+            c0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, (L - 1) & (kWave - 1));
+            c1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, (L - 1) & (kWave - 1));
+            float acc = __uint_as_float(s);
+    #pragma unroll
+            for (int k = 0; k < SL4; ++k) acc = fold4(acc, seg[k]);
+            s = (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(acc), L);
+            ++j;
         }
-        // Fold segment j alone.  The entry of segment j + 1 is read first so
-        // that its latency hides under the fold chain.  Every lane folds its
-        // own segment from s (same cost as one lane under an exec mask,
-        // without the mask changes); lane 63 - j's sum is the one kept.
-        const int L = kSegs - 1 - j;
-        c0 = (uint32_t)__builtin_amdgcn_readlane((int)e_w0, (L - 1) & (kWave - 1));
-        c1 = (uint32_t)__builtin_amdgcn_readlane((int)e_w1, (L - 1) & (kWave - 1));
-        float acc = __uint_as_float(s);
-#pragma unroll
-        for (int k = 0; k < SL4; ++k) acc = fold4(acc, seg[k]);
-        s = (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(acc), L);
-        ++j;
+    };
+    if (W == 1) {
+        resolve(1);
+    } else {
+        for (int turn = 0; turn < W; ++turn) {
+            if (turn == wave) {
+                if (turn) s = __builtin_amdgcn_readfirstlane(__float_as_uint(meet[2 * W]));
+                resolve(turn ? 0 : 1);
+                if (lane == 0) meet[2 * W] = __uint_as_float(s);
+            }
+            __syncthreads();
+        }
+        s = __builtin_amdgcn_readfirstlane(__float_as_uint(meet[2 * W]));
     }
     const float ss = __uint_as_float(s);
     __builtin_amdgcn_s_setprio(0);
@@ -488,48 +555,71 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     // measured slower: 14.0 -> 14.4 us at 4096 x 2560).
     f32x4 wv[NCH];
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-        const uint32_t f = (uint32_t)c * kWave + lane;
-        wv[c] = (FULL || f < cols4) ? ld_cached(w4 + f) : zero;
+    for (int c = 0; c < NCH; ++c) wv[c] = ld_weight(part0 + (uint32_t)c * kWave + lane);
+    if (RAGGED && (args.cols & 3u)) {
+        const f32x4 last = ld_last(args.w);
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+            if (part0 + (uint32_t)c * kWave + lane == whole4) wv[c] = last;
     }
 
     // cpu_fused.rs:181-182 with IEEE sqrt and division (ss is uniform).
     const float inv = 1.0f / sqrtf(ss / (float)args.cols + args.eps);
 
-    if (Out == NormOut::F32) {
-        f32x4* yr = reinterpret_cast<f32x4*>(args.y) + row * cols4;
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            const uint32_t f = (uint32_t)c * kWave + lane;
-            if (FULL || f < cols4) st_stream(yr + f, (xv[c] * inv) * wv[c]);
+    f32x4 last = zero;  // RAGGED: the row's last float4, in the lane that holds it
+    float* yr = args.y + row * args.cols;
+    auto st = [&](uint32_t f, f32x4 v) {
+        if (RAGGED) {
+            if (f < whole4) __builtin_nontemporal_store((f32x4_a4)v, reinterpret_cast<f32x4_a4*>(yr) + f);
+            if (f == whole4) last = v;
+        } else if (FULL || f < cols4) {
+            st_stream(reinterpret_cast<f32x4*>(yr) + f, v);
         }
+    };
+    // whole4 is one of this wave's float4, and this lane's
+    const uint32_t last_at = whole4 - part0;  // wraps past the end for earlier float4
+    const bool has_last = RAGGED && (args.cols & 3u) && last_at < (uint32_t)(kWave * SL4) &&
+                          (last_at & (kWave - 1)) == (uint32_t)lane;
+    auto st_last = [&]() {
+        if (has_last) {
+            float* p = yr + 4u * whole4;
+            const uint32_t n = args.cols & 3u;
+            p[0] = last.x;
+            if (n > 1) p[1] = last.y;
+            if (n > 2) p[2] = last.z;
+        }
+    };
+
+    if (Out == NormOut::F32) {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) st(part0 + (uint32_t)c * kWave + lane, (xv[c] * inv) * wv[c]);
+        st_last();
     } else if (Out == NormOut::SiluGate) {
         // cpu_fused.rs:466-471: x_hat = (x*inv)*g; y = x_hat * silu(z).
-        const f32x4* zr = reinterpret_cast<const f32x4*>(args.z) + row * cols4;
-        f32x4* yr = reinterpret_cast<f32x4*>(args.y) + row * cols4;
+        const float* zr = args.z + row * args.cols;
         // x_hat first, so that the weights are dead before z is loaded
         // (keeps the 2560-column kernel within 128 VGPRs: four waves a SIMD)
 #pragma unroll
         for (int c = 0; c < NCH; ++c) xv[c] = (xv[c] * inv) * wv[c];
         f32x4 zv[NCH];
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            const uint32_t f = (uint32_t)c * kWave + lane;
-            zv[c] = (FULL || f < cols4) ? ld_stream(zr + f) : zero;
+        for (int c = 0; c < NCH; ++c) zv[c] = ld(zr, part0 + (uint32_t)c * kWave + lane);
+        if (RAGGED && (args.cols & 3u)) {
+            const f32x4 lz = ld_last(zr);
+#pragma unroll
+            for (int c = 0; c < NCH; ++c)
+                if (part0 + (uint32_t)c * kWave + lane == whole4) zv[c] = lz;
         }
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            const uint32_t f = (uint32_t)c * kWave + lane;
-            if (FULL || f < cols4) {
-                const f32x4 xh = xv[c];
-                f32x4 g;
-                g.x = silu_fast(zv[c].x);
-                g.y = silu_fast(zv[c].y);
-                g.z = silu_fast(zv[c].z);
-                g.w = silu_fast(zv[c].w);
-                st_stream(yr + f, xh * g);
-            }
+            f32x4 g;
+            g.x = silu_fast(zv[c].x);
+            g.y = silu_fast(zv[c].y);
+            g.z = silu_fast(zv[c].z);
+            g.w = silu_fast(zv[c].w);
+            st(part0 + (uint32_t)c * kWave + lane, xv[c] * g);
         }
+        st_last();
     } else {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) xv[c] = (xv[c] * inv) * wv[c];
@@ -538,58 +628,70 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) amax = abs_max4(amax, xv[c]);
         amax = wave_max_nonneg(amax);
-        uint32_t* qr = reinterpret_cast<uint32_t*>(args.q) + row * cols4;
-        if (amax < kFastAmaxLimit) {
-            amax = amax < 1e-8f ? 1.0f : amax;  // kore-btes/src/quantize.rs:10
-            const float rcp = 1.0f / amax;
+        if (W > 1) {
+            if (lane == 0) meet[W + wave] = amax;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < W; ++w) amax = fmaxf(amax, meet[W + w]);
+            amax = read_lane(amax, 0);
+        }
+        int8_t* qr = args.q + row * args.cols;
+        uint32_t last_q = 0;
+        auto st_q = [&](uint32_t f, uint32_t d) {
+            if (RAGGED) {
+                if (f < whole4) reinterpret_cast<u32_a1*>(qr)[f] = d;
+                if (f == whole4) last_q = d;
+            } else if (FULL || f < cols4) {
+                reinterpret_cast<uint32_t*>(qr)[f] = d;
+            }
+        };
+        auto exact = [&](f32x4 v, float rcp) {
+            return pack4(quant_code(v.x, amax, rcp), quant_code(v.y, amax, rcp), quant_code(v.z, amax, rcp),
+                         quant_code(v.w, amax, rcp));
+        };
+        const bool fast = amax < kFastAmaxLimit;
+        amax = amax < 1e-8f ? 1.0f : amax;  // kore-btes/src/quantize.rs:10
+        const float rcp = 1.0f / amax;
+        if (lane == 0 && (W == 1 || wave == 0)) args.scale[row] = amax / 127.0f;
+        if (fast) {
             const float c127 = 127.0f * rcp;
-            if (lane == 0) args.scale[row] = amax / 127.0f;
             uint64_t redo[NCH];
             uint64_t any = 0;
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
-                const uint32_t f = (uint32_t)c * kWave + lane;
+                const uint32_t f = part0 + (uint32_t)c * kWave + lane;
                 uint32_t fm = 0;
                 const uint32_t d = flr_pack4(xv[c], c127, fm);
                 redo[c] = __ballot((FULL || f < cols4) && fm >= kFractLimit);
                 any |= redo[c];
-                if (FULL || f < cols4) qr[f] = d;
+                st_q(f, d);
             }
             if (any) {
                 // Rare: exact codes for the lanes whose brackets failed (they
                 // overwrite the stores above, in program order).
 #pragma unroll
                 for (int c = 0; c < NCH; ++c) {
-                    if ((redo[c] >> lane) & 1u) {
-                        const f32x4 v = xv[c];
-                        qr[(uint32_t)c * kWave + lane] =
-                            pack4(quant_code(v.x, amax, rcp), quant_code(v.y, amax, rcp),
-                                  quant_code(v.z, amax, rcp), quant_code(v.w, amax, rcp));
-                    }
+                    if ((redo[c] >> lane) & 1u) st_q(part0 + (uint32_t)c * kWave + lane, exact(xv[c], rcp));
                 }
             }
         } else {
             // An absmax of 2^120 or more, infinite, or NaN (every xn NaN):
             // exact codes.
-            amax = amax < 1e-8f ? 1.0f : amax;  // kore-btes/src/quantize.rs:10
-            const float rcp = 1.0f / amax;
-            if (lane == 0) args.scale[row] = amax / 127.0f;
 #pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                const uint32_t f = (uint32_t)c * kWave + lane;
-                if (FULL || f < cols4) {
-                    const f32x4 v = xv[c];
-                    qr[f] = pack4(quant_code(v.x, amax, rcp), quant_code(v.y, amax, rcp),
-                                  quant_code(v.z, amax, rcp), quant_code(v.w, amax, rcp));
-                }
-            }
+            for (int c = 0; c < NCH; ++c) st_q(part0 + (uint32_t)c * kWave + lane, exact(xv[c], rcp));
+        }
+        if (has_last) {
+            int8_t* p = qr + 4u * whole4;
+            const uint32_t n = args.cols & 3u;
+            p[0] = (int8_t)last_q;
+            if (n > 1) p[1] = (int8_t)(last_q >> 8);
+            if (n > 2) p[2] = (int8_t)(last_q >> 16);
         }
     }
 }
 
-// Scalar path for any shape/alignment: one thread per row, the reference loop
-// verbatim.  Used for cols % 4 != 0, unaligned views and rows longer than
-// the vector path's register budget.
+// Scalar path for rows of more than 16384 columns: one thread per row, the
+// reference loop verbatim.
 template <NormOut Out>
 __global__ __launch_bounds__(64) void row_norm_scalar_kernel(NormArgs args) {
     const uint64_t row = (uint64_t)blockIdx.x * 64 + threadIdx.x;
@@ -621,16 +723,18 @@ __global__ __launch_bounds__(64) void row_norm_scalar_kernel(NormArgs args) {
     }
 }
 
-template <NormOut Out, int SL4, int WPB>
-static int launch_vec_wpb(NormArgs a, hipStream_t s) {
-    const size_t lds = (size_t)WPB * wave_lds_f4(SL4, WPB) * sizeof(f32x4);
-    const uint64_t blocks = (a.rows + WPB - 1) / WPB;
+template <NormOut Out, int SL4, int WPB, int W, bool Half>
+static int launch_form(NormArgs a, RowForm form, hipStream_t s) {
+    const size_t lds = (size_t)WPB * wave_lds_f4(SL4, Half) * sizeof(f32x4);
+    const uint64_t blocks = (a.rows * W + WPB - 1) / WPB;
     if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-    if (a.cols == (uint32_t)(4 * kWave * SL4))
-        hipLaunchKernelGGL((row_norm_kernel<Out, SL4, true, WPB>), dim3((uint32_t)blocks), dim3(kWave * WPB), lds, s, a);
+    const dim3 grid((uint32_t)blocks), block(kWave * WPB);
+    if (form == RowForm::Ragged)
+        hipLaunchKernelGGL((row_norm_kernel<Out, SL4, RowForm::Ragged, WPB, W, Half>), grid, block, lds, s, a);
+    else if (a.cols == (uint32_t)(4 * kWave * SL4 * W))
+        hipLaunchKernelGGL((row_norm_kernel<Out, SL4, RowForm::Full, WPB, W, Half>), grid, block, lds, s, a);
     else
-        hipLaunchKernelGGL((row_norm_kernel<Out, SL4, false, WPB>), dim3((uint32_t)blocks), dim3(kWave * WPB), lds, s,
-                           a);
+        hipLaunchKernelGGL((row_norm_kernel<Out, SL4, RowForm::Part, WPB, W, Half>), grid, block, lds, s, a);
     return launch_status();
 }
 
@@ -639,35 +743,55 @@ static int launch_vec_wpb(NormArgs a, hipStream_t s) {
 // over more dispatchers and start sooner; 32 x 2048 RMSNorm 4.4 -> 4.0 us,
 // 64 x 2560 gate 6.0 -> 5.6 us) and, at any row count, for the row lengths
 // where the whole-row tiles still leave the register-bound occupancy: up to
-// 2048 columns, and 4096 or 8192 (RMSNorm 16384 x 2048 47.2 -> 46.0 us,
-// 8192 x 2048 26.5 -> 24.5, 16384 x 4096 94.7 -> 90.6, 16384 x 8192 202 ->
-// 182, pre-quant 4096 x 8192 54.7 -> 46.9; ties within 1% elsewhere).  For
-// SL4 = 10, 12 and 24 (2560, 3072 and 6144 columns) the whole-row tiles cap
-// a CU below the waves its registers allow, and four waves per workgroup
-// sharing half-row tiles are faster (pre-quant 4096 x 2560 13.0 against
-// 15.1 us, RMSNorm 4096 x 3072 16.3 against 21.4).
+// 2048 columns (RMSNorm 16384 x 2048 47.2 -> 46.0 us, 8192 x 2048 26.5 ->
+// 24.5).  For
+// SL4 = 10 and 12 (2560 and 3072 columns) the whole-row tiles cap a CU below
+// the waves its registers allow, and four waves per workgroup sharing half-row
+// tiles are faster (pre-quant 4096 x 2560 13.0 against 15.1 us, RMSNorm 4096 x
+// 3072 16.3 against 21.4).
 constexpr uint64_t kSmallRows = 256;
 
 template <NormOut Out, int SL4>
-static int launch_vec(NormArgs a, hipStream_t s) {
-    if constexpr (SL4 == 10 || SL4 == 12 || SL4 == 24) {
-        if (a.rows > kSmallRows) return launch_vec_wpb<Out, SL4, kWavesPerBlock>(a, s);
+static int launch_vec(NormArgs a, RowForm form, hipStream_t s) {
+    if constexpr (SL4 == 10 || SL4 == 12) {
+        if (a.rows > kSmallRows) return launch_form<Out, SL4, kWavesPerBlock, 1, true>(a, form, s);
     }
-    return launch_vec_wpb<Out, SL4, 1>(a, s);
+    return launch_form<Out, SL4, 1, 1, false>(a, form, s);
+}
+
+// Rows of W waves, from 3073 columns: at 4096 columns one wave a row leaves
+// three waves a SIMD (two at 3584, in the 4096 kernel's registers), at 8192 one.
+// Measured, one wave against several, RMSNorm / pre-quant in us: 4096 x 3584
+// 26.3 / 22.6 -> 20.9 / 18.9, 4096 x 4096 26.4 / 21.7 -> 22.4 / 18.9, 4096 x
+// 6912 58.6 / 53.6 -> 43.5 / 33.7, 4096 x 8192 52.6 / 47.1 -> 49.9 / 36.1; in
+// graph replays 1 x 6912 10.6 / 10.6 -> 5.9 / 6.0, 1 x 8192 7.3 / 9.0 -> 4.9 /
+// 5.4.  Past 8192 columns one thread folded a row: 2048 x 14336 4480 / 6376 ->
+// 45.7 / 35.3.  Four waves from 4097 columns (two: 4096 x 6912 46.3 / 37.0,
+// eight 44.3 / 38.7) and to 16384 (eight: 2048 x 14336 48.2 / 41.7).  Two waves
+// at 2560-3072 columns lose where rows are few (1 x 3072 3.6 -> 4.4).
+template <NormOut Out, int SL4, int W>
+static int launch_split(NormArgs a, RowForm form, hipStream_t s) {
+    return launch_form<Out, SL4, W, W, (SL4 & 1) == 0>(a, form, s);
 }
 
 template <NormOut Out>
-static int launch_sl4(NormArgs a, uint32_t nch, hipStream_t s) {
-    if (nch <= 1) return launch_vec<Out, 1>(a, s);
-    if (nch <= 2) return launch_vec<Out, 2>(a, s);
-    if (nch <= 4) return launch_vec<Out, 4>(a, s);
-    if (nch <= 6) return launch_vec<Out, 6>(a, s);
-    if (nch <= 8) return launch_vec<Out, 8>(a, s);
-    if (nch <= 10) return launch_vec<Out, 10>(a, s);
-    if (nch <= 12) return launch_vec<Out, 12>(a, s);
-    if (nch <= 16) return launch_vec<Out, 16>(a, s);
-    if (nch <= 24) return launch_vec<Out, 24>(a, s);
-    return launch_vec<Out, 32>(a, s);
+static int launch_sl4(NormArgs a, uint32_t nch, RowForm form, hipStream_t s) {
+    if (nch <= 1) return launch_vec<Out, 1>(a, form, s);
+    if (nch <= 2) return launch_vec<Out, 2>(a, form, s);
+    if (nch <= 4) return launch_vec<Out, 4>(a, form, s);
+    if (nch <= 6) return launch_vec<Out, 6>(a, form, s);
+    if (nch <= 8) return launch_vec<Out, 8>(a, form, s);
+    if (nch <= 10) return launch_vec<Out, 10>(a, form, s);
+    if (nch <= 12) return launch_vec<Out, 12>(a, form, s);
+    if (nch <= 16) return launch_split<Out, 8, 2>(a, form, s);
+    if (nch <= 20) return launch_split<Out, 5, 4>(a, form, s);
+    if (nch <= 24) return launch_split<Out, 6, 4>(a, form, s);
+    if (nch <= 28) return launch_split<Out, 7, 4>(a, form, s);
+    if (nch <= 32) return launch_split<Out, 8, 4>(a, form, s);
+    if (nch <= 40) return launch_split<Out, 10, 4>(a, form, s);
+    if (nch <= 48) return launch_split<Out, 12, 4>(a, form, s);
+    if (nch <= 56) return launch_split<Out, 14, 4>(a, form, s);
+    return launch_split<Out, 16, 4>(a, form, s);
 }
 
 // One row per wave: with the half-row tile a wave needs ~8 KB of LDS and
@@ -686,19 +810,19 @@ static int norm_launch(NormArgs a, hipStream_t s) {
     if (Out == NormOut::I8 && (!a.q || !a.scale)) return KORE_HIP_ERR_NULL_PTR;
     uint64_t elems;
     if (!mul_ok(a.rows, a.cols, &elems) || elems > kMaxElements) return KORE_HIP_ERR_OVERFLOW;
-    const uint32_t cols4 = a.cols / 4;
-    const uint32_t nch = (cols4 + kWave - 1) / kWave;
-    bool vec = a.cols % 4 == 0 && aligned16(a.x) && aligned16(a.w) && nch <= 32;
-    if (Out == NormOut::F32) vec = vec && aligned16(a.y);
-    else if (Out == NormOut::SiluGate) vec = vec && aligned16(a.y) && aligned16(a.z);
-    else vec = vec && (reinterpret_cast<uintptr_t>(a.q) & 3u) == 0;
+    const uint32_t nch = (uint32_t)(((uint64_t)a.cols + 255) / 256);
+    const bool vec = nch <= 64;
+    bool whole = a.cols % 4 == 0 && aligned16(a.x) && aligned16(a.w);
+    if (Out == NormOut::F32) whole = whole && aligned16(a.y);
+    else if (Out == NormOut::SiluGate) whole = whole && aligned16(a.y) && aligned16(a.z);
+    else whole = whole && (reinterpret_cast<uintptr_t>(a.q) & 3u) == 0;
     if (!vec) {
         uint64_t blocks = (a.rows + 63) / 64;
         if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
         hipLaunchKernelGGL(row_norm_scalar_kernel<Out>, dim3((uint32_t)blocks), dim3(64), 0, s, a);
         return launch_status();
     }
-    return launch_sl4<Out>(a, nch, s);
+    return launch_sl4<Out>(a, nch, whole ? RowForm::Part : RowForm::Ragged, s);
 }
 
 }  // namespace kore

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from inputs import assert_close, assert_close_scaled, normal, rmsnorm_inputs
+from inputs import assert_bitexact, assert_close, assert_close_scaled, normal, rmsnorm_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -161,3 +161,65 @@ def test_softmax_long_and_ragged_nonfinite_rows(cols):
                       (rocm.rocm_softmax_causal_f32(DEV, at(x, 0), 6, cols, 3), oracle.softmax_causal(x, 3))):
         got = got.to_host(np.float32).reshape(6, cols)
         assert_close(got, want, rtol=1e-5 + cols * U32, what="nonfinite rows")
+
+
+# ------------------------------------------------- RMSNorm, pre-quant, gate
+# Bit-exact for every plan: one wave a row to 4096 columns, two to 8192, four to 16384, each at its first and last
+# length, whole, partly filled (a wave without any column) and ragged; 16385 is the scalar kernel's.
+NORM_LENGTHS = [(3, 1, 1), (5, 6, 3), (300, 255, 2), (7, 1021, 1), (9, 1537, 0), (260, 2561, 3), (300, 3071, 0),
+                (2, 4095, 2), (3, 4096, 1), (300, 4097, 0), (2, 4100, 0), (5, 5119, 1), (270, 5120, 0), (3, 6144, 0),
+                (300, 6912, 0), (3, 6915, 2), (2, 7168, 0), (4, 7172, 0), (300, 8192, 0), (3, 8191, 3), (2, 8193, 0),
+                (2, 9000, 0), (3, 10240, 0), (2, 12285, 1), (3, 12288, 0), (259, 14336, 0), (2, 16383, 2),
+                (3, 16384, 0), (2, 16385, 0)]
+
+
+def _norm_rows(rows, cols, seed):
+    """Ordinary rows with outliers, and rows whose running sum creeps, overflows, vanishes or holds NaN."""
+    x = normal((rows, cols), seed)
+    x[normal((rows, cols), seed + 1) > 2.3] *= np.float32(20.0)
+    if rows > 2:
+        x[1] *= np.float32(2.0 ** -70)
+        x[2] = np.float32(1e19)
+    if rows > 6:
+        x[3] = 0.0
+        x[4, cols // 2] = np.nan
+        x[5, -1] = np.inf
+        x[6, cols // 2:] = 0.0
+    return x
+
+
+@pytest.mark.parametrize("rows,cols,offset", NORM_LENGTHS)
+def test_norm_family_long_and_ragged_bit_exact(rows, cols, offset):
+    print(f"norm family rows={rows} cols={cols} offset={offset}", flush=True)
+    x, w = _norm_rows(rows, cols, cols), normal((cols,), cols + 2, 1.0, 0.02)
+    n = rows * cols
+    b, t, start = room(n, offset)
+    rocm.rocm_rms_norm_f32(DEV, at(x, offset), at(w, offset), rows, cols, 1e-6, b)
+    torch.cuda.synchronize()
+    got = inside(t, start, n).reshape(rows, cols)
+    assert_bitexact(got, oracle.rms_norm(x, w, 1e-6), "rms_norm")
+    q = torch.full((n + 16,), 99, dtype=torch.int8, device="cuda:0")
+    s, s_all, s_at = room(rows, offset)
+    rocm.rocm_rms_norm_quant_i8(DEV, at(x, offset), at(w, offset), rows, cols, 1e-6,
+                                HipBuffer.from_tensor(q[4 + offset:4 + offset + n]), s)
+    torch.cuda.synchronize()
+    q = q.cpu().numpy()
+    assert (q[:4 + offset] == 99).all() and (q[4 + offset + n:] == 99).all()
+    want_q, want_s = oracle.rms_norm_quant_i8(x, w, 1e-6)
+    assert_bitexact(q[4 + offset:4 + offset + n].reshape(rows, cols), want_q, "codes")
+    assert_bitexact(inside(s_all, s_at, rows), want_s, "scales")
+    z = normal((rows, cols), cols + 3) * 3
+    b, t, start = room(n, offset)
+    rocm.rocm_fused_rms_norm_silu_gate_f32(DEV, at(x, offset), at(w, offset), at(z, offset), rows, cols, 1e-6, b)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        assert_close(inside(t, start, n).reshape(rows, cols), oracle.rms_norm_silu_gate(x, w, z, 1e-6),
+                     what="silu gate")
+
+
+@pytest.mark.parametrize("cols", [4097, 6912, 8192, 14336])
+def test_norm_in_place_rows_of_several_waves(cols):
+    x, w = normal((70, cols), 5), normal((cols,), 6, 1.0, 0.02)
+    b = at(x, 0)
+    rocm.rocm_rms_norm_f32(DEV, b, at(w, 0), 70, cols, 1e-6, out=b)
+    assert_bitexact(b.to_host(np.float32).reshape(70, cols), oracle.rms_norm(x, w, 1e-6), "in place")

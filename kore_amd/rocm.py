@@ -18,6 +18,7 @@ dims imply raises ``RocmError.MemoryError`` instead of reaching the GPU.
 """
 from __future__ import annotations
 
+import os
 from typing import Optional, Tuple
 
 import numpy as np
@@ -46,7 +47,7 @@ class RocmError(RuntimeError):
 
 def _check(status: int, context: str) -> None:
     """``check_hip`` (rocm/ffi.rs:211-220): map a C status to RocmError."""
-    if status == _lib.KORE_HIP_OK:
+    if not status:  # KORE_HIP_OK
         return
     text = _lib.status_string(status)
     if status > 0:
@@ -61,6 +62,34 @@ def _require_device(device_idx: int):
         raise RocmError("NotAvailable", f"device {device_idx} does not exist")
     _lib.load()  # fail loudly if the native library is missing
     return torch.device("cuda", device_idx)
+
+
+# What every call needs, kept cheap: on one token an op's kernel takes 3-6 us, so
+# host time per call bounds a decode step.  Looking the devices up and building
+# a Stream object on each call took 2.4 of its 7.2 us; it is 4.4 us now, 3.3 of
+# them the launch (a 6-call MLP block on one token 46.9 -> 30.3 us).  The device
+# count is looked up until a device has been found (a process's devices do not
+# change), and again in a forked child, where torch refuses to go on.
+_devices = 0
+
+
+def _forget_devices() -> None:
+    global _devices
+    _devices = 0
+
+
+os.register_at_fork(after_in_child=_forget_devices)
+_raw_stream = getattr(getattr(torch, "_C", None), "_cuda_getCurrentRawStream", None)
+
+
+def _library(device_idx: int):
+    """The loaded library, for an op on a device that exists."""
+    global _devices
+    if not 0 <= device_idx < _devices:
+        _require_device(device_idx)
+        torch.cuda.init()
+        _devices = torch.cuda.device_count()
+    return _lib._lib or _lib.load()
 
 
 class HipBuffer:
@@ -108,7 +137,7 @@ class HipBuffer:
 
     @property
     def ptr(self) -> int:
-        return self._t.data_ptr() if self._t.numel() else 0
+        return self._t.data_ptr()  # 0 when empty
 
     def tensor(self, dtype=None):
         """View of the bytes as a torch tensor of ``dtype`` (no copy)."""
@@ -120,18 +149,21 @@ class HipBuffer:
 
 
 def _stream(device_idx: int) -> int:
+    """The raw handle of torch's current stream (without building a Stream object where torch can say it)."""
+    if _raw_stream is not None:
+        return _raw_stream(int(device_idx))
     return torch.cuda.current_stream(device_idx).cuda_stream
 
 
-def _need(buf: HipBuffer, nbytes: int, what: str) -> None:
+def _need(buf: HipBuffer, nbytes: int, *what: str) -> None:
     if buf.nbytes < nbytes:
-        raise RocmError("MemoryError", f"{what}: buffer holds {buf.nbytes} bytes, op needs {nbytes}")
+        raise RocmError("MemoryError", f"{' '.join(what)}: buffer holds {buf.nbytes} bytes, op needs {nbytes}")
 
 
-def _out(device_idx: int, out: Optional[HipBuffer], nbytes: int, what: str) -> HipBuffer:
+def _out(device_idx: int, out: Optional[HipBuffer], nbytes: int, *what: str) -> HipBuffer:
     if out is None:
         return HipBuffer.empty(device_idx, nbytes)
-    _need(out, nbytes, what)
+    _need(out, nbytes, *what)
     return out
 
 
@@ -140,12 +172,12 @@ def rocm_rms_norm_f32(device_idx: int, input: HipBuffer, weight: HipBuffer, rows
                       eps: float, out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_rms_norm_f32`` (cuda/ops.rs:517-541); bit-exact twin of
     ``fused_rms_norm`` (crates/kore-kernels/src/cpu_fused.rs:160-190)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(input, n, "rms_norm input")
     _need(weight, cols * 4, "rms_norm weight")
     o = _out(device_idx, out, n, "rms_norm out")
-    _check(_lib.load().kore_hip_rms_norm_f32(input.ptr, weight.ptr, o.ptr, rows, cols, eps,
+    _check(lib.kore_hip_rms_norm_f32(input.ptr, weight.ptr, o.ptr, rows, cols, eps,
                                              _stream(device_idx)), "rms_norm_f32")
     return o
 
@@ -155,58 +187,57 @@ def rocm_fused_rms_norm_silu_gate_f32(device_idx: int, input: HipBuffer, gamma: 
                                       out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_fused_rms_norm_silu_gate_f32`` (cuda/ops.rs:717-751):
     y = RMSNorm(x) * silu(z), RMSNorm bit-exact as ``rocm_rms_norm_f32``."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(input, n, "rms_norm_silu_gate input")
     _need(gamma, cols * 4, "rms_norm_silu_gate gamma")
     _need(gate, n, "rms_norm_silu_gate gate")
     o = _out(device_idx, out, n, "rms_norm_silu_gate out")
-    _check(_lib.load().kore_hip_rms_norm_silu_gate_f32(input.ptr, gamma.ptr, gate.ptr, o.ptr, rows, cols, eps,
+    _check(lib.kore_hip_rms_norm_silu_gate_f32(input.ptr, gamma.ptr, gate.ptr, o.ptr, rows, cols, eps,
                                                        _stream(device_idx)), "rms_norm_silu_gate_f32")
     return o
 
 
 # ------------------------------------------------------------ activations
-def _unary(name: str, device_idx: int, a: HipBuffer, n: int, out: Optional[HipBuffer]) -> HipBuffer:
-    _require_device(device_idx)
-    _need(a, n * 4, f"{name} input")
-    o = _out(device_idx, out, n * 4, f"{name} out")
-    _check(getattr(_lib.load(), f"kore_hip_{name}_f32")(a.ptr, o.ptr, n, _stream(device_idx)), f"{name}_f32")
+def _unary(symbol: str, name: str, device_idx: int, a: HipBuffer, n: int, out: Optional[HipBuffer]) -> HipBuffer:
+    lib = _library(device_idx)
+    _need(a, n * 4, name, "input")
+    o = _out(device_idx, out, n * 4, name, "out")
+    _check(getattr(lib, symbol)(a.ptr, o.ptr, n, _stream(device_idx)), symbol[9:])
     return o
 
 
 def rocm_gelu_f32(device_idx: int, a: HipBuffer, n: int, out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_gelu_f32`` (cuda/ops.rs:197-204); twin of ``kore_nn::activations::gelu``."""
-    return _unary("gelu", device_idx, a, n, out)
+    return _unary("kore_hip_gelu_f32", "gelu", device_idx, a, n, out)
 
 
 def rocm_silu_f32(device_idx: int, a: HipBuffer, n: int, out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_silu_f32`` (cuda/ops.rs:206-213); twin of ``kore_nn::activations::silu``."""
-    return _unary("silu", device_idx, a, n, out)
+    return _unary("kore_hip_silu_f32", "silu", device_idx, a, n, out)
 
 
-def _binary(name: str, device_idx: int, a: HipBuffer, b: HipBuffer, n: int,
+def _binary(symbol: str, name: str, device_idx: int, a: HipBuffer, b: HipBuffer, n: int,
             out: Optional[HipBuffer]) -> HipBuffer:
-    _require_device(device_idx)
-    _need(a, n * 4, f"{name} a")
-    _need(b, n * 4, f"{name} b")
-    o = _out(device_idx, out, n * 4, f"{name} out")
-    _check(getattr(_lib.load(), f"kore_hip_{name}_f32")(a.ptr, b.ptr, o.ptr, n, _stream(device_idx)),
-           f"{name}_f32")
+    lib = _library(device_idx)
+    _need(a, n * 4, name, "a")
+    _need(b, n * 4, name, "b")
+    o = _out(device_idx, out, n * 4, name, "out")
+    _check(getattr(lib, symbol)(a.ptr, b.ptr, o.ptr, n, _stream(device_idx)), symbol[9:])
     return o
 
 
 def rocm_mul_f32(device_idx: int, a: HipBuffer, b: HipBuffer, n: int,
                  out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_mul_f32`` (cuda/ops.rs:100-108); twin of ``Tensor::mul``."""
-    return _binary("mul", device_idx, a, b, n, out)
+    return _binary("kore_hip_mul_f32", "mul", device_idx, a, b, n, out)
 
 
 def rocm_swiglu_f32(device_idx: int, gate: HipBuffer, up: HipBuffer, n: int,
                     out: Optional[HipBuffer] = None) -> HipBuffer:
     """silu(gate) * up in one pass (the reference composes silu then mul,
     crates/kore-serve/src/layered/engine.rs:633-643)."""
-    return _binary("swiglu", device_idx, gate, up, n, out)
+    return _binary("kore_hip_swiglu_f32", "swiglu", device_idx, gate, up, n, out)
 
 
 # ------------------------------------------------------------------- RoPE
@@ -230,10 +261,10 @@ def rocm_rope_f32(device_idx: int, data: HipBuffer, inv_freq: HipBuffer, batch: 
     [batch, seq_len, num_heads, head_dim]; half-split pairs by default
     (crates/kore-edge/src/ops/rope.rs:9-36), interleaved pairs as
     kore-serve's ``apply_rope`` (engine.rs:706-727)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(data, batch * seq_len * num_heads * head_dim * 4, "rope data")
     _need(inv_freq, (head_dim // 2) * 4, "rope inv_freq")
-    _check(_lib.load().kore_hip_rope_f32(data.ptr, inv_freq.ptr, batch, seq_len, num_heads, head_dim,
+    _check(lib.kore_hip_rope_f32(data.ptr, inv_freq.ptr, batch, seq_len, num_heads, head_dim,
                                          start_pos, int(bool(interleaved)), _stream(device_idx)), "rope_f32")
 
 
@@ -242,11 +273,11 @@ def rocm_rope_qk_f32(device_idx: int, q: HipBuffer, k: HipBuffer, inv_freq: HipB
                      interleaved: bool = False) -> None:
     """Q and K of one layer rotated in one launch (same results as two
     ``rocm_rope_f32`` calls)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(q, batch * seq_len * q_heads * head_dim * 4, "rope q")
     _need(k, batch * seq_len * k_heads * head_dim * 4, "rope k")
     _need(inv_freq, (head_dim // 2) * 4, "rope inv_freq")
-    _check(_lib.load().kore_hip_rope_qk_f32(q.ptr, k.ptr, inv_freq.ptr, batch, seq_len, q_heads, k_heads,
+    _check(lib.kore_hip_rope_qk_f32(q.ptr, k.ptr, inv_freq.ptr, batch, seq_len, q_heads, k_heads,
                                             head_dim, start_pos, int(bool(interleaved)), _stream(device_idx)),
            "rope_qk_f32")
 
@@ -256,11 +287,11 @@ def rocm_embedding_f32(device_idx: int, table: HipBuffer, ids: HipBuffer, n_ids:
                        out: Optional[HipBuffer] = None) -> HipBuffer:
     """``Embedding::lookup`` (crates/kore-nn/src/embedding.rs:55-72) on the
     device: ids are u32/i32, out-of-range ids give zero rows."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(table, vocab * dim * 4, "embedding table")
     _need(ids, n_ids * 4, "embedding ids")
     o = _out(device_idx, out, n_ids * dim * 4, "embedding out")
-    _check(_lib.load().kore_hip_embedding_f32(table.ptr, ids.ptr, o.ptr, n_ids, vocab, dim, _stream(device_idx)),
+    _check(lib.kore_hip_embedding_f32(table.ptr, ids.ptr, o.ptr, n_ids, vocab, dim, _stream(device_idx)),
            "embedding_f32")
     return o
 
@@ -270,11 +301,11 @@ def rocm_embedding_forward_f32(device_idx: int, table: HipBuffer, ids: HipBuffer
     """``Embedding::forward`` (crates/kore-nn/src/embedding.rs:91-98) on the
     device: ids are an f32 buffer converted like Rust's ``v as usize`` (NaN
     and values below 1 -> 0, saturating), then looked up as ``lookup``."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(table, vocab * dim * 4, "embedding table")
     _need(ids, n_ids * 4, "embedding ids")
     o = _out(device_idx, out, n_ids * dim * 4, "embedding out")
-    _check(_lib.load().kore_hip_embedding_forward_f32(table.ptr, ids.ptr, o.ptr, n_ids, vocab, dim,
+    _check(lib.kore_hip_embedding_forward_f32(table.ptr, ids.ptr, o.ptr, n_ids, vocab, dim,
                                                       _stream(device_idx)), "embedding_forward_f32")
     return o
 
@@ -285,12 +316,12 @@ def rocm_rms_norm_quant_i8(device_idx: int, input: HipBuffer, weight: HipBuffer,
                            out_scale: Optional[HipBuffer] = None) -> Tuple[HipBuffer, HipBuffer]:
     """RMSNorm + per-row absmax int8 in one pass; returns (q int8[rows, cols],
     scale f32[rows]) with x ~= q * scale."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(input, rows * cols * 4, "prequant input")
     _need(weight, cols * 4, "prequant weight")
     q = _out(device_idx, out_q, rows * cols, "prequant q")
     s = _out(device_idx, out_scale, rows * 4, "prequant scale")
-    _check(_lib.load().kore_hip_rms_norm_quant_i8(input.ptr, weight.ptr, q.ptr, s.ptr, rows, cols, eps,
+    _check(lib.kore_hip_rms_norm_quant_i8(input.ptr, weight.ptr, q.ptr, s.ptr, rows, cols, eps,
                                                   _stream(device_idx)), "rms_norm_quant_i8")
     return q, s
 
@@ -307,11 +338,11 @@ def rocm_softmax_f32(device_idx: int, a: HipBuffer, rows: int, cols: int,
                      out: Optional[HipBuffer] = None) -> HipBuffer:
     """``cuda_softmax_f32`` (cuda/ops.rs:486-511); twin of ``fused_softmax``
     (cpu_fused.rs:195-231)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(a, n, "softmax input")
     o = _out(device_idx, out, n, "softmax out")
-    _check(_lib.load().kore_hip_softmax_f32(a.ptr, o.ptr, rows, cols, _stream(device_idx)), "softmax_f32")
+    _check(lib.kore_hip_softmax_f32(a.ptr, o.ptr, rows, cols, _stream(device_idx)), "softmax_f32")
     return o
 
 
@@ -319,11 +350,11 @@ def rocm_softmax_causal_f32(device_idx: int, a: HipBuffer, rows: int, cols: int,
                             out: Optional[HipBuffer] = None) -> HipBuffer:
     """The ``softmax_causal_f32`` kernel (cuda/kernels/softmax.cu:88-157): row r
     keeps columns < seq_offset + r + 1."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(a, n, "softmax_causal input")
     o = _out(device_idx, out, n, "softmax_causal out")
-    _check(_lib.load().kore_hip_softmax_causal_f32(a.ptr, o.ptr, rows, cols, seq_offset, _stream(device_idx)),
+    _check(lib.kore_hip_softmax_causal_f32(a.ptr, o.ptr, rows, cols, seq_offset, _stream(device_idx)),
            "softmax_causal_f32")
     return o
 
@@ -332,12 +363,12 @@ def rocm_softmax_backward_f32(device_idx: int, grad_output: HipBuffer, output: H
                               out: Optional[HipBuffer] = None) -> HipBuffer:
     """``fused_softmax_backward`` (cpu_fused_backward.rs:86-115) on the device:
     grad_input = y * (dy - sum(y * dy))."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(grad_output, n, "softmax_backward grad_output")
     _need(output, n, "softmax_backward output")
     o = _out(device_idx, out, n, "softmax_backward grad_input")
-    _check(_lib.load().kore_hip_softmax_backward_f32(grad_output.ptr, output.ptr, o.ptr, rows, cols,
+    _check(lib.kore_hip_softmax_backward_f32(grad_output.ptr, output.ptr, o.ptr, rows, cols,
                                                      _stream(device_idx)), "softmax_backward_f32")
     return o
 
@@ -346,12 +377,12 @@ def rocm_cross_entropy_backward_f32(device_idx: int, logits: HipBuffer, targets:
                                     num_classes: int, out: Optional[HipBuffer] = None) -> HipBuffer:
     """``fused_cross_entropy_backward`` (cpu_fused_backward.rs:130-170) on the
     device: (softmax(logits) - one_hot(targets)) / batch; targets are f32."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = batch * num_classes * 4
     _need(logits, n, "cross_entropy_backward logits")
     _need(targets, batch * 4, "cross_entropy_backward targets")
     o = _out(device_idx, out, n, "cross_entropy_backward grad")
-    _check(_lib.load().kore_hip_cross_entropy_backward_f32(logits.ptr, targets.ptr, o.ptr, batch, num_classes,
+    _check(lib.kore_hip_cross_entropy_backward_f32(logits.ptr, targets.ptr, o.ptr, batch, num_classes,
                                                            _stream(device_idx)), "cross_entropy_backward_f32")
     return o
 
@@ -367,7 +398,7 @@ def rocm_rms_norm_backward_f32(device_idx: int, grad_output: HipBuffer, input: H
                                grad_input: Optional[HipBuffer] = None, grad_gamma: Optional[HipBuffer] = None):
     """``fused_rms_norm_backward`` (cpu_fused_backward.rs:20-81) on the device
     -> (grad_input, grad_gamma).  The workspace is allocated when not given."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     n = rows * cols * 4
     _need(grad_output, n, "rms_norm_backward grad_output")
     _need(input, n, "rms_norm_backward input")
@@ -376,7 +407,7 @@ def rocm_rms_norm_backward_f32(device_idx: int, grad_output: HipBuffer, input: H
     gg = _out(device_idx, grad_gamma, cols * 4, "rms_norm_backward grad_gamma")
     wsb = rocm_rms_norm_backward_workspace_bytes(rows, cols)
     ws = workspace if workspace is not None else HipBuffer.empty(device_idx, max(wsb, 16))
-    _check(_lib.load().kore_hip_rms_norm_backward_f32(grad_output.ptr, input.ptr, gamma.ptr, gx.ptr, gg.ptr, ws.ptr,
+    _check(lib.kore_hip_rms_norm_backward_f32(grad_output.ptr, input.ptr, gamma.ptr, gx.ptr, gg.ptr, ws.ptr,
                                                       ws.nbytes, rows, cols, eps, _stream(device_idx)),
            "rms_norm_backward_f32")
     return gx, gg
@@ -390,13 +421,13 @@ def rocm_ternary_matmul_i8(device_idx: int, a_packed: HipBuffer, a_scales: HipBu
     * q[n, k]) * a_scales[m]) * q_scales[n], with the base-243 weights of
     ``pack_weights_ternary`` (cpu_ternary_matmul.rs:198-240) and the epilogue
     of ``ternary_ternary_matmul`` (cpu_ternary_matmul.rs:188)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(a_packed, m * ((k + 4) // 5), "ternary weights")
     _need(a_scales, m * 4, "ternary scales")
     _need(q, n * k, "ternary codes")
     _need(q_scales, n * 4, "ternary code scales")
     c = _out(device_idx, out, m * n * 4, "ternary out")
-    _check(_lib.load().kore_hip_ternary_matmul_i8(a_packed.ptr, a_scales.ptr, q.ptr, q_scales.ptr, c.ptr, m, n, k,
+    _check(lib.kore_hip_ternary_matmul_i8(a_packed.ptr, a_scales.ptr, q.ptr, q_scales.ptr, c.ptr, m, n, k,
                                                   _stream(device_idx)), "ternary_matmul_i8")
     return c
 
@@ -407,12 +438,12 @@ def rocm_ternary_matmul_f32(device_idx: int, a_packed: HipBuffer, a_scales: HipB
     calls it): c[m, n] = (sum over k in order of trit[m, k] * b[k, n]) *
     a_scales[m] with f32 activations b[K, N], the sum the reference's
     sequential f32 fold (bit-exact)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(a_packed, m * ((k + 4) // 5), "ternary weights")
     _need(a_scales, m * 4, "ternary scales")
     _need(b, k * n * 4, "ternary activations")
     c = _out(device_idx, out, m * n * 4, "ternary out")
-    _check(_lib.load().kore_hip_ternary_matmul_f32(a_packed.ptr, a_scales.ptr, b.ptr, c.ptr, m, n, k,
+    _check(lib.kore_hip_ternary_matmul_f32(a_packed.ptr, a_scales.ptr, b.ptr, c.ptr, m, n, k,
                                                    _stream(device_idx)), "ternary_matmul_f32")
     return c
 
@@ -424,14 +455,14 @@ def rocm_bit_linear_f32(device_idx: int, a_packed: HipBuffer, a_scales: HipBuffe
     out] = ternary_matmul(W, scales, x^T)^T + bias with the layer's input
     x[batch, in] as stored and the output in the layer's layout; bias None for
     a layer without bias (bit-exact)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(a_packed, out_features * ((in_features + 4) // 5), "ternary weights")
     _need(a_scales, out_features * 4, "ternary scales")
     _need(x, batch * in_features * 4, "layer input")
     if bias is not None:
         _need(bias, out_features * 4, "bias")
     y = _out(device_idx, out, batch * out_features * 4, "layer output")
-    _check(_lib.load().kore_hip_bit_linear_f32(a_packed.ptr, a_scales.ptr, x.ptr, bias.ptr if bias else None, y.ptr,
+    _check(lib.kore_hip_bit_linear_f32(a_packed.ptr, a_scales.ptr, x.ptr, bias.ptr if bias else None, y.ptr,
                                                out_features, batch, in_features, _stream(device_idx)),
            "bit_linear_f32")
     return y
@@ -443,7 +474,7 @@ def rocm_bit_linear_i8(device_idx: int, a_packed: HipBuffer, a_scales: HipBuffer
     """The BitLinear layer on pre-quant codes q[batch, in] / q_scales[batch]:
     y[b, o] = c[o, b] + bias[o] with c of ``rocm_ternary_matmul_i8``, in the
     layer's [batch, out] layout (bit-exact)."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(a_packed, out_features * ((in_features + 4) // 5), "ternary weights")
     _need(a_scales, out_features * 4, "ternary scales")
     _need(q, batch * in_features, "codes")
@@ -451,7 +482,7 @@ def rocm_bit_linear_i8(device_idx: int, a_packed: HipBuffer, a_scales: HipBuffer
     if bias is not None:
         _need(bias, out_features * 4, "bias")
     y = _out(device_idx, out, batch * out_features * 4, "layer output")
-    _check(_lib.load().kore_hip_bit_linear_i8(a_packed.ptr, a_scales.ptr, q.ptr, q_scales.ptr,
+    _check(lib.kore_hip_bit_linear_i8(a_packed.ptr, a_scales.ptr, q.ptr, q_scales.ptr,
                                               bias.ptr if bias else None, y.ptr, out_features, batch, in_features,
                                               _stream(device_idx)), "bit_linear_i8")
     return y
@@ -463,12 +494,12 @@ def rocm_pack_weights_ternary(device_idx: int, w: HipBuffer, m: int, k: int, thr
     """``pack_weights_ternary`` (cpu_ternary_matmul.rs:198-240): f32 weights
     w[m, k] -> (base-243 packed bytes [m, ceil(k/5)], per-row scales [m]),
     bit-exact."""
-    _require_device(device_idx)
+    lib = _library(device_idx)
     _need(w, m * k * 4, "weights")
     kp = (k + 4) // 5
     p = _out(device_idx, packed, m * kp, "packed weights")
     sc = _out(device_idx, scales, m * 4, "weight scales")
-    _check(_lib.load().kore_hip_pack_weights_ternary(w.ptr, m, k, threshold, p.ptr, sc.ptr, _stream(device_idx)),
+    _check(lib.kore_hip_pack_weights_ternary(w.ptr, m, k, threshold, p.ptr, sc.ptr, _stream(device_idx)),
            "pack_weights_ternary")
     return p, sc
 

@@ -23,10 +23,10 @@
 // own CUDA kernel is.  exp(d) is evaluated on the reference's d = x - m
 // (rounded the same way) as the hardware exp2(d * log2(e)); see exp_diff.
 //
-// Shapes: a row of up to 1024 floats, or of 2049-4096, is held in one wave's
-// registers (one wave per row, 4 rows per workgroup); 1025-2048 floats and
-// up to 16384 in one workgroup's (256 threads; 512 for the 1025-2048
-// backward); up to 135168 (vocabularies) in the registers and LDS of a CU
+// Shapes: a row of up to 1024 floats is held in one wave's registers (one wave
+// per row, 4 rows per workgroup); up to 16384 in one workgroup's (256 threads;
+// 512 for the 1025-2048 backward and for 2049-4096, where some row counts take
+// a wave per row); up to 135168 (vocabularies) in the registers and LDS of a CU
 // (forward and cross-entropy); still longer rows, and the backward's from
 // 16385, stream through a workgroup in three passes (two).  Rows of any length
 // and alignment take the same kernels, their last cols % 4 floats one by one.
@@ -103,7 +103,7 @@ __device__ __forceinline__ float block_combine(float v, float* red) {
 // Row in registers.  Wave mode (Block = false): one wave per row, element f4
 // index = c*64 + lane, 4 rows per 256-thread workgroup.  Block mode: one
 // workgroup of BS threads per row, index = c*BS + tid.
-// Ragged: rows of any length and alignment (ld_row4).  Causal rows read only
+// Ragged: rows of any length and alignment (ld_row4_now).  Causal rows read only
 // the float4 that hold a column they keep.
 template <SmKind K, int NCH, bool Block, bool Ragged, int BS = kSmBlock>
 __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
@@ -117,6 +117,8 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
     const int me = Block ? (int)threadIdx.x : lane;
     const uint32_t cols = (uint32_t)a.cols;               // <= 16384 here
     const uint32_t lim = (uint32_t)row_limit<K>(a, row);  // <= cols
+    // columns to read: causal rows leave out the float4 past their last one
+    const uint32_t need = K == SmKind::Causal && lim + 3u < cols ? (lim + 3u) & ~3u : cols;
     const float* ar = a.a + row * cols;
     const float* br = a.b + row * cols;
     float* orow = a.out + row * cols;
@@ -125,8 +127,8 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const uint32_t f = (uint32_t)(c * step + me);
-        v[c] = ld_row4<Ragged>(ar, f, K == SmKind::Causal && !Ragged ? (lim + 3u) & ~3u : (K == SmKind::Causal ? lim : cols));
-        if (K == SmKind::Bwd) g[c] = ld_row4<Ragged>(br, f, cols);
+        v[c] = ld_row4_now<Ragged>(ar, f, need);
+        if (K == SmKind::Bwd) g[c] = ld_row4_now<Ragged>(br, f, cols);
     }
 
     if (K == SmKind::Bwd) {
@@ -471,7 +473,14 @@ static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
         else
             hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
     }
-    else if (cols4 <= 1024) launch_wave<K, 16, Ragged>(a, s);
+    else if (cols4 <= 1024) {
+        // 2049-4096 columns: a workgroup of 512 threads per row (8192 x 4096
+        // forward 47.1 -> 43.8 us, backward 67.8 -> 62.5; 512 x 4096 5.8 ->
+        // 4.7 and 6.5 -> 5.9 in graph replays), but one wave per row where the
+        // rows about fill the chip once (2048 x 4096 11.7 against 13.6).
+        if (a.rows > 1024 && a.rows < 3072) launch_wave<K, 16, Ragged>(a, s);
+        else hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true, Ragged, 512>), grid, dim3(512), 0, s, a);
+    }
     else if (cols4 <= 2048)
         hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
     else if (cols4 <= 4096)
@@ -499,8 +508,10 @@ static int softmax_launch(const SmArgs& a, hipStream_t s) {
                          (K != SmKind::Bwd || aligned16(a.b));
     if (aligned)
         softmax_dispatch<K, false>(a, s);
-    else
+    else if (a.cols >= 4)
         softmax_dispatch<K, true>(a, s);
+    else  // ragged rows are read four floats at a time
+        hipLaunchKernelGGL((softmax_loop_kernel<K, false>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
     return launch_status();
 }
 

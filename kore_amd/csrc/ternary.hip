@@ -31,13 +31,13 @@
 //   same for both operands, so any assignment gives the same sum);
 //   accumulator register r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
 //   column l % 32.
-// n <= 8: the small-n path (dot4 on decoded windows, no MFMA); 8 < n <= 64:
-// the skinny path (32 weight rows per workgroup, K split over its waves and
-// summed exactly in LDS); at least 144 tiles of 256 x 256: the wide kernel
-// (below); few output tiles beyond that: the tile kernel over
-// K ranges, summed with exact int32 atomics into the output (zeroed first,
-// finished in place).  Code rows that are not 16-byte aligned (K % 16 != 0
-// or an unaligned q) take the tile kernel with dword-window loads.
+// One code row (two with long K): the small-n path (dot4 on decoded windows, no
+// MFMA); then up to 256 tiles of 128 x 128 (k >= 16): the skinny path (32 or 64
+// weight rows per workgroup, K split over its waves and summed exactly in LDS);
+// at least 144 tiles of 256 x 256: the wide kernel (below); otherwise the tile
+// kernel.  Code rows that are not 16-byte aligned (K % 16 != 0 or an unaligned
+// q) take the skinny kernel and, beyond it, the tile kernel with dword-window
+// loads.
 // Generic path (K = 0, or an output not 4-byte aligned): one thread per
 // output, the reference loop order.
 //
@@ -75,7 +75,6 @@ struct TernArgs {
     const float* sq;    // [N]
     float* c;           // [M, N], or [N, M] with trans
     uint32_t m, n, k, kp;
-    uint32_t splits, kt_per;  // split-K: K-tile ranges of kt_per per workgroup
     const float* bias;  // [M] added to every output of row m, or null
     uint32_t trans;     // 1: output (m, n) at c[n * M + m] (BitLinear::forward's layout)
 };
@@ -118,11 +117,7 @@ __device__ __forceinline__ uint64_t trit_lut_entry(uint32_t b) {
 // dwordx4; otherwise as the five dwords around the 16 bytes, shifted into
 // place (a row's last partial piece, and the matrix's last bytes, byte by
 // byte).
-// kSplit: the workgroup covers K-tiles [split * kt_per, (split + 1) * kt_per)
-// of its output tile and adds its int32 sums into c (zeroed, read as int32)
-// with integer atomics -- exact and order-free, so the result is the same on
-// every run; ternary_i8_finish_kernel then applies the epilogue in place.
-template <bool kAlignedA, bool kAlignedB, bool kSplit, bool kTrans>
+template <bool kAlignedA, bool kAlignedB, bool kTrans>
 __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
     __shared__ uint64_t lut[256];
     __shared__ __attribute__((aligned(16))) uint8_t As[kTmM * kTmPitch];
@@ -138,12 +133,9 @@ __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
     // CU's neighbours work on share weights and codes in that XCD's L2.
     const uint32_t tm_n = (p.m + kTmM - 1) / kTmM, tn_n = (p.n + kTmN - 1) / kTmN;
     const uint32_t ntiles = tm_n * tn_n;
-    const uint32_t nwork = ntiles * (kSplit ? p.splits : 1u);
-    const uint32_t per = (nwork + kXcds - 1) / kXcds;
-    const uint32_t work = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-    if (work >= nwork) return;  // whole workgroup: no barrier reached yet
-    const uint32_t lin = kSplit ? work / p.splits : work;
-    const uint32_t kt_lo = kSplit ? (work % p.splits) * p.kt_per : 0u;
+    const uint32_t per = (ntiles + kXcds - 1) / kXcds;
+    const uint32_t lin = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+    if (lin >= ntiles) return;  // whole workgroup: no barrier reached yet
     const uint32_t grp = lin / (kGroupM * tn_n);
     const uint32_t first_m = grp * kGroupM;
     const uint32_t gsz = min(tm_n - first_m, (uint32_t)kGroupM);
@@ -157,8 +149,7 @@ __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
     const uint8_t* arow8 = p.a + (uint64_t)(arow_ok ? m0 + ar : 0) * p.kp;
     const u32x4* arow = reinterpret_cast<const u32x4*>(arow8);
     // B staging: 16-byte pieces c = t + 256u (u < 5) of the 128 x 160 tile.
-    const uint32_t nkt_all = (p.k + kTmK - 1) / kTmK;
-    const uint32_t nkt = kSplit ? min(nkt_all, kt_lo + p.kt_per) : nkt_all;
+    const uint32_t nkt = (p.k + kTmK - 1) / kTmK;
     const u32x4 zero_bytes = {kZeroByte * 0x01010101u, kZeroByte * 0x01010101u, kZeroByte * 0x01010101u,
                               kZeroByte * 0x01010101u};
     const u32x4 zero4 = {0u, 0u, 0u, 0u};
@@ -241,8 +232,8 @@ __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
 
     u32x4 av, bv[5];
     uint32_t ae = 0u, be[5] = {0u, 0u, 0u, 0u, 0u};
-    load_tile(kt_lo, av, ae, bv, be);
-    for (uint32_t kt = kt_lo; kt < nkt; ++kt) {
+    load_tile(0, av, ae, bv, be);
+    for (uint32_t kt = 0; kt < nkt; ++kt) {
         __syncthreads();  // previous tile's MFMA reads (and the LUT fill) are done
         if (!kAlignedA) av = shift20(av, ae, sh_a);
         if (!kAlignedB) {
@@ -320,12 +311,8 @@ __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
                 const uint32_t n = n0 + wn * 64 + j * 32 + (kTrans ? rr : cc);
                 if (n < p.n && m < p.m) {
                     const uint64_t o = out_idx(p, m, n);
-                    if (kSplit) {
-                        atomicAdd(reinterpret_cast<int*>(p.c) + o, acc[i][j][r]);
-                    } else {
-                        const float v = ((float)acc[i][j][r] * p.sa[m]) * p.sq[n];
-                        __builtin_nontemporal_store(add_bias(p.bias, v, m), p.c + o);
-                    }
+                    const float v = ((float)acc[i][j][r] * p.sa[m]) * p.sq[n];
+                    __builtin_nontemporal_store(add_bias(p.bias, v, m), p.c + o);
                 }
             }
         }
@@ -785,216 +772,280 @@ __global__ __launch_bounds__(256, 1) void ternary_i8_wide_kernel(TernArgs p) {
     }
 }
 
-// Skinny path (8 < n <= 64, the vector path's alignment): a decode batch
-// against a tall weight matrix.  A workgroup owns 32 weight rows and every
-// code row (NT tiles of 32); its kWaves waves split K (160-column blocks kb =
-// w, w + kWaves, ...), and their exact int32 partials meet in LDS, each wave
-// adding one slice of the accumulators over all waves in wave order -- no
-// atomics, no zero / finish launches.  A lane decodes its own weight row's
-// 16 packed bytes per block straight into MFMA operands: the k order inside a
-// block is permuted the same way for both operands (step s, lane half h ->
-// columns 80 h + 16 s .. + 16), which leaves each 32-deep MFMA's sum
-// unchanged.  The block's codes are read coalesced (10 lanes per 160-byte row
-// piece) into the wave's LDS tile, then read back as operands with that
-// mapping.  The next block's loads are in flight during the current block's
-// MFMAs.
-constexpr int kSkRows = 32;
-constexpr uint64_t kSkMaxN = 64;
+// Skinny path: decode batches and short prompts.  A workgroup owns 32 MR
+// weight rows and 32 NT code rows; its kWaves waves split K (160-column blocks
+// kb = w, w + kWaves, ...) and work alone until their exact int32 partials meet
+// in LDS, each wave adding one slice of the accumulators over all waves in wave
+// order -- no barrier in the K loop, no atomics, no zero / finish launches.  A
+// lane decodes its own weight rows' 16 packed bytes per block straight into
+// MFMA operands: the k order inside a block is permuted the same way for both
+// operands (step s, lane half h -> columns 80 h + 16 s .. + 16), which leaves
+// each 32-deep MFMA's sum unchanged.  The block's codes are read coalesced (10
+// lanes per 160-byte row piece) into the wave's LDS tile, then read back as
+// operands with that mapping.  The next block's loads are in flight during the
+// current block's MFMAs.
+// Code rows of any length and alignment (k >= 16): 16-byte loads need no
+// alignment; a row's last partial piece is read as its last 16 bytes and
+// shifted into place when it is staged.
 constexpr int kSkPitch = 176;  // LDS bytes per code row of a block (160 + 16)
 
-template <int NT, bool kAlignedA, int kWaves, bool kTrans>
+typedef uint32_t u32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+
+// v's 16 bytes moved down by sh (0..16) bytes, zeros behind them.
+__device__ __forceinline__ u32x4 bytes_down(u32x4 v, uint32_t sh) {
+    const uint32_t d = sh >> 2, b = sh & 3u;
+    const uint32_t w[4] = {v[0], v[1], v[2], v[3]};
+    uint32_t x[5];  // dwords moved down by d
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        x[i] = 0;
+#pragma unroll
+        for (int j = i; j < 4; ++j) x[i] = d == (uint32_t)(j - i) ? w[j] : x[i];
+    }
+    return u32x4{__builtin_amdgcn_alignbyte(x[1], x[0], b), __builtin_amdgcn_alignbyte(x[2], x[1], b),
+                 __builtin_amdgcn_alignbyte(x[3], x[2], b), __builtin_amdgcn_alignbyte(x[4], x[3], b)};
+}
+
+template <int NT, int kWaves> struct Skinny {
+    static constexpr int kTile = 32 * NT * kSkPitch;   // bytes of one wave's code tile
+    static constexpr int kPart = NT * kWave * 64;      // bytes of one wave's partial sums of 32 rows
+    static constexpr int kRegion = kTile > kPart ? kTile : kPart;
+    static constexpr size_t kLds = (size_t)256 * 8 + (size_t)kWaves * kRegion;
+};
+
+template <int MR, int NT, bool kAlignedA, int kWaves, bool kTrans>
 __global__ __launch_bounds__(kWaves * kWave) void ternary_i8_skinny_kernel(TernArgs p) {
-    constexpr int kRowsB = 32 * NT;                   // code rows of the workgroup
-    constexpr int kPieces = kRowsB * 10 / kWave;     // 16-byte code pieces per lane and block
-    constexpr int kTileB = kRowsB * kSkPitch;        // bytes of one wave's code tile
-    constexpr int kPart = NT * kWave * 64;           // bytes of one wave's partial sums
-    constexpr int kRegion = kTileB > kPart ? kTileB : kPart;
-    __shared__ uint64_t lut[256];
-    __shared__ __attribute__((aligned(16))) uint8_t smem[kWaves * kRegion];
+    using G = Skinny<NT, kWaves>;
+    constexpr int kPieces = 32 * NT * 10 / kWave;  // 16-byte code pieces per lane and block
+    extern __shared__ __attribute__((aligned(16))) uint8_t sklds[];
+    uint64_t* lut = reinterpret_cast<uint64_t*>(sklds);
+    uint8_t* smem = sklds + (size_t)256 * 8;
     const int t = threadIdx.x;
     const int lane = t & (kWave - 1);
-    const int wave = t / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
     const int r = lane & 31, h = lane >> 5;
-    uint8_t* region = smem + wave * kRegion;
-    if (t < 256) lut[t] = trit_lut_entry((uint32_t)t);
-    const uint32_t m0 = blockIdx.x * kSkRows;
-    const bool row_ok = m0 + r < p.m;
-    const uint8_t* arow8 = p.a + (uint64_t)(row_ok ? m0 + r : 0) * p.kp;
-    const uintptr_t a_hi = reinterpret_cast<uintptr_t>(p.a) + (uintptr_t)p.m * p.kp;
+    uint8_t* region = smem + wave * G::kRegion;
+    for (int e = t; e < 256; e += kWaves * kWave) lut[e] = trit_lut_entry((uint32_t)e);
+    // n-tiles fastest: the workgroups that share weight rows run together
+    const uint32_t ntn = (p.n + 32 * NT - 1) / (32 * NT);
+    const uint32_t m0 = blockIdx.x / ntn * (32 * MR), n0 = blockIdx.x % ntn * (32 * NT);
     const uint32_t nkb = (p.k + kTmK - 1) / kTmK;
-    const u32x4 zero_bytes = {kZeroByte * 0x01010101u, kZeroByte * 0x01010101u, kZeroByte * 0x01010101u,
-                              kZeroByte * 0x01010101u};
-    const u32x4 zero4 = {0u, 0u, 0u, 0u};
+    // Weight rows past m read row m - 1 (their outputs are not stored).
     // Unaligned rows: the 20 bytes from the dword boundary below the 16
     // (x and its fifth dword e), shifted into place by the row's byte offset
     // only when the block is decoded -- a shift right after the loads would
     // wait for them (and the code loads behind them) before the MFMAs that
     // are meant to cover them.  Bytes past a row's end meet only zero codes
-    // (code pieces at columns >= k are zero); only where the 20 bytes would
+    // (code pieces are zero at columns >= k); only where the 20 bytes would
     // pass the matrix's end are they read byte by byte.
-    const uint32_t sh_a = (uint32_t)(reinterpret_cast<uintptr_t>(arow8) & 3u);
-    auto load_a = [&](uint32_t kb, uint32_t& e) -> u32x4 {
+    const uint8_t* arow8[MR];
+    uint32_t sh_a[MR];
+#pragma unroll
+    for (int i = 0; i < MR; ++i) {
+        arow8[i] = p.a + (uint64_t)min(m0 + 32 * i + r, p.m - 1u) * p.kp;
+        sh_a[i] = (uint32_t)(reinterpret_cast<uintptr_t>(arow8[i]) & 3u);
+    }
+    const uintptr_t a_hi = reinterpret_cast<uintptr_t>(p.a) + (uintptr_t)p.m * p.kp;
+    auto load_a = [&](uint32_t kb, u32x4 (&av)[MR], uint32_t (&ae)[MR]) {
         const uint32_t ab = kb * kTmKp + 16u * h;
-        if (kAlignedA) return (row_ok && ab < p.kp) ? *reinterpret_cast<const u32x4*>(arow8 + ab) : zero_bytes;
-        const uintptr_t w0 = reinterpret_cast<uintptr_t>(arow8 + ab) & ~(uintptr_t)3;
-        if (__builtin_expect(w0 + 20u <= a_hi, 1)) {
-            e = *reinterpret_cast<const uint32_t*>(w0 + 16);
-            return *reinterpret_cast<const u32x4_a4*>(w0);
-        }
-        uint32_t w[5];
 #pragma unroll
-        for (int d = 0; d < 5; ++d) {
-            w[d] = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uintptr_t o = w0 + 4 * d + j;
-                w[d] |= (o < a_hi ? (uint32_t)*reinterpret_cast<const uint8_t*>(o) : 0u) << (8 * j);
+        for (int i = 0; i < MR; ++i) {
+            if (kAlignedA) {  // kp % 16 == 0: a window past kp reads the row's first one
+                av[i] = *reinterpret_cast<const u32x4*>(arow8[i] + (ab < p.kp ? ab : 0u));
+                continue;
             }
+            const uintptr_t w0 = reinterpret_cast<uintptr_t>(arow8[i] + ab) & ~(uintptr_t)3;
+            if (__builtin_expect(w0 + 20u <= a_hi, 1)) {
+                ae[i] = *reinterpret_cast<const uint32_t*>(w0 + 16);
+                av[i] = *reinterpret_cast<const u32x4_a4*>(w0);
+                continue;
+            }
+            uint32_t w[5];
+#pragma unroll
+            for (int d = 0; d < 5; ++d) {
+                w[d] = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uintptr_t o = w0 + 4 * d + j;
+                    w[d] |= (o < a_hi ? (uint32_t)*reinterpret_cast<const uint8_t*>(o) : 0u) << (8 * j);
+                }
+            }
+            ae[i] = w[4];
+            av[i] = u32x4{w[0], w[1], w[2], w[3]};
         }
-        e = w[4];
-        return u32x4{w[0], w[1], w[2], w[3]};
     };
-    // piece u of this lane: row (u * 64 + lane) / 10, 16-byte piece % 10
+    // piece u of this lane: row (u * 64 + lane) / 10 (past n: row n - 1, its
+    // outputs not stored), 16-byte piece % 10.  Pieces past or across the
+    // row's end read its last 16 bytes and are put right when staged.
+    const int8_t* qn0 = p.q + (uint64_t)n0 * p.k;
+    uint32_t brow[kPieces], bcol[kPieces];
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+        const uint32_t pc = (uint32_t)(u * kWave + lane);
+        brow[u] = min(pc / 10u, p.n - 1u - n0) * p.k;  // from row n0; at most 63 * 2^24
+        bcol[u] = 16u * (pc % 10u);
+    }
     auto load_b = [&](uint32_t kb, u32x4 (&bv)[kPieces]) {
+        const uint32_t c0 = kb * kTmK;
 #pragma unroll
         for (int u = 0; u < kPieces; ++u) {
-            const uint32_t pc = (uint32_t)(u * kWave + lane);
-            const uint32_t n = pc / 10u, c = kb * kTmK + 16u * (pc % 10u);
-            const bool ok = n < p.n && c < p.k;
-            const u32x4 v = *reinterpret_cast<const u32x4*>(p.q + (ok ? (uint64_t)n * p.k + c : 0u));
-            bv[u] = ok ? v : zero4;
+            const uint32_t c = min(c0 + bcol[u], p.k - 16u);
+            bv[u] = *reinterpret_cast<const u32x4_a1*>(qn0 + (brow[u] + c));
         }
     };
 
-    i32x16 acc[NT];
+    i32x16 acc[MR][NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int i = 0; i < MR; ++i)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[j][q] = 0;
-    __syncthreads();  // table filled
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0;
     uint32_t kb = (uint32_t)wave;
-    u32x4 av = zero_bytes;
-    uint32_t ae = 0u;
+    u32x4 av[MR];
+    uint32_t ae[MR];
     u32x4 bv[kPieces];
     if (kb < nkb) {
-        av = load_a(kb, ae);
+        load_a(kb, av, ae);
         load_b(kb, bv);
     }
+    __syncthreads();  // table filled
     for (; kb < nkb; kb += kWaves) {
         // this block's codes into the wave's tile (after the last block's reads)
+        if (kb == nkb - 1u) {
+#pragma unroll
+            for (int u = 0; u < kPieces; ++u) {
+                const uint32_t c = kb * kTmK + bcol[u];
+                bv[u] = bytes_down(bv[u], c + 16u <= p.k ? 0u : min(c + 16u - p.k, 16u));
+            }
+        }
         wave_lds_sync();
 #pragma unroll
         for (int u = 0; u < kPieces; ++u) {
             const uint32_t pc = (uint32_t)(u * kWave + lane);
             *reinterpret_cast<u32x4*>(region + (pc / 10u) * kSkPitch + 16u * (pc % 10u)) = bv[u];
         }
-        // decode this block's 16 packed bytes into 80 trits (20 dwords)
-        uint32_t out[20];
+        // decode this block's 16 packed bytes per row into 80 trits (20 dwords)
+        uint32_t out[MR][20];
 #pragma unroll
-        for (int d = 0; d < 20; ++d) out[d] = 0;
-        if (!kAlignedA)
-            av = u32x4{__builtin_amdgcn_alignbyte(av[1], av[0], sh_a), __builtin_amdgcn_alignbyte(av[2], av[1], sh_a),
-                       __builtin_amdgcn_alignbyte(av[3], av[2], sh_a), __builtin_amdgcn_alignbyte(ae, av[3], sh_a)};
-        uint64_t lv[16];
+        for (int i = 0; i < MR; ++i) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) lv[i] = lut[(av[i >> 2] >> (8 * (i & 3))) & 0xffu];
+            for (int d = 0; d < 20; ++d) out[i][d] = 0;
+            if (!kAlignedA)
+                av[i] = u32x4{__builtin_amdgcn_alignbyte(av[i][1], av[i][0], sh_a[i]),
+                              __builtin_amdgcn_alignbyte(av[i][2], av[i][1], sh_a[i]),
+                              __builtin_amdgcn_alignbyte(av[i][3], av[i][2], sh_a[i]),
+                              __builtin_amdgcn_alignbyte(ae[i], av[i][3], sh_a[i])};
+            uint64_t lv[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int off = 5 * i, d = off >> 2, sh = (off & 3) * 8;
-            out[d] |= (uint32_t)(lv[i] << sh);
-            out[d + 1] |= (uint32_t)(lv[i] >> (32 - sh));
+            for (int e = 0; e < 16; ++e) lv[e] = lut[(av[i][e >> 2] >> (8 * (e & 3))) & 0xffu];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int off = 5 * e, d = off >> 2, sh = (off & 3) * 8;
+                out[i][d] |= (uint32_t)(lv[e] << sh);
+                out[i][d + 1] |= (uint32_t)(lv[e] >> (32 - sh));
+            }
         }
         const uint32_t kn = kb + kWaves;
         if (kn < nkb) {
-            av = load_a(kn, ae);
+            load_a(kn, av, ae);
             load_b(kn, bv);
         }
         wave_lds_sync();
 #pragma unroll
         for (int s = 0; s < 5; ++s) {
-            const i32x4 a = {(int)out[4 * s], (int)out[4 * s + 1], (int)out[4 * s + 2], (int)out[4 * s + 3]};
+            i32x4 w[MR];
+#pragma unroll
+            for (int i = 0; i < MR; ++i)
+                w[i] = i32x4{(int)out[i][4 * s], (int)out[i][4 * s + 1], (int)out[i][4 * s + 2], (int)out[i][4 * s + 3]};
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 const i32x4 b = *reinterpret_cast<const i32x4*>(region + (32 * j + r) * kSkPitch + 80 * h + 16 * s);
-                acc[j] = mfma_wq<kTrans>(a, b, acc[j]);
+#pragma unroll
+                for (int i = 0; i < MR; ++i) acc[i][j] = mfma_wq<kTrans>(w[i], b, acc[i][j]);
             }
         }
     }
-    // every wave stores its partial sums; wave w then adds accumulator
-    // registers [w * kSlice, (w + 1) * kSlice) over all waves, in wave order
+    // 32 rows at a time, every wave stores its partial sums; wave w then adds
+    // accumulator quads w, w + kWaves, ... over all waves, in wave order
     // (exact), and applies the epilogue to them
-    __syncthreads();  // all waves are done with their code tiles
     i32x4* mypart = reinterpret_cast<i32x4*>(region);
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int i = 0; i < MR; ++i) {
+        __syncthreads();  // all waves are done with their code tiles, or the last 32 rows' sums
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-            mypart[(j * 4 + q4) * kWave + lane] = i32x4{acc[j][4 * q4], acc[j][4 * q4 + 1], acc[j][4 * q4 + 2],
-                                                        acc[j][4 * q4 + 3]};
-    __syncthreads();
-    constexpr int kQuads = NT * 4;  // 4-register groups per lane
-    for (int g = wave; g < kQuads; g += kWaves) {
-        i32x4 sum = {0, 0, 0, 0};
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) sum += reinterpret_cast<const i32x4*>(smem + w * kRegion)[g * kWave + lane];
-        const int j = g / 4, q4 = g % 4;
-        if (kTrans) {
-            // accumulator rows over n, lanes over m: stores run along c[n, m]'s rows
-            const uint32_t m = m0 + (uint32_t)r;
-            if (m < p.m) {
-                const float sam = p.sa[m];
+            for (int q4 = 0; q4 < 4; ++q4)
+                mypart[(j * 4 + q4) * kWave + lane] = i32x4{acc[i][j][4 * q4], acc[i][j][4 * q4 + 1],
+                                                            acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]};
+        __syncthreads();
+        const uint32_t mb = m0 + 32u * i;
+        constexpr int kQuads = NT * 4;  // 4-register groups per lane
+        for (int g = wave; g < kQuads; g += kWaves) {
+            i32x4 sum = {0, 0, 0, 0};
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w)
+                sum += reinterpret_cast<const i32x4*>(smem + w * G::kRegion)[g * kWave + lane];
+            const int j = g / 4, q4 = g % 4;
+            if (kTrans) {
+                // accumulator rows over n, lanes over m: stores run along c[n, m]'s rows
+                const uint32_t m = mb + (uint32_t)r;
+                if (m < p.m) {
+                    const float sam = p.sa[m];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t n = n0 + (uint32_t)j * 32u + 8u * q4 + 4u * h + e;  // register 4 q4 + e
+                        if (n < p.n) p.c[out_idx(p, m, n)] = add_bias(p.bias, ((float)sum[e] * sam) * p.sq[n], m);
+                    }
+                }
+                continue;
+            }
+            const uint32_t n = n0 + (uint32_t)j * 32u + (uint32_t)r;
+            if (n < p.n) {
+                const float sqn = p.sq[n];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint32_t n = (uint32_t)j * 32u + 8u * q4 + 4u * h + e;  // register 4 q4 + e
-                    if (n < p.n) p.c[out_idx(p, m, n)] = add_bias(p.bias, ((float)sum[e] * sam) * p.sq[n], m);
+                    const uint32_t m = mb + 8 * q4 + 4 * h + e;  // register 4 q4 + e
+                    if (m < p.m) p.c[out_idx(p, m, n)] = add_bias(p.bias, ((float)sum[e] * p.sa[m]) * sqn, m);
                 }
-            }
-            continue;
-        }
-        const uint32_t n = (uint32_t)j * 32u + (uint32_t)r;
-        if (n < p.n) {
-            const float sqn = p.sq[n];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t m = m0 + 8 * q4 + 4 * h + e;  // register 4 q4 + e
-                if (m < p.m) p.c[out_idx(p, m, n)] = add_bias(p.bias, ((float)sum[e] * p.sa[m]) * sqn, m);
             }
         }
     }
 }
 
-// Split-K helpers: zero c as int32 (a kernel, not hipMemsetAsync, so the
-// call can be captured in a graph), then turn the int32 sums into
-// ((float)acc * a_scale) * q_scale in place.
-__global__ __launch_bounds__(kTmBlock) void ternary_i8_zero_kernel(int32_t* c, uint64_t total) {
-    const uint64_t i = (uint64_t)blockIdx.x * kTmBlock + threadIdx.x;
-    if (i < total) c[i] = 0;
+template <int MR, int NT, int kWaves>
+static int launch_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
+    using G = Skinny<NT, kWaves>;
+    static_assert(G::kLds <= 160 * 1024, "skinny kernel LDS");
+    const uint64_t blocks = (uint64_t)((p.m + 32 * MR - 1) / (32 * MR)) * ((p.n + 32 * NT - 1) / (32 * NT));
+    if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+    const dim3 g((uint32_t)blocks), b(kWaves * kWave);
+    const auto launch = [&](auto A_, auto T_) {
+        constexpr bool A = decltype(A_)::value, T = decltype(T_)::value;
+        hipLaunchKernelGGL((ternary_i8_skinny_kernel<MR, NT, A, kWaves, T>), g, b, G::kLds, s, p);
+    };
+    if (aligned_a && p.trans) launch(std::true_type(), std::true_type());
+    else if (aligned_a) launch(std::true_type(), std::false_type());
+    else if (p.trans) launch(std::false_type(), std::true_type());
+    else launch(std::false_type(), std::false_type());
+    return launch_status();
 }
 
-__global__ __launch_bounds__(kTmBlock) void ternary_i8_finish_kernel(TernArgs p) {
-    const uint64_t i = (uint64_t)blockIdx.x * kTmBlock + threadIdx.x;
-    if (i >= (uint64_t)p.m * p.n) return;
-    const uint32_t m = (uint32_t)(p.trans ? i % p.m : i / p.n), n = (uint32_t)(p.trans ? i / p.m : i % p.n);
-    const int32_t acc = reinterpret_cast<const int32_t*>(p.c)[i];
-    p.c[i] = add_bias(p.bias, ((float)acc * p.sa[m]) * p.sq[n], m);
-}
-
-// Small-n path (n <= 8, k % 8 == 0, 8-byte aligned codes): a group of waves
+// Small-n path (one or two code rows, k % 8 == 0, 8-byte aligned codes): a group of waves
 // owns 4 weight rows and every lane a 40-column window of them (8 packed
-// bytes per row), decoded through the LDS table and reused for up to 4 code
-// rows at a time: 10 v_dot4_i32_i8 per row and code row, then exact integer
+// bytes per row), decoded through the LDS table and reused for both code
+// rows: 10 v_dot4_i32_i8 per row and code row, then exact integer
 // wave sums (DPP) and the same epilogue.  K is walked in chunks of 2560
 // columns (512 packed bytes) shared by the group's waves.  Bound by the
 // packed weights' bytes (m * ceil(k/5)) and latency where the MFMA tiles
 // would waste most of their columns.
 constexpr int kGvRows = 4;     // weight rows per wave group
 constexpr int kGvChunk = 2560; // columns per lane-window sweep (64 lanes x 40)
-// Largest n the small-n path takes, by measured crossover against the
-// split-K MFMA tiles: n = 8 is faster here (6912 x 8 x 2560: 10.4 vs 10.7 us;
-// 2560 x 8 x 6912: 13.6 vs 15.9 us), n = 16 is not (6912 x 16 x 2560: 18.5
-// vs 10.4 us).  It also spares k % 16 == 8 shapes the one-thread-per-output
-// kernel (2560 x 8 x 6920: 12.5 vs 334 us).
-constexpr uint64_t kGvMaxN = 8;
+// One code row, and two from this many columns; the skinny kernel takes the
+// others (measured, graph replays: 6912 x 2 x 2560 5.2 us here against 4.8, x 8
+// 12.0 against 5.1; 2560 x 2 x 6912 6.8 against 7.8, x 4 9.0 against 8.1).
+constexpr uint64_t kGvTwoK = 5120;
 
 __device__ __forceinline__ int32_t wave_sum_i32(int32_t v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
@@ -3317,20 +3368,19 @@ __global__ __launch_bounds__(kPackWaves * kWave) void ternary_pack_kernel(const 
 }  // namespace kore
 
 namespace kore {
-template <bool kSplit, bool kTrans>
+template <bool kTrans>
 static void launch_mfma_t(bool aligned_a, bool aligned_b, dim3 grid, hipStream_t s, const TernArgs& p) {
     if (aligned_a && aligned_b)
-        hipLaunchKernelGGL((ternary_i8_mfma_kernel<true, true, kSplit, kTrans>), grid, dim3(kTmBlock), 0, s, p);
+        hipLaunchKernelGGL((ternary_i8_mfma_kernel<true, true, kTrans>), grid, dim3(kTmBlock), 0, s, p);
     else if (aligned_b)
-        hipLaunchKernelGGL((ternary_i8_mfma_kernel<false, true, kSplit, kTrans>), grid, dim3(kTmBlock), 0, s, p);
+        hipLaunchKernelGGL((ternary_i8_mfma_kernel<false, true, kTrans>), grid, dim3(kTmBlock), 0, s, p);
     else if (aligned_a)
-        hipLaunchKernelGGL((ternary_i8_mfma_kernel<true, false, kSplit, kTrans>), grid, dim3(kTmBlock), 0, s, p);
-    else hipLaunchKernelGGL((ternary_i8_mfma_kernel<false, false, kSplit, kTrans>), grid, dim3(kTmBlock), 0, s, p);
+        hipLaunchKernelGGL((ternary_i8_mfma_kernel<true, false, kTrans>), grid, dim3(kTmBlock), 0, s, p);
+    else hipLaunchKernelGGL((ternary_i8_mfma_kernel<false, false, kTrans>), grid, dim3(kTmBlock), 0, s, p);
 }
-template <bool kSplit>
 static void launch_mfma(bool aligned_a, bool aligned_b, dim3 grid, hipStream_t s, const TernArgs& p) {
-    if (p.trans) launch_mfma_t<kSplit, true>(aligned_a, aligned_b, grid, s, p);
-    else launch_mfma_t<kSplit, false>(aligned_a, aligned_b, grid, s, p);
+    if (p.trans) launch_mfma_t<true>(aligned_a, aligned_b, grid, s, p);
+    else launch_mfma_t<false>(aligned_a, aligned_b, grid, s, p);
 }
 // Two-workgroups-per-CU path (the wide path's shapes): a workgroup owns a
 // 256 (m) x 128 (n) output tile, wave w its weight rows [64 w, 64 w + 64)
@@ -3686,6 +3736,37 @@ static void launch_wide(bool aligned_a, dim3 g, hipStream_t s, const TernArgs& p
 
 using namespace kore;
 
+// Where the skinny kernel runs: up to 256 tiles of 128 x 128 (the tile kernel's:
+// one round of the CUs, its K split over workgroups and summed with atomics in
+// two more launches where they are few).  Its form follows from how many
+// workgroups each gives.  Measured in graph replays, us, m x k at n codes:
+//   6912 x 2560: n = 8 (the small-n kernel before) 12.0 -> 5.1, 100 (the tile
+//     kernel, as all that follow) 24.0 -> 10.6, 200 29.9 -> 16.3, 400 32.2 ->
+//     27.4; at 800 (378 tiles) the tile kernel's 39.7 against 41.2;
+//   2560 x 6912: 45 (32 rows x 64 codes, 8 waves before) 11.7 -> 8.8, 200 28.5
+//     -> 17.6, 400 39.9 -> 30.4, 800 67 -> 47;
+//   3712 x 2375 (code rows not 16-byte aligned): 1 16.6 -> 5.2, 45 17.3 -> 7.1,
+//     200 27.4 -> 13.4, 800 42.8 -> 31.4;
+//   1024 x 1001: 100 13.9 -> 5.7, 800 17.7 -> 10.2.
+static bool skinny_wins(uint64_t m, uint64_t n) {
+    return ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN) <= 256;
+}
+
+static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
+    const uint64_t m32 = (p.m + 31) / 32, n32 = (p.n + 31) / 32, m64 = (p.m + 63) / 64, n64 = (p.n + 63) / 64;
+    // 32 x 32 outputs a workgroup of 8 waves while that is up to two a CU (more
+    // of them, shorter; 2560 x 45 x 6912 8.8 us against 11.7 with 32 x 64, 3712
+    // x 100 x 2375 10.0 against 12.6 with 64 x 64);
+    if (n32 == 1 || m32 * n32 <= (n64 == 1 ? 416u : 512u)) return launch_skinny<1, 1, 8>(p, aligned_a, s);
+    // one code tile: 32 x 64 (6912 x 64 x 2560 7.0 against 7.6);
+    if (n64 == 1) return launch_skinny<1, 2, 8>(p, aligned_a, s);
+    // then 64 x 64, each staged code read by two MFMAs, of 8 waves up to one a
+    // CU (3712 x 200 x 2375 13.4 against 14.9) and of 4 beyond (6912 x 200 x
+    // 2560 16.3 against 19.8).
+    if (m64 * n64 <= kCus) return launch_skinny<2, 2, 8>(p, aligned_a, s);
+    return launch_skinny<2, 2, 4>(p, aligned_a, s);
+}
+
 // The int8 matmul with the output in either layout (trans: c[n, m]) and an
 // optional bias per weight row.
 static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const int8_t* q, const float* q_scales,
@@ -3700,8 +3781,7 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
     if (!mul_ok(m, n, &mn) || mn > kMaxElements || !mul_ok(n, k, &nk) || nk > kMaxElements)
         return KORE_HIP_ERR_OVERFLOW;
     const uint64_t kp = (k + 4) / 5;
-    // c is written (and, with split-K, zeroed first) while the inputs are
-    // read: it must not overlap any of them.
+    // c is written while the inputs are read: it must not overlap any of them.
     {
         const char* c0 = reinterpret_cast<const char*>(c);
         const char* c1 = c0 + mn * sizeof(float);
@@ -3713,41 +3793,24 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
             if (in.p && in.bytes && i0 < c1 && c0 < i0 + in.bytes) return KORE_HIP_ERR_ALIAS;
         }
     }
-    TernArgs p{a_packed, a_scales, q,  q_scales, c, (uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)kp, 1u, 0u,
+    TernArgs p{a_packed, a_scales, q,  q_scales, c, (uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)kp,
                bias,     trans ? 1u : 0u};
     const bool c_ok = (reinterpret_cast<uintptr_t>(c) & 3u) == 0;
-    if (n <= kGvMaxN && k > 0 && k % 8 == 0 && (reinterpret_cast<uintptr_t>(q) & 7u) == 0 && c_ok) {
+    if (n <= (k > kGvTwoK ? 2u : 1u) && k > 0 && k % 8 == 0 && (reinterpret_cast<uintptr_t>(q) & 7u) == 0 && c_ok) {
         // grid: at most m / 4 blocks of one wave group (m < 2^31)
         const bool al8 = kp % 8 == 0 && (reinterpret_cast<uintptr_t>(a_packed) & 7u) == 0;
         if (al8) {
             if (n <= 1) launch_gemv<1, true>(p, m, k, s);
-            else if (n <= 2) launch_gemv<2, true>(p, m, k, s);
-            else launch_gemv<4, true>(p, m, k, s);
+            else launch_gemv<2, true>(p, m, k, s);
         } else {
             if (n <= 1) launch_gemv<1, false>(p, m, k, s);
-            else if (n <= 2) launch_gemv<2, false>(p, m, k, s);
-            else launch_gemv<4, false>(p, m, k, s);
+            else launch_gemv<2, false>(p, m, k, s);
         }
         return launch_status();
     }
     const bool vec = k > 0 && k % 16 == 0 && aligned16(q) && c_ok;
-    if (vec && n <= kSkMaxN) {
-        const uint64_t blocks = (m + kSkRows - 1) / kSkRows;
-        if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-        const bool al = kp % 16 == 0 && aligned16(a_packed);
-        const dim3 g((uint32_t)blocks);
-        const int nt = (int)((n + 31) / 32);
-#define KORE_SKINNY(NT, AL, TR) hipLaunchKernelGGL((ternary_i8_skinny_kernel<NT, AL, 8, TR>), g, dim3(8 * kWave), 0, s, p)
-        if (trans) {
-            if (al) { if (nt == 1) KORE_SKINNY(1, true, true); else KORE_SKINNY(2, true, true); }
-            else { if (nt == 1) KORE_SKINNY(1, false, true); else KORE_SKINNY(2, false, true); }
-        } else {
-            if (al) { if (nt == 1) KORE_SKINNY(1, true, false); else KORE_SKINNY(2, true, false); }
-            else { if (nt == 1) KORE_SKINNY(1, false, false); else KORE_SKINNY(2, false, false); }
-        }
-#undef KORE_SKINNY
-        return launch_status();
-    }
+    if (k >= 16 && c_ok && skinny_wins(m, n))
+        return ternary_i8_skinny(p, kp % 16 == 0 && aligned16(a_packed), s);
     const uint64_t wide_tiles = ((m + kWdM - 1) / kWdM) * ((n + kWdN - 1) / kWdN);
     if (vec && wide_tiles >= kWdMinTiles && nk < (1ull << 31)) {
         // Many output tiles: the wide kernel (one 256 x 256 tile per CU), or
@@ -3786,30 +3849,9 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
     if (k > 0 && c_ok) {
         // codes 16-byte aligned row by row (vec) or not
         const uint64_t tiles = ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN);
-        const uint64_t nkt = (k + kTmK - 1) / kTmK;
-        // Few output tiles (small m * n): split K so that ~512 workgroups run,
-        // each over at least two K-tiles.
-        uint64_t splits = 1;
-        if (tiles < 128 && nkt >= 4) {
-            splits = std::min<uint64_t>(nkt / 2, (512 + tiles - 1) / tiles);
-            const uint64_t kt_per = (nkt + splits - 1) / splits;
-            splits = (nkt + kt_per - 1) / kt_per;
-            p.splits = (uint32_t)splits;
-            p.kt_per = (uint32_t)kt_per;
-        }
-        const uint64_t work = tiles * splits;
-        const uint64_t per = (work + kXcds - 1) / kXcds;
+        const uint64_t per = (tiles + kXcds - 1) / kXcds;
         if (per * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-        const dim3 grid((uint32_t)(per * kXcds));
-        const bool al = kp % 16 == 0 && aligned16(a_packed);
-        if (splits > 1) {
-            const dim3 eg((uint32_t)((mn + kTmBlock - 1) / kTmBlock));
-            hipLaunchKernelGGL(ternary_i8_zero_kernel, eg, dim3(kTmBlock), 0, s, reinterpret_cast<int32_t*>(c), mn);
-            launch_mfma<true>(al, vec, grid, s, p);
-            hipLaunchKernelGGL(ternary_i8_finish_kernel, eg, dim3(kTmBlock), 0, s, p);
-        } else {
-            launch_mfma<false>(al, vec, grid, s, p);
-        }
+        launch_mfma(kp % 16 == 0 && aligned16(a_packed), vec, dim3((uint32_t)(per * kXcds)), s, p);
     } else {
         const uint64_t blocks = (mn + kTmBlock - 1) / kTmBlock;
         if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;

@@ -1,0 +1,49 @@
+"""Every form of the int8 ternary matmul around the sizes where the choice between them changes, on code rows and packed
+rows of every alignment: bit-exact against the oracle (an exact integer sum, one epilogue)."""
+import numpy as np
+import pytest
+
+import oracle
+from inputs import assert_bitexact, normal, raw_packed, rng
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from kore_amd import rocm  # noqa: E402
+from kore_amd.rocm import HipBuffer  # noqa: E402
+
+DEV = 0
+
+
+def at(arr: np.ndarray, offset: int) -> HipBuffer:
+    """arr's bytes on the device, `offset` bytes past a 16-byte boundary, with nothing of the allocation after them."""
+    raw = torch.from_numpy(np.ascontiguousarray(arr).reshape(-1).view(np.uint8).copy())
+    t = torch.empty(offset + raw.numel(), dtype=torch.uint8, device="cuda:0")
+    t[offset:].copy_(raw)
+    return HipBuffer.from_tensor(t[offset:])
+
+
+# m, n, k, byte offset of the codes, of the packed rows.  Two codes either side of the small-n path's K; one block of 32
+# codes and the next; the number of workgroups around each form's limit (32 x 32 to 416, 64 x 64 of 8 waves to 256, of 4
+# beyond, 256 tiles of 128 x 128 then the tile kernel); K of one partial piece, one block, and one column more or less.
+FORMS = [(5, 1, 15, 0, 0), (5, 1, 16, 0, 0), (33, 1, 17, 1, 1), (64, 2, 5120, 0, 0), (64, 2, 5128, 0, 0), (7, 2, 2563, 3, 2),
+         (300, 3, 2560, 0, 0), (129, 8, 2568, 0, 0), (31, 32, 31, 5, 3), (32, 33, 159, 0, 0), (65, 33, 160, 0, 0),
+         (64, 31, 161, 9, 1), (97, 40, 1001, 7, 0), (6656, 64, 320, 0, 0), (6657, 64, 320, 0, 0), (6657, 45, 175, 15, 3),
+         (4096, 65, 163, 0, 0), (8200, 65, 336, 0, 0), (8192, 100, 164, 2, 1), (1024, 1000, 177, 0, 0),
+         (2100, 1000, 1283, 1, 0), (4096, 1024, 165, 0, 2), (4100, 1024, 176, 0, 0), (4100, 1020, 171, 3, 1),
+         (70, 3000, 335, 0, 0), (1, 4000, 480, 0, 0)]
+
+
+@pytest.mark.parametrize("m,n,k,oq,oa", FORMS)
+def test_ternary_i8_forms(m, n, k, oq, oa):
+    print(f"ternary i8 m={m} n={n} k={k} codes+{oq} packed+{oa}", flush=True)
+    p = raw_packed(m, k, m + k)
+    q = rng(n + k).integers(-128, 128, size=(n, k), dtype=np.int64).astype(np.int8)
+    sa, sq = normal((m,), 8, 1.0, 0.1), np.abs(normal((n,), 9, 0.02, 0.005))
+    bias = normal((m,), 10)
+    want = oracle.ternary_matmul_i8(p, sa, q, sq, m, n, k)
+    ab, qb, sab, sqb = at(p, oa), at(q, oq), at(sa, 0), at(sq, 0)
+    got = rocm.rocm_ternary_matmul_i8(DEV, ab, sab, qb, sqb, m, n, k).to_host(np.float32).reshape(m, n)
+    assert_bitexact(got, want, "c[m, n]")
+    got = rocm.rocm_bit_linear_i8(DEV, ab, sab, qb, sqb, at(bias, 0), m, n, k).to_host(np.float32).reshape(n, m)
+    assert_bitexact(got, want.T + bias, "layer")

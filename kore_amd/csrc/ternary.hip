@@ -1984,12 +1984,10 @@ __global__ __launch_bounds__(W * kWave) void ternary_f32_rows_dma_kernel(TernF32
 // LDS once per R rows; measured: 16- and 32-column tiles ran 6-12% slower
 // with 4 than with 2 at every m tried, 64-column tiles 8-20% faster) while
 // that leaves at least 1.5 waves per SIMD, else fewer.
-template <int CT, bool TM>
-static int launch_f32_rows(uint64_t m, uint64_t n, hipStream_t s, const TernF32Args& p) {
-    constexpr uint64_t kSlots = kWave / CT;
-    const uint64_t gy = (n + CT - 1) / CT;
-    uint32_t r = CT == 64 ? 4 : 2;
-    if (r == 4 && (m + 4 * kSlots - 1) / (4 * kSlots) * gy < kRowsMinWaves) r = 2;
+static uint32_t f32_rows_per_lane(uint64_t m, uint64_t gy, int ct) {
+    const uint64_t slots = (uint64_t)(kWave / ct);
+    uint32_t r = ct == 64 ? 4 : 2;
+    if (r == 4 && (m + 4 * slots - 1) / (4 * slots) * gy < kRowsMinWaves) r = 2;
     if (r == 4) {
         // Many rows: the SIMDs run the waves in rounds, so R rows per wave
         // cost R * ceil(waves / 1024); 5 or 7 rows where that is lower and
@@ -2004,7 +2002,15 @@ static int launch_f32_rows(uint64_t m, uint64_t n, hipStream_t s, const TernF32A
             if (best == 0 || rr * rounds < best) best = rr * rounds, r = rr;
         }
     }
-    if ((m + 2 * kSlots - 1) / (2 * kSlots) * gy < kRowsMinWaves) r = 1;
+    if ((m + 2 * slots - 1) / (2 * slots) * gy < kRowsMinWaves) r = 1;
+    return r;
+}
+
+template <int CT, bool TM>
+static int launch_f32_rows(uint64_t m, uint64_t n, hipStream_t s, const TernF32Args& p) {
+    constexpr uint64_t kSlots = kWave / CT;
+    const uint64_t gy = (n + CT - 1) / CT;
+    const uint32_t r = f32_rows_per_lane(m, gy, CT);
     constexpr uint32_t W = TM ? kRowsWTm : kRowsW;
     const uint64_t rows = r * kSlots * W;  // rows per workgroup
     const uint64_t bx = (m + rows - 1) / rows;
@@ -2396,11 +2402,12 @@ __global__ __launch_bounds__(kMfThreads) void ternary_f32_mfma_kernel(TernF32Arg
     }
 }
 
-// The matrix-core kernel where its waves (64 rows x 16 columns each, one
-// dependent chain of k MFMAs) give most SIMDs one: with fewer, the vector
+// [K, N] b: the matrix-core kernel where its waves (64 rows x 16 columns each,
+// one dependent chain of k MFMAs) give most SIMDs one: with fewer, the vector
 // kernel's shorter chains win (measured: 6912 x 128 x 2560 83 against
 // 103 us, 6912 x 64 x 2560 76-82 against 68-70, 2560 x 256 x 6912 214
-// against 209; from 1024 columns about 2x).
+// against 209; from 1024 columns about 2x).  The layer's token-major b:
+// f32_layer_form.
 constexpr uint64_t kMfMinWaves = 768;
 static bool f32_use_mfma(uint64_t m, uint64_t n, uint64_t k) {
     return k > 0 && k < (1ull << 31) && ((m + 63) / 64) * ((n + 15) / 16) >= kMfMinWaves;
@@ -2543,7 +2550,7 @@ __global__ __launch_bounds__(W * kWave) void ternary_f32_mf4_kernel(TernF32Args 
             e[5] = e[6] = e[7] = 0.0f;
         }
     };
-    // b staging.  b is below 6 MB here (n <= 192, k <= 7680) and loads
+    // b staging.  b is below 2 GB here (the dispatch's condition) and loads
     // through a range-checked resource at 32-bit byte offsets fixed for the
     // kernel: a column past n sits past the end of b and reads zeros, and
     // the resource checks each dword.
@@ -2852,30 +2859,55 @@ static uint32_t f32_mf4_slice(uint64_t kp) {
     return words * 4u <= kM4MaxSlice ? (uint32_t)(words * 4u) : 0u;
 }
 
-// Where the 4 x 4 kernel runs: 41 to 192 columns, K from 2560 (its fixed
-// costs -- the packed-row copy, the staging prologue -- spread over enough
-// chunks), no 16 x 16 launch for the shape, and at least 640 waves of 4
-// rows x 64 columns with token-major b (the layer), 1024 with [K, N] b (the
-// plain ternary_matmul).  Up to 1024 waves a SIMD runs one wave, whose
-// chain time does not shrink with m, so below that the row-broadcast
-// kernel, whose time does, wins at some m.  Measured (HIP events; the
-// row-broadcast kernel on the same box; layer, then [K, N]):
-//   6912 x 64 x 2560 (1728 waves): 42.2 and 46.0 us against 70 and 66;
-//   6912 x 96 x 2560: 81 and 90 against 107 and 102;
-//   2560 x {96, 192} x 6912 (1280-1920 waves): 105-110 and 116-125 against
-//   143-195;
-//   2560 x 64 x 6912 (640 waves): 104 and 114 against 116 and 104;
-//   3500 x 64 x 4096 (875 waves): 64 and 71 against 67 and 71;
-//   3000 x 64 x 2560 (750 waves): 40.5 and 45.1 against 45.4 and 42.1;
-//   2048 x 64 x 6912 (512 waves): 104 and 114 against 80 and 80;
-//   24 and 32 columns: 47-49 against 38-39 us at 6912 x 2560 (the 64-column
-//   waves half empty).
+// Where the 4 x 4 kernel runs on [K, N] b: 41 to 192 columns, K from 2560 (its
+// fixed costs -- the packed-row copy, the staging prologue -- spread over
+// enough chunks), no 16 x 16 launch for the shape, and at least 1024 waves of 4
+// rows x 64 columns.  Up to 1024 waves a SIMD runs one wave, whose chain time
+// does not shrink with m, so below that the row-broadcast kernel, whose time
+// does, wins at some m.  Measured (HIP events; the row-broadcast kernel on the
+// same box): 6912 x 64 x 2560 (1728 waves) 46.0 us against 66, 6912 x 96 x 2560
+// 90 against 102, 2560 x {96, 192} x 6912 (1280-1920 waves) 116-125 against
+// 143-195, 2560 x 64 x 6912 (640 waves) 114 against 104, 3500 x 64 x 4096 (875
+// waves) 71 against 71, 2048 x 64 x 6912 (512 waves) 114 against 80.
 // Two chains per wave (8 rows, each b read shared by both; 864 waves at
 // 6912 x 64) measured 5% slower, and workgroups of 7 waves (247 instead of
 // 216 workgroups at 6912 rows, one per CU) 6% slower.
-static bool f32_use_mf4(uint64_t m, uint64_t n, uint64_t k, uint64_t kp, bool tm) {
+static bool f32_use_mf4(uint64_t m, uint64_t n, uint64_t k, uint64_t kp) {
     if (n < 41 || n > 192 || k < 2560 || f32_use_mfma(m, n, k) || f32_mf4_slice(kp) == 0) return false;
-    return (m + 3) / 4 * ((n + kWave - 1) / kWave) >= (tm ? 640u : 1024u);
+    return (m + 3) / 4 * ((n + kWave - 1) / kWave) >= 1024u;
+}
+
+// The layer (token-major b) takes the form with the least expected time.  All
+// three are chains over k, so a form costs its time per K column times the
+// rounds its waves (or workgroups) need, plus a start; the constants (us, us
+// per K column) are fitted to every form forced on 8 matrices (512-6912 rows,
+// K 896-6912) at 16 to 600 columns, and within 15% of nearly all of them:
+//   16 x 16: 2560 x 200 x 6912 145 us (189 where the row-broadcast kernel ran
+//     below 768 waves), 6912 x 96 x 2560 57 (79.5 4 x 4), 3712 x 200 x 2375 58
+//     (110), 5376 x 96 x 896 25 (39);
+//   4 x 4: 3712 x 96 x 2375 41 (56 where it needed K >= 2560), 2048 x 200 x 2048
+//     35 (50), 6912 x 40 x 2560 43 (59 below 41 columns);
+//   row-broadcast: 2560 x 64 x 6912 89 (102 from 640 waves of the 4 x 4).
+// Up to 32 columns the row-broadcast kernel's narrower tiles win everywhere
+// (6912 x 32 x 2560 37 against 43 and 56).
+enum class F32Form { Rows, Mf4, Mfma };
+static F32Form f32_layer_form(uint64_t m, uint64_t n, uint64_t k, uint64_t kp) {
+    if ((n + 15) / 16 > 65535) return F32Form::Mfma;  // refused there, as ever
+    if (n <= 32) return F32Form::Rows;
+    const uint64_t n64 = (n + 63) / 64;
+    const auto rounds = [](uint64_t have, uint64_t at_once) { return (double)((have + at_once - 1) / at_once); };
+    const double kd = (double)k;
+    const double mfma = 4.0 + kd * (0.0072 + 0.0139 * rounds((m + 63) / 64 * ((n + 15) / 16), kSimds));
+    const double mf4 = 4.0 + kd * 0.0150 * rounds((m + 3) / 4 * n64, 2 * kSimds);
+    // row-broadcast: by rows per lane, and by workgroups on a CU
+    const uint32_t r = f32_rows_per_lane(m, n64, 64);
+    const double per = r == 1 ? 0.0081 : (r == 2 ? 0.0136 : 0.0056 * r);
+    const double wgs = rounds((m + r * kRowsWTm - 1) / (r * kRowsWTm) * n64, kCus);
+    const double rows = 3.0 + kd * per * (wgs <= 1.0 ? 1.0 : (wgs <= 2.0 ? 1.63 : 0.8 * wgs));
+    // the 4 x 4 kernel's 32-bit offsets: b below 2 GB
+    const bool mf4_ok = f32_mf4_slice(kp) != 0 && n * k < (1ull << 29) - 1024;
+    if (mf4_ok && mf4 <= mfma && mf4 <= rows) return F32Form::Mf4;
+    return mfma <= rows ? F32Form::Mfma : F32Form::Rows;
 }
 
 template <bool TM, int CH, int W>
@@ -3917,12 +3949,16 @@ static int ternary_f32_run(const uint8_t* a_packed, const float* a_scales, const
             q.m = (uint32_t)std::min<uint64_t>(span, m - r0);
             q.c += trans ? r0 : r0 * n;  // c[n, m]: columns r0 .. of every row, row stride m
             if (bias) q.bias += r0;
-            if (f32_use_mf4(q.m, n, k, kp, tm)) {
+            const F32Form form = tm ? f32_layer_form(q.m, n, k, kp)
+                                    : f32_use_mf4(q.m, n, k, kp)  ? F32Form::Mf4
+                                    : f32_use_mfma(q.m, n, k) ? F32Form::Mfma
+                                                              : F32Form::Rows;
+            if (form == F32Form::Mf4) {
                 const int st = tm ? launch_f32_mf4<true>(q.m, n, s, q) : launch_f32_mf4<false>(q.m, n, s, q);
                 if (st != KORE_HIP_OK) return st;
                 continue;
             }
-            if (f32_use_mfma(q.m, n, k)) {
+            if (form == F32Form::Mfma) {
                 const int st = tm ? launch_f32_mfma<true>(q.m, n, s, q) : launch_f32_mfma<false>(q.m, n, s, q);
                 if (st != KORE_HIP_OK) return st;
                 continue;

@@ -51,7 +51,7 @@ template <bool Ragged, bool Stream = true>
 __device__ __forceinline__ f32x4 ld_row4(const float* row, uint32_t f, uint32_t n) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (!Ragged) {
-        if (4 * f < n) {
+        if (f < n >> 2) {
             const f32x4* p = reinterpret_cast<const f32x4*>(row) + f;
             v = Stream ? ld_stream(p) : *p;
         }
@@ -92,7 +92,7 @@ template <bool Ragged, bool Stream = true>
 __device__ __forceinline__ void st_row4(float* row, uint32_t f, uint32_t n, f32x4 v) {
     if (!Ragged) {
         f32x4* p = reinterpret_cast<f32x4*>(row) + f;
-        if (4 * f < n) {
+        if (f < n >> 2) {
             if (Stream) st_stream(p, v);
             else *p = v;
         }

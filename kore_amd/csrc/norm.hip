@@ -352,7 +352,8 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     };
 
     // ---- HBM reads: coalesced, chunk-major, all in flight.
-    const float* xr = args.x + row * (FULL ? (uint64_t)(4 * kWave * SL4 * W) : args.cols);
+    const uint64_t row_at = row * (FULL ? (uint64_t)(4 * kWave * SL4 * W) : args.cols);
+    const float* xr = args.x + row_at;
     f32x4 xv[NCH];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) xv[c] = ld(xr, part0 + (uint32_t)c * kWave + lane);
@@ -567,7 +568,7 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     const float inv = 1.0f / sqrtf(ss / (float)args.cols + args.eps);
 
     f32x4 last = zero;  // RAGGED: the row's last float4, in the lane that holds it
-    float* yr = args.y + row * args.cols;
+    float* yr = args.y + row_at;
     auto st = [&](uint32_t f, f32x4 v) {
         if (RAGGED) {
             if (f < whole4) __builtin_nontemporal_store((f32x4_a4)v, reinterpret_cast<f32x4_a4*>(yr) + f);
@@ -596,7 +597,7 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
         st_last();
     } else if (Out == NormOut::SiluGate) {
         // cpu_fused.rs:466-471: x_hat = (x*inv)*g; y = x_hat * silu(z).
-        const float* zr = args.z + row * args.cols;
+        const float* zr = args.z + row_at;
         // x_hat first, so that the weights are dead before z is loaded
         // (keeps the 2560-column kernel within 128 VGPRs: four waves a SIMD)
 #pragma unroll
@@ -635,7 +636,7 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
             for (int w = 0; w < W; ++w) amax = fmaxf(amax, meet[W + w]);
             amax = read_lane(amax, 0);
         }
-        int8_t* qr = args.q + row * args.cols;
+        int8_t* qr = args.q + row_at;
         uint32_t last_q = 0;
         auto st_q = [&](uint32_t f, uint32_t d) {
             if (RAGGED) {

@@ -69,10 +69,10 @@ __device__ __forceinline__ float sum4(f32x4 a) { return (a.x + a.y) + (a.z + a.w
 // sweeps one contiguous band of rows (measured 89 -> 80 us at 16384 x 2048
 // against giving each workgroup a contiguous block of rows).  Per row, the S
 // waves' partial sums meet in LDS (slot parity double-buffered, one barrier
-// per iteration) and are added in q order.  Each wave keeps its dgamma partial
-// in registers; at the end the row slots' partials are added in j order
-// through LDS and written as partial row b.  Rows from dx_rows on leave their
-// inv and coeff in ws instead of writing dx.
+// per iteration) and are added in q order (by a fixed tree for S >= 8).  Each
+// wave keeps its dgamma partial in registers; at the end the row slots'
+// partials are added in j order through LDS and written as partial row b.
+// Rows from dx_rows on leave their inv and coeff in ws instead of writing dx.
 // Ragged: rows of any length and alignment (see ld_row4).
 template <int NCHW, int S, int kWaves, bool Ragged>
 __global__ __launch_bounds__(kWave * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
@@ -80,14 +80,17 @@ void rms_bwd_rows_kernel(BwArgs a) {
     constexpr bool kLong = kWaves != kBwWaves;
     constexpr int kThreads = kWaves * kWave;
     constexpr int kSlots = kWaves / S;
-    extern __shared__ f32x4 gam[];  // [cols4]: gamma, then the dgamma combine
+    // gamma (0 past cols), then the dgamma combine: whole chunks, so that a
+    // lane's entries lie at fixed offsets
+    constexpr int kGam = NCHW * S * kWave;
+    __shared__ f32x4 gam[kGam];
     __shared__ float red[2][kWaves][2];
     const int lane = threadIdx.x & (kWave - 1);
     // a scalar, so that row addresses live in SGPRs
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int j = wave / S, q = wave % S;
     const uint32_t cols = (uint32_t)a.cols;
-    const uint32_t cols4 = (cols + 3) >> 2;
+    const uint32_t cols4 = Ragged ? (cols + 3) >> 2 : cols >> 2;
     const float fcols = (float)a.cols;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     // iteration it of block b: row (it * P + b) * slots + j -- the grid sweeps
@@ -120,7 +123,7 @@ void rms_bwd_rows_kernel(BwArgs a) {
     // gamma lives in LDS for the whole sweep: its reads are LDS operations,
     // so they neither hold registers nor make a wait for them also wait for
     // the prefetched row.
-    for (uint32_t f = threadIdx.x; f < cols4; f += kThreads) gam[f] = ld_row4<Ragged, false>(a.g, f, cols);
+    for (uint32_t f = threadIdx.x; f < (uint32_t)kGam; f += kThreads) gam[f] = ld_row4<Ragged, false>(a.g, f, cols);
     __syncthreads();
     for (uint32_t it = 0; it < a.rpw; ++it) {
         const uint64_t r = rbase + (uint64_t)it * rstride + j;
@@ -132,7 +135,7 @@ void rms_bwd_rows_kernel(BwArgs a) {
         for (int k = 0; k < NCHW; ++k) {
             const uint32_t f = col4(k);
             ss += sum4(xv[k] * xv[k]);
-            dot += sum4((xv[k] * dv[k]) * gam[f < cols4 ? f : 0]);
+            dot += sum4((xv[k] * dv[k]) * gam[f]);
         }
         ss = wave_sum_dpp(ss);
         dot = wave_sum_dpp(dot);
@@ -143,12 +146,18 @@ void rms_bwd_rows_kernel(BwArgs a) {
                 red[par][wave][1] = dot;
             }
             __syncthreads();
-            ss = red[par][j * S][0];
-            dot = red[par][j * S][1];
+            if (S >= 8) {  // one read a lane and a tree, instead of 2 S values in registers
+                const bool mine = lane < S;
+                ss = wave_sum_dpp(mine ? red[par][j * S + lane][0] : 0.0f);
+                dot = wave_sum_dpp(mine ? red[par][j * S + lane][1] : 0.0f);
+            } else {
+                ss = red[par][j * S][0];
+                dot = red[par][j * S][1];
 #pragma unroll
-            for (int t = 1; t < S; ++t) {
-                ss += red[par][j * S + t][0];
-                dot += red[par][j * S + t][1];
+                for (int t = 1; t < S; ++t) {
+                    ss += red[par][j * S + t][0];
+                    dot += red[par][j * S + t][1];
+                }
             }
         }
         const float inv = 1.0f / sqrtf(ss / fcols + a.eps);
@@ -167,7 +176,7 @@ void rms_bwd_rows_kernel(BwArgs a) {
 #pragma unroll
             for (int k = 0; k < NCHW; ++k) {
                 const uint32_t f = col4(k);
-                if (f < cols4) st_row4<Ragged>(orow, f, cols, (gam[f] * inv) * dv[k] - coeff * xv[k]);
+                st_row4<Ragged>(orow, f, cols, (gam[f] * inv) * dv[k] - coeff * xv[k]);
             }
         }
 #pragma unroll
@@ -185,7 +194,7 @@ void rms_bwd_rows_kernel(BwArgs a) {
 #pragma unroll
             for (int k = 0; k < NCHW; ++k) {
                 const uint32_t f = col4(k);
-                if (f < cols4) gam[f] = (jj == 0) ? acc[k] : gam[f] + acc[k];
+                gam[f] = (jj == 0) ? acc[k] : gam[f] + acc[k];
             }
         }
         __syncthreads();
@@ -355,8 +364,7 @@ static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols) {
 
 template <int NCHW, int S>
 static void launch_rows(const BwArgs& a, hipStream_t s) {
-    const size_t lds = a.cols / 4 * sizeof(f32x4);
-    hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwWaves, false>), dim3((uint32_t)a.partials), dim3(kBwBlock), lds,
+    hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwWaves, false>), dim3((uint32_t)a.partials), dim3(kBwBlock), 0,
                        s, a);
 }
 
@@ -375,12 +383,11 @@ constexpr uint64_t kBwLongBlocks = 256;
 template <int NCHW, int S>
 static void launch_long(const BwArgs& a, bool ragged, hipStream_t s) {
     constexpr int W = S > kBwLongWaves ? S : kBwLongWaves;
-    const size_t lds = (a.cols + 3) / 4 * sizeof(f32x4);
     const dim3 grid((uint32_t)a.partials), block(W * kWave);
     if (ragged)
-        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, true>), grid, block, lds, s, a);
+        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, true>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, false>), grid, block, lds, s, a);
+        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, false>), grid, block, 0, s, a);
 }
 
 // Library-held scratch for the allocation-free entry point: the dgamma

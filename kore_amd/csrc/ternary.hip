@@ -34,10 +34,10 @@
 // One code row (two with long K): the small-n path (dot4 on decoded windows, no
 // MFMA); then up to 256 tiles of 128 x 128 (k >= 16): the skinny path (32 or 64
 // weight rows per workgroup, K split over its waves and summed exactly in LDS);
-// at least 144 tiles of 256 x 256: the wide kernel (below); otherwise the tile
-// kernel.  Code rows that are not 16-byte aligned (K % 16 != 0 or an unaligned
-// q) take the skinny kernel and, beyond it, the tile kernel with dword-window
-// loads.
+// then tiles of 256 x 128, and at least 144 tiles of 256 x 256: the wide kernel
+// (both below).  Code rows that are not 16-byte aligned (K % 16 != 0 or an
+// unaligned q) take the skinny kernel and, beyond it, the tile kernel with
+// dword-window loads, as do 2^31 codes and more.
 // Generic path (K = 0, or an output not 4-byte aligned): one thread per
 // output, the reference loop order.
 //
@@ -3768,13 +3768,14 @@ static void launch_wide(bool aligned_a, dim3 g, hipStream_t s, const TernArgs& p
 
 using namespace kore;
 
-// Where the skinny kernel runs: up to 256 tiles of 128 x 128 (the tile kernel's:
-// one round of the CUs, its K split over workgroups and summed with atomics in
-// two more launches where they are few).  Its form follows from how many
+// Where the skinny kernel runs: up to 256 tiles of 128 x 128 (what the tile
+// kernel ran there before: one round of the CUs, its K split over workgroups
+// and summed with atomics in two more launches where they were few).  Its form follows from how many
 // workgroups each gives.  Measured in graph replays, us, m x k at n codes:
 //   6912 x 2560: n = 8 (the small-n kernel before) 12.0 -> 5.1, 100 (the tile
 //     kernel, as all that follow) 24.0 -> 10.6, 200 29.9 -> 16.3, 400 32.2 ->
-//     27.4; at 800 (378 tiles) the tile kernel's 39.7 against 41.2;
+//     27.4; past 256 tiles the 256 x 128 kernel (600 codes 28.8 against 39.1,
+//     at 400 both 28);
 //   2560 x 6912: 45 (32 rows x 64 codes, 8 waves before) 11.7 -> 8.8, 200 28.5
 //     -> 17.6, 400 39.9 -> 30.4, 800 67 -> 47;
 //   3712 x 2375 (code rows not 16-byte aligned): 1 16.6 -> 5.2, 45 17.3 -> 7.1,
@@ -3844,6 +3845,22 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
     if (k >= 16 && c_ok && skinny_wins(m, n))
         return ternary_i8_skinny(p, kp % 16 == 0 && aligned16(a_packed), s);
     const uint64_t wide_tiles = ((m + kWdM - 1) / kWdM) * ((n + kWdN - 1) / kWdN);
+    const bool al = kp % 16 == 0 && aligned16(a_packed);
+    const auto launch_w2 = [&]() -> int {
+        const uint64_t tiles = ((m + kWdM - 1) / kWdM) * ((n + kW2N - 1) / kW2N);
+        const uint64_t per = (tiles + kXcds - 1) / kXcds;
+        if (per * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+        const dim3 g((uint32_t)(per * kXcds));
+        if (p.trans) launch_w2_t<true>(al, g, s, p);
+        else launch_w2_t<false>(al, g, s, p);
+        return launch_status();
+    };
+    // Past the skinny kernel's range and below the wide one's: 256 x 128 tiles,
+    // about one a CU, their K loop two to three times the 128 x 128 kernel's
+    // rate (measured, graph replays: 6912 x 800 x 2560 39.4 -> 30.2 us, 2560 x
+    // 1600 x 6912 87.3 -> 70.4, 5376 x 1000 x 896 25.3 -> 19.1, 4096 x 1200 x
+    // 4096 57.8 -> 45.5, 2048 x 3000 x 2048 37.7 -> 28.3).
+    if (vec && wide_tiles < kWdMinTiles && nk < (1ull << 31)) return launch_w2();
     if (vec && wide_tiles >= kWdMinTiles && nk < (1ull << 31)) {
         // Many output tiles: the wide kernel (one 256 x 256 tile per CU), or
         // 256 x 192 tiles where the rounds of 256 CUs they need, at ~0.8 of a
@@ -3858,7 +3875,6 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         const uint64_t per = (tiles + kXcds - 1) / kXcds;
         if (per * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
         const dim3 g((uint32_t)(per * kXcds));
-        const bool al = kp % 16 == 0 && aligned16(a_packed);
         // Few K steps on 256 x 256 tiles: 256 x 128 tiles, two workgroups per
         // CU, so one workgroup's epilogue (an HBM write burst of a whole tile)
         // and its first K step overlap the other's matrix-core work.
@@ -3866,14 +3882,7 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         // -> 177, 6912 x 4096 x 640 44.7 -> 35.4; at 26 K steps no gain:
         // 4096 x 4096 x 4096 74.5 -> 76.5; on 192-wide tiles a loss:
         // 2560 x 4096 x 6912 92 -> 105)
-        if (!n192 && (k + kTmK - 1) / kTmK <= kW2MaxSteps) {
-            const uint64_t per2 = (((m + kWdM - 1) / kWdM) * ((n + kW2N - 1) / kW2N) + kXcds - 1) / kXcds;
-            if (per2 * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-            const dim3 g2((uint32_t)(per2 * kXcds));
-            if (p.trans) launch_w2_t<true>(al, g2, s, p);
-            else launch_w2_t<false>(al, g2, s, p);
-            return launch_status();
-        }
+        if (!n192 && (k + kTmK - 1) / kTmK <= kW2MaxSteps) return launch_w2();
         if (n192) launch_wide<6>(al, g, s, p);
         else launch_wide<8>(al, g, s, p);
         return launch_status();
@@ -3883,7 +3892,7 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         const uint64_t tiles = ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN);
         const uint64_t per = (tiles + kXcds - 1) / kXcds;
         if (per * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-        launch_mfma(kp % 16 == 0 && aligned16(a_packed), vec, dim3((uint32_t)(per * kXcds)), s, p);
+        launch_mfma(al, vec, dim3((uint32_t)(per * kXcds)), s, p);
     } else {
         const uint64_t blocks = (mn + kTmBlock - 1) / kTmBlock;
         if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;

@@ -47,3 +47,24 @@ def test_ternary_i8_forms(m, n, k, oq, oa):
     assert_bitexact(got, want, "c[m, n]")
     got = rocm.rocm_bit_linear_i8(DEV, ab, sab, qb, sqb, at(bias, 0), m, n, k).to_host(np.float32).reshape(n, m)
     assert_bitexact(got, want.T + bias, "layer")
+
+
+# 256 x 128 tiles from just past the skinny kernel's range: one and several K steps, more of them than the
+# two-workgroup form takes on larger outputs, ragged in every dimension, packed rows at each byte offset.
+@pytest.mark.parametrize("m,n,k,oa", [(4100, 1025, 16, 0), (4097, 1030, 176, 1), (2600, 1700, 2736, 0), (2570, 1665, 4112, 3),
+                                      (6912, 601, 2560, 0), (129, 33000, 336, 2)])
+def test_ternary_i8_mid_sizes(m, n, k, oa):
+    print(f"ternary i8 mid m={m} n={n} k={k} packed+{oa}", flush=True)
+    p = raw_packed(m, k, m + k)
+    q = rng(n + k).integers(-128, 128, size=(n, k), dtype=np.int64).astype(np.int8)
+    sa, sq, bias = normal((m,), 8, 1.0, 0.1), np.abs(normal((n,), 9, 0.02, 0.005)), normal((m,), 10)
+    b = p.astype(np.int32)
+    trits = np.stack([np.where(b < 243, b // 3 ** i % 3 - 1, 0) for i in range(5)], -1).reshape(m, -1)[:, :k]
+    # every partial sum is a whole number below 2^24: exact in f32 in any order
+    acc = (torch.from_numpy(trits.astype(np.float32)) @ torch.from_numpy(q.astype(np.float32)).t()).numpy()
+    want = (acc * sa[:, None]) * sq[None, :]
+    ab, qb, sab, sqb = at(p, oa), at(q, 0), at(sa, 0), at(sq, 0)
+    got = rocm.rocm_ternary_matmul_i8(DEV, ab, sab, qb, sqb, m, n, k).to_host(np.float32).reshape(m, n)
+    assert_bitexact(got, want, "c[m, n]")
+    got = rocm.rocm_bit_linear_i8(DEV, ab, sab, qb, sqb, at(bias, 0), m, n, k).to_host(np.float32).reshape(n, m)
+    assert_bitexact(got, want.T + bias, "layer")

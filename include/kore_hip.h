@@ -14,11 +14,13 @@
  *     hipError_t value when the launch itself fails.  No entry point aborts.
  *   - A call with zero elements of work returns 0 and launches nothing, as the
  *     reference CPU ops return empty tensors.
- *   - Pointers that are not 16-byte aligned, or rows whose length is not a
- *     multiple of 4 floats, take a scalar path with identical results (the
- *     ternary matmuls read unaligned packed rows and code rows through
- *     dword windows in their vector kernels; only an output that is not
- *     4-byte aligned, or K = 0, takes their one-thread-per-output path).
+ *   - Pointers need no more than their element's alignment, and rows may have
+ *     any length: the row kernels (norms, softmax, backward) and the ternary
+ *     matmuls read and write unaligned rows through their vector kernels;
+ *     element-wise ops, RoPE and the gather take a scalar path for unaligned
+ *     pointers, with identical results.  One thread per row or output remains
+ *     for norm rows of more than 16384 columns and for a ternary matmul whose
+ *     output is not 4-byte aligned or whose K is 0.
  *   - Entry points are reentrant and keep no state between calls.
  *
  * Each declaration names the reference function it replaces (paths relative

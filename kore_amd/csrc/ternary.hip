@@ -44,8 +44,8 @@
 // kore_hip_ternary_matmul_f32: the reference's f32-activation ternary_matmul,
 // a sequential fold per output (at the end): ternary_f32_mfma_kernel (fp32
 // matrix cores, 16 x 16 x 1) for prefill-sized shapes,
-// ternary_f32_mf4_kernel (4 x 4 x 1) for the layer's token-major input at
-// 41-192 tokens, ternary_f32_rows_kernel for five columns and more,
+// ternary_f32_mf4_kernel (4 x 4 x 1) for decode batches (f32_layer_form,
+// f32_use_mf4), ternary_f32_rows_kernel for the others of five columns and more,
 // ternary_f32_pipe_kernel for one to four columns, ternary_f32_seq_kernel for
 // K = 0 and matrices of fewer than 20 packed bytes.
 #include <algorithm>
@@ -3414,7 +3414,8 @@ static void launch_mfma(bool aligned_a, bool aligned_b, dim3 grid, hipStream_t s
     if (p.trans) launch_mfma_t<true>(aligned_a, aligned_b, grid, s, p);
     else launch_mfma_t<false>(aligned_a, aligned_b, grid, s, p);
 }
-// Two-workgroups-per-CU path (the wide path's shapes): a workgroup owns a
+// Two-workgroups-per-CU path (the wide path's shapes and those between it and
+// the skinny kernel's): a workgroup owns a
 // 256 (m) x 128 (n) output tile, wave w its weight rows [64 w, 64 w + 64)
 // against the tile's 128 code rows: 2 x 4 MFMA tiles of 32 x 32 (128 int32
 // accumulators per lane), 128 VGPRs + 128 AGPRs, so that each SIMD runs one
@@ -3429,7 +3430,10 @@ static void launch_mfma(bool aligned_a, bool aligned_b, dim3 grid, hipStream_t s
 // runs MFMAs meanwhile), then runs 40 MFMAs with the code operands read one
 // group ahead and the next step's code tile loaded into the other buffer by
 // direct global -> LDS loads; one barrier per step.  The byte -> five-trit
-// table is held in 16 copies (copy c for lanes c, c + 16, c + 32, c + 48).
+// table is held in 16 copies (copy c for lanes c, c + 16, c + 32, c + 48); a
+// table of 4-byte entries, the fifth trits computed, halves its LDS bytes but
+// measured slower (6912 x 4096 x 2560 92.7 -> 96-98 us), and v_perm splices
+// made no difference.
 // Code tile, K order, masking of trits past k, the alignment of packed rows
 // and the output layouts as in the wide path.
 constexpr int kW2N = 128;

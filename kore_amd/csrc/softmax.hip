@@ -24,9 +24,10 @@
 // (rounded the same way) as the hardware exp2(d * log2(e)); see exp_diff.
 //
 // Shapes: a row of up to 1024 floats is held in one wave's registers (one wave
-// per row, 4 rows per workgroup); up to 16384 in one workgroup's (256 threads;
-// 512 for the 1025-2048 backward and for 2049-4096, where some row counts take
-// a wave per row); up to 135168 (vocabularies) in the registers and LDS of a CU
+// per row, 4 rows per workgroup; two waves a row for most ragged rows of 769-1024 and for 1024);
+// up to 16384 in one workgroup's (256 threads; 512 for the 1025-2048 backward,
+// for 2049-4096, where some row counts take a wave per row, and for few rows of
+// more than 8192); up to 135168 (vocabularies) in the registers and LDS of a CU
 // (forward and cross-entropy); still longer rows, and the backward's from
 // 16385, stream through a workgroup in three passes (two).  Rows of any length
 // and alignment take the same kernels, their last cols % 4 floats one by one.
@@ -455,6 +456,24 @@ static void launch_long(const SmArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((softmax_long_kernel<K, R, kLds, Ragged>), dim3((uint32_t)a.rows), dim3(kLongThreads), lds, s, a);
 }
 
+// Ragged rows of 769-1024 columns and whole ones of 1024: a workgroup of 128
+// threads x 2 float4 per row instead of a wave x 4 of each of four rows, whose
+// workgroup ends with its slowest row (graph replays, us: causal 1023 x 1023 4.33
+// -> 4.05, 16368 x 1023 25.7 -> 24.3, softmax 32768 x 1023 49.7 -> 45.8, 64 x 1024
+// 2.50 -> 2.29).  Up to 768 columns a quarter of its threads idle (8000 x 600
+// 8.6 against 9.4), and whole rows that do not fill them are slower too (512 x
+// 964 3.3 against 3.5, 1023 x 900 3.6 against 3.9).  Backward: ragged rows
+// 256 threads x 1 float4 of each operand (512 x 1023 3.9 -> 3.5, 16368 x 1023
+// 36.8 -> 33.9), but 3000 x 1023 7.8 against 8.7; whole float4 only for few rows
+// (64 x 1024 2.17 -> 1.97; 3000 x 1024 7.3 against 7.6, 32768 61.8 against 63.6),
+// as the logits' (4096 x 1024 6.3 against 6.4).
+template <SmKind K, bool Ragged>
+static bool one_row_groups(uint64_t rows) {
+    if (K == SmKind::Bwd && Ragged) return rows <= 1536 || rows >= 5120;
+    if (K == SmKind::Bwd || (K == SmKind::CeBwd && !Ragged)) return rows <= 2048;
+    return true;
+}
+
 // The kernel for the row length.
 template <SmKind K, bool Ragged>
 static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
@@ -462,6 +481,10 @@ static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
     const dim3 grid((uint32_t)a.rows);
     if (cols4 <= 64) launch_wave<K, 1, Ragged>(a, s);
     else if (cols4 <= 128) launch_wave<K, 2, Ragged>(a, s);
+    else if (cols4 > (Ragged ? 192u : 255u) && cols4 <= 256 && one_row_groups<K, Ragged>(a.rows)) {
+        constexpr int BS = K == SmKind::Bwd && Ragged ? 256 : 128;
+        hipLaunchKernelGGL((softmax_reg_kernel<K, 256 / BS, true, Ragged, BS>), grid, dim3(BS), 0, s, a);
+    }
     else if (cols4 <= 256) launch_wave<K, 4, Ragged>(a, s);
     else if (cols4 <= 512) {
         // 1025-2048 columns: one workgroup per row streams faster than one
@@ -483,6 +506,11 @@ static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
     }
     else if (cols4 <= 2048)
         hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    else if (cols4 <= 4096 && K != SmKind::Bwd && a.rows <= 512)
+        // 8193-16384 columns: 512 threads while the rows are few (512 x 16384
+        // 12.0 -> 10.9 us, 300 x 9000 7.3 -> 6.7, 64 x 12345 6.6 -> 5.5; 1024 x
+        // 12288 logits 18.2 against 20.2, and 300 x 9000 backward 8.2 against 8.6).
+        hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged, 512>), grid, dim3(512), 0, s, a);
     else if (cols4 <= 4096)
         hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
     else if (K != SmKind::Bwd && a.cols <= kLongCols) {

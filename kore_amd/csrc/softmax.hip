@@ -506,13 +506,16 @@ static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
     }
     else if (cols4 <= 2048)
         hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
-    else if (cols4 <= 4096 && K != SmKind::Bwd && a.rows <= 512)
+    else if (cols4 <= 4096) {
         // 8193-16384 columns: 512 threads while the rows are few (512 x 16384
         // 12.0 -> 10.9 us, 300 x 9000 7.3 -> 6.7, 64 x 12345 6.6 -> 5.5; 1024 x
         // 12288 logits 18.2 against 20.2, and 300 x 9000 backward 8.2 against 8.6).
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged, 512>), grid, dim3(512), 0, s, a);
-    else if (cols4 <= 4096)
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+        constexpr int kFew = K == SmKind::Bwd ? kSmBlock : 512;
+        if (a.rows <= 512)
+            hipLaunchKernelGGL((softmax_reg_kernel<K, 4096 / kFew, true, Ragged, kFew>), grid, dim3(kFew), 0, s, a);
+        else
+            hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    }
     else if (K != SmKind::Bwd && a.cols <= kLongCols) {
         if constexpr (K != SmKind::Bwd) {
             if (cols4 <= 8 * kLongThreads) launch_long<K, 8, Ragged>(a, s);

@@ -12,6 +12,12 @@ namespace kore {
 // 2^31 blocks and every byte offset far from 64-bit overflow.
 constexpr uint64_t kMaxElements = 1ull << 46;
 
+// Rows one launch takes.  A launch holds fewer than 2^32 threads (a larger grid
+// wraps without an error, and rows are left out), at up to 1024 threads a row;
+// calls with more rows are enqueued in bands of this many, each of them enough
+// to fill the chip hundreds of times over.
+constexpr uint64_t kLaunchRows = 1ull << 21;
+
 // Status of the launch just enqueued: 0, or the hipError_t it raised.
 // hipGetLastError also clears a sticky launch error so it is reported once.
 inline int launch_status() {

@@ -48,6 +48,7 @@ struct SmArgs {
     uint64_t rows;
     uint64_t cols;
     uint64_t seq_offset;
+    uint64_t batch;  // rows of the whole call (cross-entropy)
 };
 
 constexpr int kSmBlock = 256;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
     if (Block) s = block_combine<false, kWavesB>(s, red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
     if (K == SmKind::CeBwd) {
-        const float inv_batch = 1.0f / (float)a.rows;
+        const float inv_batch = 1.0f / (float)a.batch;
         const float scale = inv * inv_batch;
         const uint64_t t = target_index(a.b[row], a.cols);
 #pragma unroll
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(kLongThreads) void softmax_long_kernel(SmArgs a) {
     o.s *= o.m == ninf ? 1.0f : exp_diff(o.m - m);
     const float s = block_combine<false, kWavesB>(wave_sum(o.s), red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
-    const float inv_batch = 1.0f / (float)a.rows;
+    const float inv_batch = 1.0f / (float)a.batch;
     const float scale = (K == SmKind::CeBwd) ? inv * inv_batch : inv;
     auto value = [&](uint32_t f, f32x4 x) {  // outputs of float4 f
 #pragma unroll
@@ -421,7 +422,7 @@ __global__ __launch_bounds__(kSmBlock) void softmax_loop_kernel(SmArgs a) {
     }
     s = block_combine<false>(wave_sum(s), red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
-    const float inv_batch = 1.0f / (float)a.rows;
+    const float inv_batch = 1.0f / (float)a.batch;
     const float scale = (K == SmKind::CeBwd) ? inv * inv_batch : inv;
     const uint64_t t = (K == SmKind::CeBwd) ? target_index(a.b[row], a.cols) : ~0ull;
     for (uint64_t i = threadIdx.x; i < n; i += kSmBlock) {
@@ -537,12 +538,23 @@ static int softmax_launch(const SmArgs& a, hipStream_t s) {
     if (K == SmKind::Causal && a.seq_offset + a.rows < a.seq_offset) return KORE_HIP_ERR_OVERFLOW;
     const bool aligned = (a.cols % 4 == 0) && aligned16(a.a) && aligned16(a.out) &&
                          (K != SmKind::Bwd || aligned16(a.b));
-    if (aligned)
-        softmax_dispatch<K, false>(a, s);
-    else if (a.cols >= 4)
-        softmax_dispatch<K, true>(a, s);
-    else  // ragged rows are read four floats at a time
-        hipLaunchKernelGGL((softmax_loop_kernel<K, false>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
+    SmArgs band = a;
+    band.batch = a.rows;
+    for (uint64_t left = a.rows; left > 0;) {
+        band.rows = left < kLaunchRows ? left : kLaunchRows;
+        if (aligned)
+            softmax_dispatch<K, false>(band, s);
+        else if (a.cols >= 4)
+            softmax_dispatch<K, true>(band, s);
+        else  // ragged rows are read four floats at a time
+            hipLaunchKernelGGL((softmax_loop_kernel<K, false>), dim3((uint32_t)band.rows), dim3(kSmBlock), 0, s, band);
+        left -= band.rows;
+        band.a += band.rows * a.cols;
+        band.out += band.rows * a.cols;
+        if (K == SmKind::Bwd) band.b += band.rows * a.cols;
+        if (K == SmKind::CeBwd) band.b += band.rows;
+        band.seq_offset += band.rows;
+    }
     return launch_status();
 }
 

@@ -1,0 +1,76 @@
+"""Row counts at which a workgroup or a wave a row comes to 2^32 threads, more than one launch holds: the calls go in
+bands of rows.  Rows around the buffer's ends, the bands' and the point where one launch would wrap, against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from inputs import assert_close, normal
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from kore_amd import rocm  # noqa: E402
+from kore_amd.rocm import HipBuffer  # noqa: E402
+
+DEV = 0
+U32 = 2.0 ** -24
+
+
+def big(rows, cols):
+    """An unset device matrix, or a skip where the card has no room for it."""
+    need = rows * cols * 4
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < need + (4 << 30):
+        pytest.skip(f"needs {need >> 30} GiB of device memory")
+    return torch.empty((rows, cols), dtype=torch.float32, device="cuda:0")
+
+
+def sample(rows):
+    return sorted({r for r in (0, 1, 777, (1 << 21) - 1, 1 << 21, rows // 2, (1 << 23) + 1, rows - 5, rows - 1) if r < rows})
+
+
+def fill(t, at, seed):
+    x = normal((len(at), t.shape[1]), seed) * 3
+    put(t, at, x)
+    return x
+
+
+def put(t, at, x):
+    for r, row in zip(at, x):
+        t[r].copy_(torch.from_numpy(row))
+
+
+def rows_of(t, at):
+    return np.stack([t[r].cpu().numpy() for r in at])
+
+
+# Just past 2^32 threads at 512 and (1024 columns) at 128 threads a row.
+@pytest.mark.parametrize("rows,cols", [((1 << 23) + 3, 2052), ((1 << 25) + 3, 1024)])
+def test_softmax_many_rows(rows, cols):
+    print(f"softmax rows={rows} cols={cols}", flush=True)
+    t, at = big(rows, cols), sample(rows)
+    b = HipBuffer.from_tensor(t.view(-1))
+    x = fill(t, at, 1)
+    rocm.rocm_softmax_f32(DEV, b, rows, cols, b)
+    assert_close(rows_of(t, at), oracle.softmax(x), rtol=1e-5 + cols * U32, what="softmax")
+    x = fill(t, at, 2)
+    rocm.rocm_softmax_causal_f32(DEV, b, rows, cols, 5, b)
+    want = np.concatenate([oracle.softmax_causal(x[i:i + 1], 5 + r) for i, r in enumerate(at)])
+    assert_close(rows_of(t, at), want, rtol=1e-5 + cols * U32, what="causal")
+    x = fill(t, at, 3)
+    targets = torch.full((rows,), 7.0, device="cuda:0")
+    rocm.rocm_cross_entropy_backward_f32(DEV, b, HipBuffer.from_tensor(targets), rows, cols, b)
+    want = oracle.softmax(x).astype(np.float64)
+    want[:, 7] -= 1.0
+    assert_close(rows_of(t, at), want / rows, rtol=1e-5 + cols * U32, atol=1e-6 / rows, what="cross entropy")
+
+
+@pytest.mark.parametrize("rows,cols", [((1 << 23) + 3, 1025), ((1 << 23) + 3, 2052)])
+def test_softmax_backward_many_rows(rows, cols):
+    print(f"softmax backward rows={rows} cols={cols}", flush=True)
+    t, at = big(rows, cols), sample(rows)
+    b = HipBuffer.from_tensor(t.view(-1))
+    y = oracle.softmax(fill(t, at, 1))
+    put(t, at, y)
+    rocm.rocm_softmax_backward_f32(DEV, b, b, rows, cols, b)
+    assert_close(rows_of(t, at), oracle.softmax_backward(y, y), rtol=1e-5 + cols * U32, atol=1e-6, what="backward")

@@ -727,9 +727,7 @@ __global__ __launch_bounds__(64) void row_norm_scalar_kernel(NormArgs args) {
 template <NormOut Out, int SL4, int WPB, int W, bool Half>
 static int launch_form(NormArgs a, RowForm form, hipStream_t s) {
     const size_t lds = (size_t)WPB * wave_lds_f4(SL4, Half) * sizeof(f32x4);
-    const uint64_t blocks = (a.rows * W + WPB - 1) / WPB;
-    if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-    const dim3 grid((uint32_t)blocks), block(kWave * WPB);
+    const dim3 grid((uint32_t)((a.rows * W + WPB - 1) / WPB)), block(kWave * WPB);  // at most 2^29 threads
     if (form == RowForm::Ragged)
         hipLaunchKernelGGL((row_norm_kernel<Out, SL4, RowForm::Ragged, WPB, W, Half>), grid, block, lds, s, a);
     else if (a.cols == (uint32_t)(4 * kWave * SL4 * W))
@@ -823,7 +821,19 @@ static int norm_launch(NormArgs a, hipStream_t s) {
         hipLaunchKernelGGL(row_norm_scalar_kernel<Out>, dim3((uint32_t)blocks), dim3(64), 0, s, a);
         return launch_status();
     }
-    return launch_sl4<Out>(a, nch, whole ? RowForm::Part : RowForm::Ragged, s);
+    if (whole && a.rows > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+    for (uint64_t left = a.rows; left > 0;) {
+        a.rows = left < kLaunchRows ? left : kLaunchRows;
+        const int st = launch_sl4<Out>(a, nch, whole ? RowForm::Part : RowForm::Ragged, s);
+        if (st != KORE_HIP_OK) return st;
+        left -= a.rows;
+        const uint64_t n = a.rows * a.cols;
+        a.x += n;
+        if (Out == NormOut::I8) a.q += n, a.scale += a.rows;
+        else a.y += n;
+        if (Out == NormOut::SiluGate) a.z += n;
+    }
+    return KORE_HIP_OK;
 }
 
 }  // namespace kore

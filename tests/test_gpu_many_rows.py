@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from inputs import assert_close, normal
+from inputs import assert_bitexact, assert_close, normal
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +74,22 @@ def test_softmax_backward_many_rows(rows, cols):
     put(t, at, y)
     rocm.rocm_softmax_backward_f32(DEV, b, b, rows, cols, b)
     assert_close(rows_of(t, at), oracle.softmax_backward(y, y), rtol=1e-5 + cols * U32, atol=1e-6, what="backward")
+
+# Just past 2^32 threads at a wave a row; odd bands start a ragged row anywhere.
+@pytest.mark.parametrize("cols", [1, 3])
+def test_norm_family_many_rows(cols):
+    rows = (1 << 26) + 3
+    print(f"norm family rows={rows} cols={cols}", flush=True)
+    t, at = big(rows, cols), sample(rows)
+    w = normal((cols,), 4, 1.0, 0.02)
+    xb, wb = HipBuffer.from_tensor(t.view(-1)), HipBuffer.from_host(DEV, w)
+    x = fill(t, at, 1)
+    q, scale = rocm.rocm_rms_norm_quant_i8(DEV, xb, wb, rows, cols, 1e-6)
+    want_q, want_s = oracle.rms_norm_quant_i8(x, w, 1e-6)
+    assert_bitexact(rows_of(q.tensor(torch.int8)[:rows * cols].view(rows, cols), at), want_q, "codes")
+    assert_bitexact(rows_of(scale.tensor(torch.float32)[:rows].view(rows, 1), at)[:, 0], want_s, "scales")
+    y = rocm.rocm_fused_rms_norm_silu_gate_f32(DEV, xb, wb, xb, rows, cols, 1e-6)
+    assert_close(rows_of(y.tensor(torch.float32)[:rows * cols].view(rows, cols), at),
+                 oracle.rms_norm_silu_gate(x, w, x, 1e-6), what="silu gate")
+    rocm.rocm_rms_norm_f32(DEV, xb, wb, rows, cols, 1e-6, out=xb)
+    assert_bitexact(rows_of(t, at), oracle.rms_norm(x, w, 1e-6), "rms_norm")

@@ -65,6 +65,8 @@ constexpr int kEwBlock = 128;
 constexpr int kEwUnroll = 1;  // float4 per thread
 
 constexpr uint64_t kEwTile = (uint64_t)kEwBlock * kEwUnroll;  // float4 per block
+// Floats a launch takes: 2^31 threads (see kLaunchRows).
+constexpr uint64_t kEwLaunch = 1ull << 33;
 
 // One block's tile.  Full = true drops every bounds check (all blocks but the
 // last), so the loads issue back to back as one clause.
@@ -190,6 +192,10 @@ static int launch_unary(const float* x, float* out, uint64_t n, hipStream_t s) {
     if (n == 0) return KORE_HIP_OK;
     if (!x || !out) return KORE_HIP_ERR_NULL_PTR;
     if (n > kMaxElements) return KORE_HIP_ERR_OVERFLOW;
+    for (; n > kEwLaunch; x += kEwLaunch, out += kEwLaunch, n -= kEwLaunch) {
+        const int st = launch_unary<Op>(x, out, kEwLaunch, s);
+        if (st != KORE_HIP_OK) return st;
+    }
     if (aligned16(x) && aligned16(out)) {
         uint64_t n4 = n / 4;
         uint32_t tail = (uint32_t)(n % 4);
@@ -211,6 +217,10 @@ static int launch_binary(const float* a, const float* b, float* out, uint64_t n,
     if (n == 0) return KORE_HIP_OK;
     if (!a || !b || !out) return KORE_HIP_ERR_NULL_PTR;
     if (n > kMaxElements) return KORE_HIP_ERR_OVERFLOW;
+    for (; n > kEwLaunch; a += kEwLaunch, b += kEwLaunch, out += kEwLaunch, n -= kEwLaunch) {
+        const int st = launch_binary<Op>(a, b, out, kEwLaunch, s);
+        if (st != KORE_HIP_OK) return st;
+    }
     if (aligned16(a) && aligned16(b) && aligned16(out)) {
         uint64_t n4 = n / 4;
         uint32_t tail = (uint32_t)(n % 4);

@@ -108,6 +108,10 @@ static int embedding_launch(const float* table, const Id* ids, float* out, uint6
     if (!mul_ok(n_ids, dim, &out_elems) || !mul_ok(vocab, dim, &table_elems) || out_elems > kMaxElements ||
         table_elems > kMaxElements || n_ids > 0x7fffffffull)
         return KORE_HIP_ERR_OVERFLOW;
+    for (; n_ids > kLaunchRows; ids += kLaunchRows, out += kLaunchRows * dim, n_ids -= kLaunchRows) {
+        const int st = embedding_launch(table, ids, out, kLaunchRows, vocab, dim, stream);
+        if (st != KORE_HIP_OK) return st;
+    }
     hipStream_t s = (hipStream_t)stream;
     dim3 grid((uint32_t)n_ids), block(kEmbBlock);
     if (dim % 4 == 0 && aligned16(out) && (vocab == 0 || aligned16(table))) {

@@ -342,12 +342,14 @@ static uint32_t bwd_split(uint64_t cols) {
 // each, two per SIMD, with the next row's loads in flight) -- measured against
 // 256, 384, 768 and 1024 at 16384 x 2048: fewer partial rows to reduce, and
 // enough waves to keep HBM busy (70.0 vs 72.7 us at 1024); at most 16
-// iterations so that large batches keep few partial rows.
+// iterations so that large batches keep few partial rows, and past 2^28 rows
+// as many as keep it at 2^30 threads (a launch holds fewer than 2^32).
 static uint32_t bwd_iters(uint64_t rows, uint32_t split) {
     const uint64_t per_iter = kBwWaves / split;
     uint64_t it = (rows + 512 * per_iter - 1) / (512 * per_iter);
     if (it < 1) it = 1;
-    if (it > 16) it = 16;
+    const uint64_t most = rows >> 22 > 16 * per_iter ? (rows >> 22) / per_iter + 1 : 16;
+    if (it > most) it = most;
     return (uint32_t)it;
 }
 

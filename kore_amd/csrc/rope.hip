@@ -24,6 +24,8 @@
 //
 // The rotation is the reference's: d[i] = x0*c - x1*s, d[j] = x0*s + x1*c,
 // with every product rounded on its own (-ffp-contract=off).
+#include <algorithm>
+
 #include "common.hpp"
 #include "kore_hip_internal.hpp"
 
@@ -268,6 +270,24 @@ static int rope_launch(float* q, uint32_t q_heads, float* k, uint32_t k_heads, c
         const char* k0 = (const char*)k;
         const char* k1 = k0 + tokens * (uint64_t)k_heads * head_dim * 4;
         if (q0 < k1 && k0 < q1) return KORE_HIP_ERR_ALIAS;
+    }
+    // A launch holds fewer than 2^32 threads (see kLaunchRows); a token takes at
+    // most one per four floats and a workgroup of each tensor: several
+    // sequences a launch, or parts of one.
+    const uint64_t most = std::max<uint64_t>(1, 0x7fffffffull / (heads_all * head_dim / 4 + kRopeMaxBlock));
+    if (tokens > most) {
+        const uint64_t nb = seq_len <= most ? most / seq_len : 1, ns = seq_len <= most ? seq_len : most;
+        for (uint64_t b = 0; b < batch; b += nb) {
+            for (uint64_t p = 0; p < seq_len; p += ns) {
+                const uint64_t at = b * seq_len + p;  // first token
+                const int st = rope_launch(q_heads ? q + at * q_heads * head_dim : nullptr, q_heads,
+                                           k_heads ? k + at * k_heads * head_dim : nullptr, k_heads, inv_freq,
+                                           batch - b < nb ? batch - b : nb, seq_len - p < ns ? seq_len - p : ns,
+                                           head_dim, start_pos + p, interleaved, s);
+                if (st != KORE_HIP_OK) return st;
+            }
+        }
+        return KORE_HIP_OK;
     }
     RopeTensor t0{q_heads ? q : k, q_heads ? q_heads : k_heads};
     RopeTensor t1{q_heads ? k : nullptr, q_heads ? k_heads : 0u};

@@ -93,3 +93,59 @@ def test_norm_family_many_rows(cols):
                  oracle.rms_norm_silu_gate(x, w, x, 1e-6), what="silu gate")
     rocm.rocm_rms_norm_f32(DEV, xb, wb, rows, cols, 1e-6, out=xb)
     assert_bitexact(rows_of(t, at), oracle.rms_norm(x, w, 1e-6), "rms_norm")
+
+
+def test_elementwise_many_threads():
+    n = (1 << 34) + 5
+    print(f"silu and mul in place n={n}", flush=True)
+    t = big(n, 1).view(-1)
+    b = HipBuffer.from_tensor(t)
+    spots = [0, 4096, (1 << 33) - 8, (1 << 33) + 100, n // 2 + 64, n - 8]
+    x = normal((len(spots), 8), 5)
+    put(t, [slice(i, i + 8) for i in spots], x)
+    rocm.rocm_silu_f32(DEV, b, n, b)
+    y = rows_of(t, [slice(i, i + 8) for i in spots])
+    assert_close(y, oracle.silu(x), what="silu")
+    rocm.rocm_mul_f32(DEV, b, b, n, b)
+    assert_bitexact(rows_of(t, [slice(i, i + 8) for i in spots]), y * y, "mul")
+
+
+def test_embedding_many_ids():
+    n, dim, vocab = (1 << 26) + 3, 4, 1000
+    print(f"embedding n={n}", flush=True)
+    table = normal((vocab, dim), 6)
+    ids = (torch.arange(n, device="cuda:0", dtype=torch.int32) * 7) % vocab
+    out = rocm.rocm_embedding_f32(DEV, HipBuffer.from_host(DEV, table), HipBuffer.from_tensor(ids), n, vocab, dim)
+    got = out.tensor(torch.float32).view(n, dim)
+    at = sample(n)
+    assert_bitexact(rows_of(got, at), oracle.embedding(table, np.array([int(ids[r]) for r in at], np.int32)), "rows")
+
+
+# One long sequence and many short ones, at 128 threads a token of 32 floats.
+@pytest.mark.parametrize("batch,seq", [(1, (1 << 25) + 3), ((1 << 22) + 1, 9)])
+def test_rope_many_tokens(batch, seq):
+    print(f"rope batch={batch} seq={seq}", flush=True)
+    t = big(batch * seq, 32)
+    at = sample(batch * seq)
+    x = fill(t, at, 7)
+    inv = rocm.rocm_rope_inv_freq_f32(DEV, 32, 10000.0)
+    rocm.rocm_rope_f32(DEV, HipBuffer.from_tensor(t.view(-1)), inv, batch, seq, 1, 32, 3, False)
+    want = np.concatenate([oracle.rope(x[i].reshape(1, 1, 1, 32), 3 + r % seq, 10000.0).reshape(1, 32)
+                           for i, r in enumerate(at)])
+    assert_close(rows_of(t, at), want, what="rope")
+
+
+def test_rms_norm_backward_many_rows():
+    rows, cols = (1 << 30) + 3, 4
+    print(f"rms_norm_backward rows={rows}", flush=True)
+    x, dy, dx = (big(rows, cols) for _ in range(3))
+    x.fill_(1.0)
+    dy.zero_()
+    at, g = sample(rows), normal((cols,), 8, 1.0, 0.02)
+    xs, ds = fill(x, at, 9), fill(dy, at, 10)
+    dxb, dgb = rocm.rocm_rms_norm_backward_f32(
+        DEV, HipBuffer.from_tensor(dy.view(-1)), HipBuffer.from_tensor(x.view(-1)), HipBuffer.from_host(DEV, g), rows,
+        cols, 1e-5, grad_input=HipBuffer.from_tensor(dx.view(-1)))
+    want_dx, want_dg = oracle.rms_norm_backward(ds, xs, g, 1e-5)  # the other rows' dy is 0
+    assert_close(rows_of(dx, at), want_dx, rtol=1e-4, atol=1e-5, what="dx")
+    assert_close(dgb.to_host(np.float32)[:cols], want_dg, rtol=1e-5, atol=1e-5, what="dgamma")

@@ -68,26 +68,6 @@ __device__ __forceinline__ f32x4 ld_row4(const float* row, uint32_t f, uint32_t 
     return v;
 }
 
-// The same for a load that is used at once, n >= 4: float4 that pass the end
-// read the row's last four floats and move the ones they want down, so that a
-// wave's loads go out together without a branch each.  It waits for the load
-// where the row ends: a load that is meant to stay in flight takes ld_row4.
-template <bool Ragged>
-__device__ __forceinline__ f32x4 ld_row4_now(const float* row, uint32_t f, uint32_t n) {
-    if (!Ragged) return ld_row4<false>(row, f, n);
-    const uint32_t at = 4 * f + 4 <= n ? 4 * f : n - 4;
-    f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(row + at));
-    const uint32_t d = 4 * f - at;  // floats before the wanted ones: 1-3 in the last float4, more past it
-    if (__builtin_expect(__ballot(d != 0) != 0, 0)) {
-        const f32x4 o = v;
-        v.x = d == 0 ? o.x : (d == 1 ? o.y : (d == 2 ? o.z : (d == 3 ? o.w : 0.f)));
-        v.y = d == 0 ? o.y : (d == 1 ? o.z : (d == 2 ? o.w : 0.f));
-        v.z = d == 0 ? o.z : (d == 1 ? o.w : 0.f);
-        v.w = d == 0 ? o.w : 0.f;
-    }
-    return v;
-}
-
 template <bool Ragged, bool Stream = true>
 __device__ __forceinline__ void st_row4(float* row, uint32_t f, uint32_t n, f32x4 v) {
     if (!Ragged) {

@@ -105,10 +105,16 @@ __device__ __forceinline__ float block_combine(float v, float* red) {
 // Row in registers.  Wave mode (Block = false): one wave per row, element f4
 // index = c*64 + lane, 4 rows per 256-thread workgroup.  Block mode: one
 // workgroup of BS threads per row, index = c*BS + tid.
-// Ragged: rows of any length and alignment (ld_row4_now).  Causal rows read only
-// the float4 that hold a column they keep.
+// Ragged: rows of any length (from 4 floats) and alignment.  Their whole float4
+// are read and written at dword alignment; float4 past the last one to read
+// repeat it, so that the loads go out without a branch each; the row's last
+// cols % 4 floats are one float each of its first threads (a branch a float4 for
+// them cost more than few rows do: backward 64 x 513 3.17 us, 2.43 here, 2.26
+// in the loop kernel's one float a thread).  Causal rows read only the float4
+// that hold a column they keep.  Two operands of 16 float4 keep three waves a
+// SIMD.
 template <SmKind K, int NCH, bool Block, bool Ragged, int BS = kSmBlock>
-__global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
+__global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void softmax_reg_kernel(SmArgs a) {
     constexpr int kWavesB = BS / kWave;
     __shared__ float red[kWavesB];
     const int lane = threadIdx.x & (kWave - 1);
@@ -119,18 +125,39 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
     const int me = Block ? (int)threadIdx.x : lane;
     const uint32_t cols = (uint32_t)a.cols;               // <= 16384 here
     const uint32_t lim = (uint32_t)row_limit<K>(a, row);  // <= cols
-    // columns to read: causal rows leave out the float4 past their last one
-    const uint32_t need = K == SmKind::Causal && lim + 3u < cols ? (lim + 3u) & ~3u : cols;
+    const uint32_t whole4 = cols >> 2;
+    // float4 to read: causal rows leave out those past their last column
+    const uint32_t need4 = K == SmKind::Causal && (lim + 3u) >> 2 < whole4 ? (lim + 3u) >> 2 : whole4;
+    const uint32_t lim4 = lim < 4 * whole4 ? lim : 4 * whole4;  // columns that take part and lie in whole float4
     const float* ar = a.a + row * cols;
     const float* br = a.b + row * cols;
     float* orow = a.out + row * cols;
+    auto load = [&](const float* r, uint32_t f) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        if (Ragged)
+            return (f32x4)__builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(r) +
+                                                     (f < need4 ? f : need4 - 1u));
+        return f < need4 ? ld_stream(reinterpret_cast<const f32x4*>(r) + f) : zero;
+    };
+    auto store = [&](uint32_t f, f32x4 o) {
+        if (f >= whole4) return;
+        if (Ragged) __builtin_nontemporal_store((f32x4_a4)o, reinterpret_cast<f32x4_a4*>(orow) + f);
+        else st_stream(reinterpret_cast<f32x4*>(orow) + f, o);
+    };
 
     f32x4 v[NCH], g[NCH];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const uint32_t f = (uint32_t)(c * step + me);
-        v[c] = ld_row4_now<Ragged>(ar, f, need);
-        if (K == SmKind::Bwd) g[c] = ld_row4_now<Ragged>(br, f, cols);
+        v[c] = load(ar, f);
+        if (K == SmKind::Bwd) g[c] = load(br, f);
+    }
+    // Ragged: this thread's one of the last floats, if any.
+    const uint32_t tc = 4 * whole4 + (uint32_t)me;
+    float tv = 0.0f, tg = 0.0f;
+    if (Ragged && tc < lim) {
+        tv = ar[tc];
+        if (K == SmKind::Bwd) tg = br[tc];
     }
 
     if (K == SmKind::Bwd) {
@@ -139,14 +166,17 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const f32x4 p = v[c] * g[c];
-            dot += (p.x + p.y) + (p.z + p.w);
+            const float d = (p.x + p.y) + (p.z + p.w);
+            dot += !Ragged || (uint32_t)(c * step + me) < whole4 ? d : 0.0f;
         }
+        if (Ragged) dot += tv * tg;
         dot = wave_sum(dot);
         if (Block) dot = block_combine<false, kWavesB>(dot, red);
+        if (Ragged && tc < cols) orow[tc] = tv * (tg - dot);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const uint32_t f = (uint32_t)(c * step + me);
-            st_row4<Ragged>(orow, f, cols, v[c] * (g[c] - dot));
+            store(f, v[c] * (g[c] - dot));
         }
         return;
     }
@@ -158,10 +188,11 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
         const uint32_t f = (uint32_t)(c * step + me);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const bool in = 4 * f + k < lim;
+            const bool in = 4 * f + k < lim4;
             m = fmaxf(m, in ? f4_get(v[c], k) : ninf);
         }
     }
+    if (Ragged) m = fmaxf(m, tc < lim ? tv : ninf);
     m = wave_max(m);
     if (Block) m = block_combine<true, kWavesB>(m, red);
     float s = 0.0f;
@@ -170,11 +201,15 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
         const uint32_t f = (uint32_t)(c * step + me);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const bool in = 4 * f + k < lim;
+            const bool in = 4 * f + k < lim4;
             const float e = in ? exp_diff(f4_get(v[c], k) - m) : 0.0f;
             f4_set(v[c], k, e);
             s += e;
         }
+    }
+    if (Ragged) {
+        tv = tc < lim ? exp_diff(tv - m) : 0.0f;
+        s += tv;
     }
     s = wave_sum(s);
     if (Block) s = block_combine<false, kWavesB>(s, red);
@@ -183,6 +218,7 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
         const float inv_batch = 1.0f / (float)a.batch;
         const float scale = inv * inv_batch;
         const uint64_t t = target_index(a.b[row], a.cols);
+        if (Ragged && tc < cols) orow[tc] = tc == t ? tv * scale - inv_batch : tv * scale;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const uint32_t f = (uint32_t)(c * step + me);
@@ -190,14 +226,15 @@ __global__ __launch_bounds__(BS) void softmax_reg_kernel(SmArgs a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
                 if ((uint64_t)(4 * f + k) == t) f4_set(o, k, f4_get(o, k) - inv_batch);
-            st_row4<Ragged>(orow, f, cols, o);
+            store(f, o);
         }
         return;
     }
+    if (Ragged && tc < cols) orow[tc] = tv * inv;
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         const uint32_t f = (uint32_t)(c * step + me);
-        st_row4<Ragged>(orow, f, cols, v[c] * inv);
+        store(f, v[c] * inv);
     }
 }
 

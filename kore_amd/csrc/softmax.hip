@@ -217,7 +217,11 @@ __global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void sof
     if (K == SmKind::CeBwd) {
         const float inv_batch = 1.0f / (float)a.batch;
         const float scale = inv * inv_batch;
-        const uint64_t t = target_index(a.b[row], a.cols);
+        // Through a vector load (the index is not a scalar): a scalar one leaves
+        // the waves of a full chip in step, all storing at once (8192 x 900 10.4
+        // us against 8.8, x 1024 10.7 against 9.0).
+        const uint64_t vrow = Block ? row : (uint64_t)blockIdx.x * kSmWaves + threadIdx.x / kWave;
+        const uint64_t t = target_index(a.b[vrow], a.cols);
         if (Ragged && tc < cols) orow[tc] = tc == t ? tv * scale - inv_batch : tv * scale;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {

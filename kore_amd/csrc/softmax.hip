@@ -24,13 +24,14 @@
 // (rounded the same way) as the hardware exp2(d * log2(e)); see exp_diff.
 //
 // Shapes: a row of up to 1024 floats is held in one wave's registers (one wave
-// per row, 4 rows per workgroup; two waves a row for most ragged rows of 769-1024 and for 1024);
-// up to 16384 in one workgroup's (256 threads; 512 for the 1025-2048 backward,
-// for 2049-4096, where some row counts take a wave per row, and for few rows of
-// more than 8192); up to 135168 (vocabularies) in the registers and LDS of a CU
-// (forward and cross-entropy); still longer rows, and the backward's from
-// 16385, stream through a workgroup in three passes (two).  Rows of any length
-// and alignment take the same kernels, their last cols % 4 floats one by one.
+// per row, 4 rows per workgroup; two waves a row where two_waves_a_row says so);
+// up to 16384 in one workgroup's (256 threads; 512 for the 1025-2048 backward of
+// whole rows and for few rows of more than 8192; 2049-4096 see mid_form); up to
+// 135168 (vocabularies) in the registers and LDS of a CU (forward and
+// cross-entropy); still longer rows, and the backward's from 16385, stream
+// through a workgroup in three passes (two), as do a backward's few short
+// ragged rows.  Rows of any length and alignment take the same kernels, their
+// last cols % 4 floats one by one.
 // Every kernel reads a row fully before writing it, so out may alias an input.
 #include <type_traits>
 
@@ -48,7 +49,7 @@ struct SmArgs {
     uint64_t rows;
     uint64_t cols;
     uint64_t seq_offset;
-    uint64_t batch;  // rows of the whole call (cross-entropy)
+    float inv_batch;  // 1 / rows of the whole call (cross-entropy)
 };
 
 constexpr int kSmBlock = 256;
@@ -114,11 +115,14 @@ __device__ __forceinline__ float block_combine(float v, float* red) {
 // that hold a column they keep.  Two operands of 16 float4 keep three waves a
 // SIMD.
 template <SmKind K, int NCH, bool Block, bool Ragged, int BS = kSmBlock>
-__global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void softmax_reg_kernel(SmArgs a) {
+__global__ __launch_bounds__(BS, NCH < 16 ? 1 : K == SmKind::Bwd ? 3 : 4) void softmax_reg_kernel(SmArgs a) {
     constexpr int kWavesB = BS / kWave;
     __shared__ float red[kWavesB];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    // A scalar, so that row addresses live in SGPRs; but not for the backward's
+    // 2049-4096 columns, whose waves it puts in step (2048 x 2500 8.7 -> 9.7 us).
+    const bool lanes = K == SmKind::Bwd && NCH == 16;
+    const int wave = lanes ? (int)(threadIdx.x / kWave) : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const uint64_t row = Block ? (uint64_t)blockIdx.x : (uint64_t)blockIdx.x * kSmWaves + wave;
     if (!Block && row >= a.rows) return;  // uniform per wave; no block barrier in wave mode
     const int step = Block ? BS : kWave;
@@ -128,7 +132,7 @@ __global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void sof
     const uint32_t whole4 = cols >> 2;
     // float4 to read: causal rows leave out those past their last column
     const uint32_t need4 = K == SmKind::Causal && (lim + 3u) >> 2 < whole4 ? (lim + 3u) >> 2 : whole4;
-    const uint32_t lim4 = lim < 4 * whole4 ? lim : 4 * whole4;  // columns that take part and lie in whole float4
+    const uint32_t lim4 = Ragged && lim > 4 * whole4 ? 4 * whole4 : lim;  // columns that take part and lie in whole float4
     const float* ar = a.a + row * cols;
     const float* br = a.b + row * cols;
     float* orow = a.out + row * cols;
@@ -215,13 +219,13 @@ __global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void sof
     if (Block) s = block_combine<false, kWavesB>(s, red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
     if (K == SmKind::CeBwd) {
-        const float inv_batch = 1.0f / (float)a.batch;
+        const float inv_batch = a.inv_batch;
         const float scale = inv * inv_batch;
         // Through a vector load (the index is not a scalar): a scalar one leaves
         // the waves of a full chip in step, all storing at once (8192 x 900 10.4
         // us against 8.8, x 1024 10.7 against 9.0).
         const uint64_t vrow = Block ? row : (uint64_t)blockIdx.x * kSmWaves + threadIdx.x / kWave;
-        const uint64_t t = target_index(a.b[vrow], a.cols);
+        const uint32_t t = (uint32_t)target_index(a.b[vrow], a.cols);  // none: past every column
         if (Ragged && tc < cols) orow[tc] = tc == t ? tv * scale - inv_batch : tv * scale;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
@@ -229,7 +233,7 @@ __global__ __launch_bounds__(BS, K == SmKind::Bwd && NCH == 16 ? 3 : 1) void sof
             f32x4 o = v[c] * scale;
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                if ((uint64_t)(4 * f + k) == t) f4_set(o, k, f4_get(o, k) - inv_batch);
+                if (4 * f + k == t) f4_set(o, k, f4_get(o, k) - inv_batch);
             store(f, o);
         }
         return;
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(kLongThreads) void softmax_long_kernel(SmArgs a) {
     o.s *= o.m == ninf ? 1.0f : exp_diff(o.m - m);
     const float s = block_combine<false, kWavesB>(wave_sum(o.s), red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
-    const float inv_batch = 1.0f / (float)a.batch;
+    const float inv_batch = a.inv_batch;
     const float scale = (K == SmKind::CeBwd) ? inv * inv_batch : inv;
     auto value = [&](uint32_t f, f32x4 x) {  // outputs of float4 f
 #pragma unroll
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(kSmBlock) void softmax_loop_kernel(SmArgs a) {
     }
     s = block_combine<false>(wave_sum(s), red);
     const float inv = (K == SmKind::Causal) ? (s > 0.0f ? 1.0f / s : 0.0f) : 1.0f / s;
-    const float inv_batch = 1.0f / (float)a.batch;
+    const float inv_batch = a.inv_batch;
     const float scale = (K == SmKind::CeBwd) ? inv * inv_batch : inv;
     const uint64_t t = (K == SmKind::CeBwd) ? target_index(a.b[row], a.cols) : ~0ull;
     for (uint64_t i = threadIdx.x; i < n; i += kSmBlock) {
@@ -498,75 +502,101 @@ static void launch_long(const SmArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((softmax_long_kernel<K, R, kLds, Ragged>), dim3((uint32_t)a.rows), dim3(kLongThreads), lds, s, a);
 }
 
-// Ragged rows of 769-1024 columns and whole ones of 1024: a workgroup of 128
-// threads x 2 float4 per row instead of a wave x 4 of each of four rows, whose
-// workgroup ends with its slowest row (graph replays, us: causal 1023 x 1023 4.33
-// -> 4.05, 16368 x 1023 25.7 -> 24.3, softmax 32768 x 1023 49.7 -> 45.8, 64 x 1024
-// 2.50 -> 2.29).  Up to 768 columns a quarter of its threads idle (8000 x 600
-// 8.6 against 9.4), and whole rows that do not fill them are slower too (512 x
-// 964 3.3 against 3.5, 1023 x 900 3.6 against 3.9).  Backward: ragged rows
-// 256 threads x 1 float4 of each operand (512 x 1023 3.9 -> 3.5, 16368 x 1023
-// 36.8 -> 33.9), but 3000 x 1023 7.8 against 8.7; whole float4 only for few rows
-// (64 x 1024 2.17 -> 1.97; 3000 x 1024 7.3 against 7.6, 32768 61.8 against 63.6),
-// as the logits' (4096 x 1024 6.3 against 6.4).
+template <SmKind K, int NCH, bool Ragged, int BS>
+static void launch_block(const SmArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((softmax_reg_kernel<K, NCH, true, Ragged, BS>), dim3((uint32_t)a.rows), dim3(BS), 0, s, a);
+}
+
 template <SmKind K, bool Ragged>
-static bool one_row_groups(uint64_t rows) {
-    if (K == SmKind::Bwd && Ragged) return rows <= 1536 || rows >= 5120;
-    if (K == SmKind::Bwd || (K == SmKind::CeBwd && !Ragged)) return rows <= 2048;
-    return true;
+static void launch_loop(const SmArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((softmax_loop_kernel<K, !Ragged>), dim3((uint32_t)a.rows), dim3(kSmBlock), 0, s, a);
+}
+
+// 513-1024 columns in a workgroup of 128 threads x 2 float4 per row instead of a
+// wave x 4 of each of four rows, whose workgroup ends with its slowest row.
+// Graph replays, us, wave against workgroup (so below too): ragged backward 64 x
+// 767 2.27 -> 2.17, 2300 x 1023 6.2 -> 5.6 (16368 x 513 18.2 against 19.7);
+// ragged forward from 769 columns, 16368 x 1023 25.7 -> 24.3, as up to 768 a
+// quarter of the workgroup idles (8000 x 600 8.6 against 9.4).  Whole rows only
+// where they fill it (512 x 964 3.3 against 3.5) and while its rounds are few: 64
+// x 1024 2.55 -> 2.31, 2560 4.46 -> 4.31, but 3300 4.89 against 5.15 and 5120 5.7
+// against 7.6 (softmax 16368 22.7 -> 21.5 again, logits 20.3 against 21.5); backward 1536 x 1024 4.25 -> 3.93, but 2048 4.9 against 5.4.
+template <SmKind K, bool Ragged>
+static bool two_waves_a_row(uint64_t rows, uint64_t cols4) {
+    if (Ragged) return cols4 > (K == SmKind::Bwd ? 128u : 192u);
+    if (cols4 != 256) return false;
+    if (K == SmKind::Fwd || K == SmKind::Causal) return rows <= 2560 || rows >= 12288;
+    return rows <= (K == SmKind::Bwd ? 1536u : 2560u);
+}
+
+// 2049-4096 columns.  Forward: 256 threads x 4 float4 per row (512 x 2, half of
+// them idle at 2052 columns, against it: 1100 x 2052 6.2 -> 5.2, 8192 27.6 ->
+// 25.3), but one wave a row where that many waves still fit the chip at once and
+// the workgroups take another round (2900 x 2052 9.1 against 10.3; 1100 6.7
+// against 5.2, 4500 16.0 against 14.8; ragged 2900 x 2049 9.2 against 10.6, 2048
+// 7.8 against 6.9, 3300 13.1 against 11.5; whole rows to 4096 where they are
+// short: 4096 x 2052 12.0 against 13.5, but x 3072 19.5 against 18.7), and 512 threads for many wide rows
+// (8192 x 4096 44.4 against 46.8).  Backward: 256 threads for ragged rows (1100 x
+// 3001 8.3 with 512, 7.8), 512 for whole ones (8192 x 3072 49.9 with a wave a
+// row, 46.4), a wave where the rows are about one or two a SIMD (1024 x 2052
+// 5.55 against 5.92, 2048 x 2052 7.0 against 8.5; 768 4.97 against 4.48, 3072
+// 13.2 against 12.4).
+enum class MidForm { Wave, Group256, Group512 };
+template <SmKind K, bool Ragged>
+static MidForm mid_form(uint64_t rows, uint64_t cols4) {
+    if (K == SmKind::Bwd && !Ragged) return rows > 768 && rows < 3072 ? MidForm::Wave : MidForm::Group512;
+    const uint64_t last = !Ragged && cols4 <= 640 ? 4096 : 3072;
+    if (K != SmKind::Bwd && rows > (Ragged ? 2304u : 1536u) && rows <= last) return MidForm::Wave;
+    return rows > 3072 && cols4 > 768 ? MidForm::Group512 : MidForm::Group256;
 }
 
 // The kernel for the row length.
 template <SmKind K, bool Ragged>
 static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
+    constexpr bool kBwd = K == SmKind::Bwd;
     const uint64_t cols4 = (a.cols + 3) / 4;
-    const dim3 grid((uint32_t)a.rows);
-    if (cols4 <= 64) launch_wave<K, 1, Ragged>(a, s);
+    // Ragged backward, up to 512 columns and few rows: a thread a float, the row
+    // read twice from the cache (512 x 255 2.14 against 2.37, 1792 x 255 2.69
+    // against 2.86; 2300 x 255 3.1 against 3.0, x 511 4.1 against 3.7).
+    if (kBwd && Ragged && cols4 <= 128 && a.rows <= 1792) launch_loop<K, Ragged>(a, s);
+    else if (cols4 <= 64) launch_wave<K, 1, Ragged>(a, s);
     else if (cols4 <= 128) launch_wave<K, 2, Ragged>(a, s);
-    else if (cols4 > (Ragged ? 192u : 255u) && cols4 <= 256 && one_row_groups<K, Ragged>(a.rows)) {
-        constexpr int BS = K == SmKind::Bwd && Ragged ? 256 : 128;
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 256 / BS, true, Ragged, BS>), grid, dim3(BS), 0, s, a);
-    }
+    else if (cols4 <= 256 && two_waves_a_row<K, Ragged>(a.rows, cols4)) launch_block<K, 2, Ragged, 128>(a, s);
     else if (cols4 <= 256) launch_wave<K, 4, Ragged>(a, s);
     else if (cols4 <= 512) {
         // 1025-2048 columns: one workgroup per row streams faster than one
         // wave per row (measured at 32768 x 2048: forward 85.8 -> 83.3 us
         // with 256 threads x 2 float4, backward 129.3 -> 121.7 us with 512
-        // threads x 1 float4 each of y and dy)
-        if (K == SmKind::Bwd)
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 1, true, Ragged, 512>), grid, dim3(512), 0, s, a);
-        else
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+        // threads x 1 float4 each of y and dy; ragged backward 1100 x 1025 4.0
+        // with 512, 3.5 with 256)
+        if constexpr (kBwd && !Ragged) launch_block<K, 1, Ragged, 512>(a, s);
+        else launch_block<K, 2, Ragged, 256>(a, s);
     }
     else if (cols4 <= 1024) {
-        // 2049-4096 columns: a workgroup of 512 threads per row (8192 x 4096
-        // forward 47.1 -> 43.8 us, backward 67.8 -> 62.5; 512 x 4096 5.8 ->
-        // 4.7 and 6.5 -> 5.9 in graph replays), but one wave per row where the
-        // rows about fill the chip once (2048 x 4096 11.7 against 13.6).
-        if (a.rows > 1024 && a.rows < 3072) launch_wave<K, 16, Ragged>(a, s);
-        else hipLaunchKernelGGL((softmax_reg_kernel<K, 2, true, Ragged, 512>), grid, dim3(512), 0, s, a);
+        switch (mid_form<K, Ragged>(a.rows, cols4)) {
+        case MidForm::Wave: return launch_wave<K, 16, Ragged>(a, s);
+        case MidForm::Group256: return launch_block<K, 4, Ragged, 256>(a, s);
+        case MidForm::Group512: return launch_block<K, 2, Ragged, 512>(a, s);
+        }
     }
-    else if (cols4 <= 2048)
-        hipLaunchKernelGGL((softmax_reg_kernel<K, 8, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    else if (cols4 <= 2048) launch_block<K, 8, Ragged, 256>(a, s);
     else if (cols4 <= 4096) {
         // 8193-16384 columns: 512 threads while the rows are few (512 x 16384
         // 12.0 -> 10.9 us, 300 x 9000 7.3 -> 6.7, 64 x 12345 6.6 -> 5.5; 1024 x
         // 12288 logits 18.2 against 20.2, and 300 x 9000 backward 8.2 against 8.6).
-        constexpr int kFew = K == SmKind::Bwd ? kSmBlock : 512;
-        if (a.rows <= 512)
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 4096 / kFew, true, Ragged, kFew>), grid, dim3(kFew), 0, s, a);
-        else
-            hipLaunchKernelGGL((softmax_reg_kernel<K, 16, true, Ragged>), grid, dim3(kSmBlock), 0, s, a);
+        if constexpr (!kBwd) {
+            if (a.rows <= 512) return launch_block<K, 8, Ragged, 512>(a, s);
+        }
+        launch_block<K, 16, Ragged, 256>(a, s);
     }
-    else if (K != SmKind::Bwd && a.cols <= kLongCols) {
-        if constexpr (K != SmKind::Bwd) {
+    else if (!kBwd && a.cols <= kLongCols) {
+        if constexpr (!kBwd) {
             if (cols4 <= 8 * kLongThreads) launch_long<K, 8, Ragged>(a, s);
             else if (cols4 <= 16 * kLongThreads) launch_long<K, 16, Ragged>(a, s);
             else launch_long<K, kLongRegs, Ragged>(a, s);
         }
     }
-    else
-        hipLaunchKernelGGL((softmax_loop_kernel<K, !Ragged>), grid, dim3(kSmBlock), 0, s, a);
+    else launch_loop<K, Ragged>(a, s);
 }
 
 template <SmKind K>
@@ -580,7 +610,7 @@ static int softmax_launch(const SmArgs& a, hipStream_t s) {
     const bool aligned = (a.cols % 4 == 0) && aligned16(a.a) && aligned16(a.out) &&
                          (K != SmKind::Bwd || aligned16(a.b));
     SmArgs band = a;
-    band.batch = a.rows;
+    band.inv_batch = 1.0f / (float)a.rows;
     for (uint64_t left = a.rows; left > 0;) {
         band.rows = left < kLaunchRows ? left : kLaunchRows;
         if (aligned)
@@ -588,7 +618,7 @@ static int softmax_launch(const SmArgs& a, hipStream_t s) {
         else if (a.cols >= 4)
             softmax_dispatch<K, true>(band, s);
         else  // ragged rows are read four floats at a time
-            hipLaunchKernelGGL((softmax_loop_kernel<K, false>), dim3((uint32_t)band.rows), dim3(kSmBlock), 0, s, band);
+            launch_loop<K, true>(band, s);
         left -= band.rows;
         band.a += band.rows * a.cols;
         band.out += band.rows * a.cols;

@@ -560,8 +560,8 @@ def _softmax64(x):
     e = np.exp(x - x.max(axis=-1, keepdims=True))
     return e / e.sum(axis=-1, keepdims=True)
 
-# one shape per kernel path: wave per row (<= 256/512/1024/2048/4096 cols),
-# workgroup per row (<= 8192/16384), looped (longer rows, cols % 4 != 0)
+# few rows of each range of lengths, whole and ragged; the row counts and lengths
+# where the kernel changes are test_gpu_row_shapes.py's
 SOFTMAX_SHAPES = [(1, 1), (3, 7), (5, 4), (4, 256), (7, 260), (9, 512), (6, 1000), (33, 2048), (5, 4096),
                   (5, 1028), (3, 1500),
                   (3, 8192), (2, 16384), (2, 20000), (3, 4099), (2, 128256)]

@@ -87,9 +87,13 @@ SM_LENGTHS = [(9, 3, 1), (5, 250, 2), (6, 257, 3), (7, 511, 0), (5, 1023, 1), (3
               (2, 4093, 3), (2, 8189, 0), (2, 16383, 2), (2, 16385, 0), (2, 16388, 0), (2, 32768, 0), (2, 32769, 1),
               (2, 65536, 0), (2, 65539, 0), (2, 98304, 3), (2, 98308, 0), (2, 131071, 0), (2, 135168, 0),
               (2, 135169, 0)]
-# The same around the lengths and row counts where a row's workgroup changes.
-SM_LENGTHS += [(5, 768, 1), (5, 769, 1), (3, 771, 0), (6, 960, 0), (6, 961, 0), (7, 964, 0), (5, 1021, 3),
-               (1537, 1001, 1), (2049, 964, 0), (5120, 801, 2), (512, 8196, 0), (513, 8193, 1)]
+# The same around the lengths and row counts where a row's kernel changes: a thread a float or a wave for a ragged
+# backward of up to 512 columns, one or two waves a row to 1024, one wave, 256 or 512 threads from 2049 to 4096 (whole
+# and ragged, forward and backward each have their own counts), 256 or 512 from 8193.
+SM_LENGTHS += [(5, 513, 2), (5, 768, 1), (5, 769, 1), (3, 771, 0), (6, 960, 0), (6, 961, 0), (7, 964, 0), (5, 1021, 3),
+               (1792, 101, 1), (1793, 102, 3), (1793, 301, 2), (1537, 1001, 1), (1537, 1024, 0), (2561, 1024, 0),
+               (2049, 964, 0), (5120, 801, 2), (768, 2052, 0), (769, 2052, 0), (1537, 2052, 0), (2305, 2049, 3),
+               (3073, 2564, 0), (3073, 3073, 1), (3073, 3076, 0), (512, 8196, 0), (513, 8196, 0), (513, 8193, 1)]
 
 
 def _rows_with_specials(rows, cols, seed):

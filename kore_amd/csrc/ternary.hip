@@ -2888,12 +2888,16 @@ static bool f32_use_mf4(uint64_t m, uint64_t n, uint64_t k, uint64_t kp) {
 //   4 x 4: 3712 x 96 x 2375 41 (56 where it needed K >= 2560), 2048 x 200 x 2048
 //     35 (50), 6912 x 40 x 2560 43 (59 below 41 columns);
 //   row-broadcast: 2560 x 64 x 6912 89 (102 from 640 waves of the 4 x 4).
-// Up to 32 columns the row-broadcast kernel's narrower tiles win everywhere
-// (6912 x 32 x 2560 37 against 43 and 56).
+// Up to 32 columns the row-broadcast kernel's narrower tiles win (6912 x 32 x
+// 2560 37 against 43 and 56) up to the rows where the 16 x 16 waves come to
+// kMfMinWaves, as on [K, N] b: 24576 x 32 x 2560 76 us there, 56 on 16 x 16;
+// 49152 x 8 80 and 57; 128256 x {8, 32} x 2560 192 and 355, 95 and 174.  The
+// same below 80 columns of K, where the starts decide, which the model does not
+// tell apart (6912 x 128 x 40 11.4 us row-broadcast, 8.1 on 16 x 16).
 enum class F32Form { Rows, Mf4, Mfma };
 static F32Form f32_layer_form(uint64_t m, uint64_t n, uint64_t k, uint64_t kp) {
     if ((n + 15) / 16 > 65535) return F32Form::Mfma;  // refused there, as ever
-    if (n <= 32) return F32Form::Rows;
+    if (n <= 32 || k < 80) return f32_use_mfma(m, n, k) ? F32Form::Mfma : F32Form::Rows;
     const uint64_t n64 = (n + 63) / 64;
     const auto rounds = [](uint64_t have, uint64_t at_once) { return (double)((have + at_once - 1) / at_once); };
     const double kd = (double)k;

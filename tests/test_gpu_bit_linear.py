@@ -231,12 +231,13 @@ def test_bit_linear_unaligned_buffers(off):
 @pytest.mark.parametrize("m,batch,k", [(4097, 48, 2563), (2049, 130, 2605), (1500, 192, 6912), (4100, 41, 2560),
                                        (6000, 64, 3201), (4100, 64, 6917), (2560, 64, 6912), (2600, 41, 2561)])
 def test_bit_linear_f32_matrix_core_decode_batches(m, batch, k):
-    """The 4 x 4 x 1 matrix-core kernel that takes the f32 layer at 41-192
-    tokens (token-major input; K >= 2560 and at least 640 waves of 4 rows x
-    64 tokens): ragged row groups (m % 4 == 1, where the packed matrix ends
-    inside a dword), partial last column tiles, K not a multiple of the
-    80-column chunk or of 5, 6912 columns of packed rows held in LDS; with Inf, NaN and subnormal inputs in some tokens (their
-    chunks fold element by element, zero trits skipped).  Bit-exact against
+    """Decode batches of the f32 layer (token-major input), on the 4 x 4 x 1
+    matrix-core kernel but for the two of 2560 and 2600 rows, which the
+    row-broadcast kernel takes: ragged row groups (m % 4 == 1, where the packed
+    matrix ends inside a dword), partial last column tiles, K not a multiple of
+    the 80-column chunk or of 5, 6912 columns of packed rows held in LDS; with
+    Inf, NaN and subnormal inputs in some tokens (their chunks fold element by
+    element, zero trits skipped).  Bit-exact against
     the oracle's composition on the tokens it finishes in seconds and against
     the device's ternary_matmul_f32 on x^T (another kernel) on every token."""
     log(f"bit_linear_f32 4x4 matrix cores m={m} batch={batch} k={k}")
@@ -270,8 +271,8 @@ def test_bit_linear_f32_prefill_nonfinite(m, batch, k):
     """The kernels that load the layer's token-major input straight into LDS
     and find Inf/NaN from the sums after each chunk (the chunk refolded with
     zero trits skipped): the 16 x 16 matrix-core kernel (K a multiple of 4)
-    and the row-broadcast kernel in 64-, 32- and 16-column tiles (7, 2 and 2
-    rows per lane; partial last chunks).  Tokens with Inf, -Inf, NaN,
+    and the row-broadcast kernel in 32- and 16-column tiles (2 rows per lane;
+    partial last chunks).  Tokens with Inf, -Inf, NaN,
     subnormal and overflowing inputs, bit-exact against the oracle on those
     tokens and against ternary_matmul_f32 on x^T (other staging) on every
     token."""
@@ -304,7 +305,7 @@ def test_bit_linear_f32_prefill_nonfinite(m, batch, k):
 
 @pytest.mark.parametrize("seed", range(6))
 def test_bit_linear_f32_matrix_core_random_shapes(seed):
-    """Random shapes across the 4 x 4 x 1 kernel's range (41-192 tokens,
+    """Random shapes that take the 4 x 4 x 1 kernel (41-192 tokens,
     2560-7680 input features, at least 1024 waves): bit-exact against the oracle on the
     first tokens and against ternary_matmul_f32 on x^T (the row-broadcast or
     16 x 16 kernel, never this one) on every token."""

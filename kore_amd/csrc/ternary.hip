@@ -31,9 +31,10 @@
 //   same for both operands, so any assignment gives the same sum);
 //   accumulator register r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
 //   column l % 32.
-// One code row (two with long K): the small-n path (dot4 on decoded windows, no
-// MFMA); then up to 256 tiles of 128 x 128 (k >= 16): the skinny path (32 or 64
-// weight rows per workgroup, K split over its waves and summed exactly in LDS);
+// One code row (two with few weight rows and long K): the small-n path (dot4 on
+// decoded windows, no MFMA); then up to 64 codes, or 256 tiles of 128 x 128 (k >=
+// 16, see skinny_wins): the skinny path (32 or 64 weight rows per workgroup, K
+// split over its waves and summed exactly in LDS);
 // then tiles of 256 x 128, and at least 144 tiles of 256 x 256: the wide kernel
 // (both below).  Code rows that are not 16-byte aligned (K % 16 != 0 or an
 // unaligned q) take the skinny kernel and, beyond it, the tile kernel with
@@ -345,11 +346,11 @@ __global__ __launch_bounds__(kTmBlock) void ternary_i8_mfma_kernel(TernArgs p) {
 // LDS traffic per MFMA is ~0.7 KB (operand reads 0.5, table reads 0.2)
 // against the ~1 KB one CU delivers per MFMA of each of its four SIMDs.
 constexpr int kWdM = 256, kWdN = 256;
-// The wide kernel runs one workgroup per CU; below 144 tiles of 256 x 256
-// the 128 x 128 kernel (more, smaller workgroups) is faster: measured wide
-// against 128 x 128 at 4096 x 2048 x 2560 (128 tiles) 45.9 vs 39.7 us, and at
-// 3072 x 3072 x 2560 (144) 41.2 vs 49.0, 2560 x 4096 x 6912 (160, unaligned
-// rows) 107.1 vs 133.6, 6912 x 2048 (216) 49.7 vs 73.7.
+// The wide kernel runs one workgroup per CU, from 144 tiles of 256 x 256; below
+// that the 256 x 128 kernel runs (more, smaller workgroups).  The line is where
+// 128 x 128 tiles, which ran below it before, stopped being faster: 4096 x 2048 x
+// 2560 (128 tiles) 45.9 us wide against 39.7, 3072 x 3072 x 2560 (144) 41.2
+// against 49.0, 2560 x 4096 x 6912 (160, unaligned rows) 107.1 against 133.6.
 constexpr uint64_t kWdMinTiles = 144;
 constexpr uint64_t kCus = 256;  // MI355X compute units
 constexpr int kWdPitch = 176;
@@ -912,11 +913,19 @@ __global__ __launch_bounds__(kWaves * kWave) void ternary_i8_skinny_kernel(TernA
     __syncthreads();  // table filled
     for (; kb < nkb; kb += kWaves) {
         // this block's codes into the wave's tile (after the last block's reads)
-        if (kb == nkb - 1u) {
+        // A block past k: whole pieces to clear where K is a multiple of 16 (the
+        // shifts cost a short K 0.2 us: 6912 x 32 x 1024 5.1 -> 5.0), else parts.
+        if (kb * kTmK + kTmK > p.k) {
+            if (p.k % 16u == 0) {
 #pragma unroll
-            for (int u = 0; u < kPieces; ++u) {
-                const uint32_t c = kb * kTmK + bcol[u];
-                bv[u] = bytes_down(bv[u], c + 16u <= p.k ? 0u : min(c + 16u - p.k, 16u));
+                for (int u = 0; u < kPieces; ++u)
+                    if (kb * kTmK + bcol[u] >= p.k) bv[u] = u32x4{0u, 0u, 0u, 0u};
+            } else {
+#pragma unroll
+                for (int u = 0; u < kPieces; ++u) {
+                    const uint32_t c = kb * kTmK + bcol[u];
+                    bv[u] = bytes_down(bv[u], c + 16u <= p.k ? 0u : min(c + 16u - p.k, 16u));
+                }
             }
         }
         wave_lds_sync();
@@ -1042,10 +1051,14 @@ static int launch_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
 // would waste most of their columns.
 constexpr int kGvRows = 4;     // weight rows per wave group
 constexpr int kGvChunk = 2560; // columns per lane-window sweep (64 lanes x 40)
-// One code row, and two from this many columns; the skinny kernel takes the
-// others (measured, graph replays: 6912 x 2 x 2560 5.2 us here against 4.8, x 8
-// 12.0 against 5.1; 2560 x 2 x 6912 6.8 against 7.8, x 4 9.0 against 8.1).
-constexpr uint64_t kGvTwoK = 5120;
+// One code row; two of them for few weight rows and long K, and below the skinny
+// kernel's 16 columns.  Measured against the skinny kernel, graph replays: 2560 x
+// 2 x 2560 4.2 against 4.5 us, x 6912 6.8 against 8.5, but x 1024 4.7 against 4.0,
+// and 6912 x 2 x 2560 5.2 against 4.7, x 6912 9.2 against 7.5; 2560 x 4 x 6912 9.0
+// against 8.1.
+static bool small_n_wins(uint64_t m, uint64_t n, uint64_t k) {
+    return n == 1 || (n == 2 && ((m <= 4096 && k > 2048) || k < 16));
+}
 
 __device__ __forceinline__ int32_t wave_sum_i32(int32_t v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
@@ -3776,21 +3789,28 @@ static void launch_wide(bool aligned_a, dim3 g, hipStream_t s, const TernArgs& p
 
 using namespace kore;
 
-// Where the skinny kernel runs: up to 256 tiles of 128 x 128 (what the tile
-// kernel ran there before: one round of the CUs, its K split over workgroups
-// and summed with atomics in two more launches where they were few).  Its form follows from how many
-// workgroups each gives.  Measured in graph replays, us, m x k at n codes:
-//   6912 x 2560: n = 8 (the small-n kernel before) 12.0 -> 5.1, 100 (the tile
-//     kernel, as all that follow) 24.0 -> 10.6, 200 29.9 -> 16.3, 400 32.2 ->
-//     27.4; past 256 tiles the 256 x 128 kernel (600 codes 28.8 against 39.1,
-//     at 400 both 28);
-//   2560 x 6912: 45 (32 rows x 64 codes, 8 waves before) 11.7 -> 8.8, 200 28.5
-//     -> 17.6, 400 39.9 -> 30.4, 800 67 -> 47;
+// Where the skinny kernel runs: up to 64 codes, and beyond up to 256 tiles of 128
+// x 128 (about one round of the CUs).  Measured in graph replays, us, m x k at n
+// codes, against the kernel that would run instead:
+//   6912 x 2560: n = 8 12.0 (small-n kernel) -> 5.1, 100 24.0 (128 x 128 tiles, as
+//     all that follow) -> 10.6, 200 29.9 -> 16.3, 400 32.2 -> 27.4; past 256 tiles
+//     the 256 x 128 kernel (600 codes 28.8 against 39.1, at 400 both 28);
+//   2560 x 6912: 200 28.5 -> 17.6, 400 39.9 -> 30.4, 800 67 -> 47;
 //   3712 x 2375 (code rows not 16-byte aligned): 1 16.6 -> 5.2, 45 17.3 -> 7.1,
 //     200 27.4 -> 13.4, 800 42.8 -> 31.4;
-//   1024 x 1001: 100 13.9 -> 5.7, 800 17.7 -> 10.2.
-static bool skinny_wins(uint64_t m, uint64_t n) {
-    return ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN) <= 256;
+//   128256 x 2560 (256 x 192 tiles): 2 66 -> 26.4, 32 71 -> 31; x 6912 64 171 ->
+//     114; x 2568 (128 x 128 tiles): 2 93 -> 34, 64 156 -> 90.
+// Aligned code rows leave to the 256 x 128 kernel what it does faster: 33-64 codes
+// from 57344 weight rows unless K is long (128256 x 64 x 2560 47 against 57, x 1024
+// 25 against 67, but x 6912 117 against 114; 50257 x 64 x 2560 32 against 28; up to
+// 512 columns from 40960: 50257 x 33 x 160 9.0 against 12.6), and 65-128 codes
+// from 28672 (32768 x 65 x 512 13.8 against 18.8, x 2560 27.4 against 30.2, but x
+// 6912 69 against 60; 24576 x 65 x 2560 27.3 against 25.1).
+constexpr uint64_t kSkLongK = 5120;
+static bool skinny_wins(uint64_t m, uint64_t n, uint64_t k, bool vec) {
+    if (n <= 32) return true;
+    if (vec && k <= kSkLongK && n <= 128 && m > (n > 64 ? 28672u : k <= 512 ? 40960u : 57344u)) return false;
+    return n <= 64 || ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN) <= 256;
 }
 
 static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
@@ -3798,9 +3818,17 @@ static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
     // 32 x 32 outputs a workgroup of 8 waves while that is up to two a CU (more
     // of them, shorter; 2560 x 45 x 6912 8.8 us against 11.7 with 32 x 64, 3712
     // x 100 x 2375 10.0 against 12.6 with 64 x 64);
-    if (n32 == 1 || m32 * n32 <= (n64 == 1 ? 416u : 512u)) return launch_skinny<1, 1, 8>(p, aligned_a, s);
-    // one code tile: 32 x 64 (6912 x 64 x 2560 7.0 against 7.6);
-    if (n64 == 1) return launch_skinny<1, 2, 8>(p, aligned_a, s);
+    if (m32 * n32 <= 2 * kCus) return launch_skinny<1, 1, 8>(p, aligned_a, s);
+    if (n64 == 1 && (n32 == 1 || p.k <= kSkLongK)) {
+        // then one to two code tiles of 32, each with 32 weight rows and 4 waves
+        // (24576 x 32 x 2560 9.8 against 11.2 with 8; 14336 x 64 x 512 6.1 against
+        // 10.0 in 32 x 64), or 64, which read the codes half as often, once those
+        // fill the chip (65536 x 9 x 6912 36 against 39, 128256 x 32 x 2560 31
+        // against 35; 50257 x 32 x 512 10.5 against 9.6) and for two tiles
+        // (24576 x 64 x 2560 13.2 against 14.4; 14336 x 64 x 512 6.8 against 6.1);
+        if (n32 == 1 ? m32 < 2048 : m32 * n32 <= 4 * kCus && p.k <= 1024) return launch_skinny<1, 1, 4>(p, aligned_a, s);
+        return launch_skinny<2, 1, 4>(p, aligned_a, s);
+    }
     // then 64 x 64, each staged code read by two MFMAs, of 8 waves up to one a
     // CU (3712 x 200 x 2375 13.4 against 14.9) and of 4 beyond (6912 x 200 x
     // 2560 16.3 against 19.8).
@@ -3837,7 +3865,7 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
     TernArgs p{a_packed, a_scales, q,  q_scales, c, (uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)kp,
                bias,     trans ? 1u : 0u};
     const bool c_ok = (reinterpret_cast<uintptr_t>(c) & 3u) == 0;
-    if (n <= (k > kGvTwoK ? 2u : 1u) && k > 0 && k % 8 == 0 && (reinterpret_cast<uintptr_t>(q) & 7u) == 0 && c_ok) {
+    if (k > 0 && small_n_wins(m, n, k) && k % 8 == 0 && (reinterpret_cast<uintptr_t>(q) & 7u) == 0 && c_ok) {
         // grid: at most m / 4 blocks of one wave group (m < 2^31)
         const bool al8 = kp % 8 == 0 && (reinterpret_cast<uintptr_t>(a_packed) & 7u) == 0;
         if (al8) {
@@ -3850,7 +3878,7 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         return launch_status();
     }
     const bool vec = k > 0 && k % 16 == 0 && aligned16(q) && c_ok;
-    if (k >= 16 && c_ok && skinny_wins(m, n))
+    if (k >= 16 && c_ok && skinny_wins(m, n, k, vec))
         return ternary_i8_skinny(p, kp % 16 == 0 && aligned16(a_packed), s);
     const uint64_t wide_tiles = ((m + kWdM - 1) / kWdM) * ((n + kWdN - 1) / kWdN);
     const bool al = kp % 16 == 0 && aligned16(a_packed);
@@ -3863,12 +3891,16 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         else launch_w2_t<false>(al, g, s, p);
         return launch_status();
     };
-    // Past the skinny kernel's range and below the wide one's: 256 x 128 tiles,
-    // about one a CU, their K loop two to three times the 128 x 128 kernel's
+    // Past the skinny kernel's range and below the wide one's, and for one tile
+    // column whatever the rows (128256 x 100 x 2560 48.8 us against 78.9 in 256 x
+    // 192 tiles, x 6912 120 against 173): 256 x 128 tiles, up to about one a CU, their K loop two to three times the 128 x 128 kernel's
     // rate (measured, graph replays: 6912 x 800 x 2560 39.4 -> 30.2 us, 2560 x
     // 1600 x 6912 87.3 -> 70.4, 5376 x 1000 x 896 25.3 -> 19.1, 4096 x 1200 x
     // 4096 57.8 -> 45.5, 2048 x 3000 x 2048 37.7 -> 28.3).
-    if (vec && wide_tiles < kWdMinTiles && nk < (1ull << 31)) return launch_w2();
+    // (up to 128 rows fill half of such a tile at most: 64 x 33000 x 2560 38 us in
+    // 128 x 128 tiles, 41 here)
+    if (vec && nk < (1ull << 31) && m > (uint64_t)kTmM && (wide_tiles < kWdMinTiles || n <= (uint64_t)kW2N))
+        return launch_w2();
     if (vec && wide_tiles >= kWdMinTiles && nk < (1ull << 31)) {
         // Many output tiles: the wide kernel (one 256 x 256 tile per CU), or
         // 256 x 192 tiles where the rounds of 256 CUs they need, at ~0.8 of a

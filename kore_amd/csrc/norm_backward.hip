@@ -30,7 +30,7 @@
 //   * other rows: their workspace is one float per row, so the partial rows
 //     wait in the last P rows of dx, and the column pass computes those rows'
 //     dx after it has added them (rms_bwd_finish_kernel).
-// Generic path (longer rows, a single row): one workgroup per row writes dx
+// Generic path (longer rows, few ragged or long ones): one workgroup per row writes dx
 // and inv[r] to the workspace; then one thread per column folds its dgamma
 // over the rows in the reference's order.
 #include <mutex>
@@ -364,6 +364,16 @@ static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols) {
     return vec > rows ? vec : rows;
 }
 
+// Rows of the generic path where the workspace plan does not run: a workgroup a
+// row and a thread a dgamma column, against the long path's two launches that
+// few rows leave waiting on 16 waves' barriers (us, generic against long path):
+// 16 x 257 5.9 against 9.2, 48 9.9 against 9.4; 64 x 1001 12.3 against 13.8, 80
+// 14.3 against 13.8; 32 x 3001 10.4 against 11.0, 48 12.4 against 11.1; 8 x 4100
+// 8.5 against 8.9, 16 9.5 against 9.1; 2 x 7000 10.6 against 9.7.
+static uint64_t bwd_generic_rows(uint64_t cols) {
+    return cols <= 512 ? 44 : cols <= 1024 ? 72 : cols <= 4096 ? 36 : cols <= 5120 ? 8 : 1;
+}
+
 template <int NCHW, int S>
 static void launch_rows(const BwArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwWaves, false>), dim3((uint32_t)a.partials), dim3(kBwBlock), 0,
@@ -384,12 +394,15 @@ constexpr uint64_t kBwLongBlocks = 256;
 
 template <int NCHW, int S>
 static void launch_long(const BwArgs& a, bool ragged, hipStream_t s) {
-    constexpr int W = S > kBwLongWaves ? S : kBwLongWaves;
-    const dim3 grid((uint32_t)a.partials), block(W * kWave);
-    if (ragged)
-        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, true>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, W, false>), grid, block, 0, s, a);
+    static_assert(S <= kBwLongWaves, "a workgroup holds a row");
+    const dim3 grid((uint32_t)a.partials), block(kBwLongWaves * kWave);
+    if constexpr (S >= 8) {  // shorter whole rows take the workspace plan
+        if (!ragged) {
+            hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwLongWaves, false>), grid, block, 0, s, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((rms_bwd_rows_kernel<NCHW, S, kBwLongWaves, true>), grid, block, 0, s, a);
 }
 
 // Library-held scratch for the allocation-free entry point: the dgamma
@@ -497,12 +510,12 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         else launch_rows<4, 4>(a, s);
         hipLaunchKernelGGL(rms_bwd_reduce_kernel, dim3((uint32_t)((cols4 + kRedCols - 1) / kRedCols)),
                            dim3(kRedCols * kRedSlots), 0, s, a);
-    } else if (cols <= 16384 && rows > 1) {
+    } else if (cols <= 16384 && rows > bwd_generic_rows(cols)) {
         // The workspace of these shapes holds one float per row, so the P
         // partial rows wait in dx's last P rows until the second launch has
         // reduced them and computes those rows' dx; 2 P <= rows, the inv and
         // coeff it needs being the workspace's first 2 P floats.
-        const uint64_t slots = split > (uint32_t)kBwLongWaves ? 1 : (uint32_t)kBwLongWaves / split;
+        const uint64_t slots = (uint32_t)kBwLongWaves / split;
         uint64_t rpb = (rows + kBwLongBlocks - 1) / kBwLongBlocks;
         if (rpb < 2) rpb = 2;
         rpb = (rpb + slots - 1) / slots * slots;

@@ -77,14 +77,15 @@ struct TernArgs {
     float* c;           // [M, N], or [N, M] with trans
     uint32_t m, n, k, kp;
     const float* bias;  // [M] added to every output of row m, or null
-    uint32_t trans;     // 1: output (m, n) at c[n * M + m] (BitLinear::forward's layout)
+    uint32_t trans;     // 1: output (m, n) at c[n * ld + m] (BitLinear::forward's layout)
+    uint32_t ld;        // row stride of c: the whole call's N, or M with trans
 };
 
 // Index of output (m, n) in c, and the layer's bias add: the output is
 // rounded first, then the bias is added to it (bit_linear.rs:220-224 adds
 // the bias to the finished matmul output).
 __device__ __forceinline__ uint64_t out_idx(const TernArgs& p, uint32_t m, uint32_t n) {
-    return p.trans ? (uint64_t)n * p.m + m : (uint64_t)m * p.n + n;
+    return (uint64_t)(p.trans ? n : m) * p.ld + (p.trans ? m : n);
 }
 __device__ __forceinline__ float add_bias(const float* bias, float v, uint32_t m) { return bias ? v + bias[m] : v; }
 
@@ -1238,23 +1239,25 @@ static void launch_gemv(const TernArgs& p, uint64_t m, uint64_t k, hipStream_t s
     else hipLaunchKernelGGL((ternary_i8_gemv_kernel<NT, kAligned8, 1>), g, b, 0, s, p);
 }
 
-// Generic path: one thread per output, integer accumulation in k order.
+// Generic path: one thread per output (in turns past 2^31 of them), integer
+// accumulation in k order.
 __global__ __launch_bounds__(kTmBlock) void ternary_i8_generic_kernel(TernArgs p) {
     __shared__ uint64_t lut[256];
     lut[threadIdx.x] = trit_lut_entry(threadIdx.x);
     __syncthreads();
-    const uint64_t idx = (uint64_t)blockIdx.x * kTmBlock + threadIdx.x;
-    if (idx >= (uint64_t)p.m * p.n) return;
-    const uint32_t m = (uint32_t)(p.trans ? idx % p.m : idx / p.n), n = (uint32_t)(p.trans ? idx / p.m : idx % p.n);
-    const uint8_t* ar = p.a + (uint64_t)m * p.kp;
-    const int8_t* qr = p.q + (uint64_t)n * p.k;
-    int32_t acc = 0;
-    for (uint32_t k = 0; k < p.k; ++k) {
-        const uint64_t v = lut[ar[k / 5]];
-        const int8_t tr = (int8_t)(uint8_t)(v >> (8 * (k % 5)));
-        acc += (int32_t)tr * (int32_t)qr[k];
+    for (uint64_t idx = (uint64_t)blockIdx.x * kTmBlock + threadIdx.x; idx < (uint64_t)p.m * p.n;
+         idx += (uint64_t)gridDim.x * kTmBlock) {
+        const uint32_t m = (uint32_t)(p.trans ? idx % p.m : idx / p.n), n = (uint32_t)(p.trans ? idx / p.m : idx % p.n);
+        const uint8_t* ar = p.a + (uint64_t)m * p.kp;
+        const int8_t* qr = p.q + (uint64_t)n * p.k;
+        int32_t acc = 0;
+        for (uint32_t k = 0; k < p.k; ++k) {
+            const uint64_t v = lut[ar[k / 5]];
+            const int8_t tr = (int8_t)(uint8_t)(v >> (8 * (k % 5)));
+            acc += (int32_t)tr * (int32_t)qr[k];
+        }
+        p.c[out_idx(p, m, n)] = add_bias(p.bias, ((float)acc * p.sa[m]) * p.sq[n], m);
     }
-    p.c[idx] = add_bias(p.bias, ((float)acc * p.sa[m]) * p.sq[n], m);
 }
 
 // ---------------------------------------------------------------------------
@@ -3694,7 +3697,7 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) sam[i] = p.sa[min(mw + 32 * i + r, p.m - 1u)];
         const uint32_t mc = mw + 4 * (lane & 15);
-        const bool vec_out = (p.m & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+        const bool vec_out = (p.ld & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
         f32x4 bias4 = {0.f, 0.f, 0.f, 0.f};
         if (p.bias) {
 #pragma unroll
@@ -3718,7 +3721,7 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
                 f32x4 v = *reinterpret_cast<const f32x4*>(slab + row * kTp + 4 * (lane & 15));
                 v = v * sqn;
                 if (p.bias) v = v + bias4;
-                float* crow = p.c + (uint64_t)n * p.m;
+                float* crow = p.c + (uint64_t)n * p.ld;
                 if (vec_out && mc + 3 < p.m) {
                     __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(crow + mc));
                 } else {
@@ -3735,7 +3738,7 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) sqn[j] = p.sq[min(n0 + 32 * j + r, p.n - 1u)];
     float* slab = reinterpret_cast<float*>(wlds) + wave * 32 * kW2EpPitch;
-    const bool vec_out = (p.n & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
+    const bool vec_out = (p.ld & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const uint32_t mb = m0 + 64 * wave + 32 * i;
@@ -3754,7 +3757,7 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
             if (m >= p.m) continue;
             f32x4 v = *reinterpret_cast<const f32x4*>(slab + row * kW2EpPitch + col);
             if (p.bias) v = v + p.bias[m];
-            float* crow = p.c + (uint64_t)m * p.n;
+            float* crow = p.c + (uint64_t)m * p.ld;
             const uint32_t nc = n0 + col;
             if (vec_out && nc + 3 < p.n) {
                 __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(crow + nc));
@@ -3836,38 +3839,22 @@ static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
     return launch_skinny<2, 2, 4>(p, aligned_a, s);
 }
 
-// The int8 matmul with the output in either layout (trans: c[n, m]) and an
-// optional bias per weight row.
-static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const int8_t* q, const float* q_scales,
-                          const float* bias, float* c, uint64_t m, uint64_t n, uint64_t k, bool trans,
-                          hipStream_t s) {
-    if (m == 0 || n == 0) return KORE_HIP_OK;
-    if (!c || !a_scales || !q_scales) return KORE_HIP_ERR_NULL_PTR;
-    if (k > 0 && (!a_packed || !q)) return KORE_HIP_ERR_NULL_PTR;
-    // |sum| <= 127 * k must stay exact in int32 and every index in 32 bits.
-    if (m > 0x7fffffffull || n > 0x7fffffffull || k > (1ull << 24)) return KORE_HIP_ERR_OVERFLOW;
-    uint64_t mn, nk;
-    if (!mul_ok(m, n, &mn) || mn > kMaxElements || !mul_ok(n, k, &nk) || nk > kMaxElements)
-        return KORE_HIP_ERR_OVERFLOW;
-    const uint64_t kp = (k + 4) / 5;
-    // c is written while the inputs are read: it must not overlap any of them.
-    {
-        const char* c0 = reinterpret_cast<const char*>(c);
-        const char* c1 = c0 + mn * sizeof(float);
-        const struct { const void* p; uint64_t bytes; } ins[] = {
-            {a_packed, m * kp}, {q, nk}, {a_scales, m * sizeof(float)}, {q_scales, n * sizeof(float)},
-            {bias, bias ? m * sizeof(float) : 0u}};
-        for (const auto& in : ins) {
-            const char* i0 = reinterpret_cast<const char*>(in.p);
-            if (in.p && in.bytes && i0 < c1 && c0 < i0 + in.bytes) return KORE_HIP_ERR_ALIAS;
-        }
-    }
-    TernArgs p{a_packed, a_scales, q,  q_scales, c, (uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)kp,
-               bias,     trans ? 1u : 0u};
-    const bool c_ok = (reinterpret_cast<uintptr_t>(c) & 3u) == 0;
-    if (k > 0 && small_n_wins(m, n, k) && k % 8 == 0 && (reinterpret_cast<uintptr_t>(q) & 7u) == 0 && c_ok) {
-        // grid: at most m / 4 blocks of one wave group (m < 2^31)
-        const bool al8 = kp % 8 == 0 && (reinterpret_cast<uintptr_t>(a_packed) & 7u) == 0;
+// Weight rows a launch of up to 128 codes takes, and code rows.  A launch holds
+// fewer than 2^32 threads (a larger grid wraps without an error, and outputs are
+// left out); the kernels for few codes give a weight row up to 64, the others an
+// output 1/64, so that more codes need no bands of rows with any output that fits
+// the memory.  Bands keep the alignment of what they start at.  The wide kernel
+// only gets whole calls: its output rows have the strides m and n.
+constexpr uint64_t kTernRows = 1ull << 24;
+constexpr uint64_t kTernCols = 1ull << 30;
+constexpr uint64_t kTernOut = 1ull << 39;  // 2 TiB of outputs are refused
+
+// The int8 matmul of one band of weight rows and codes.
+static int ternary_i8_launch(const TernArgs& p, hipStream_t s) {
+    const uint64_t m = p.m, n = p.n, k = p.k, kp = p.kp, nk = n * k;
+    const bool c_ok = (reinterpret_cast<uintptr_t>(p.c) & 3u) == 0;
+    if (k > 0 && small_n_wins(m, n, k) && k % 8 == 0 && (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0 && c_ok) {
+        const bool al8 = kp % 8 == 0 && (reinterpret_cast<uintptr_t>(p.a) & 7u) == 0;
         if (al8) {
             if (n <= 1) launch_gemv<1, true>(p, m, k, s);
             else launch_gemv<2, true>(p, m, k, s);
@@ -3877,11 +3864,11 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         }
         return launch_status();
     }
-    const bool vec = k > 0 && k % 16 == 0 && aligned16(q) && c_ok;
+    const bool vec = k > 0 && k % 16 == 0 && aligned16(p.q) && c_ok;
     if (k >= 16 && c_ok && skinny_wins(m, n, k, vec))
-        return ternary_i8_skinny(p, kp % 16 == 0 && aligned16(a_packed), s);
+        return ternary_i8_skinny(p, kp % 16 == 0 && aligned16(p.a), s);
     const uint64_t wide_tiles = ((m + kWdM - 1) / kWdM) * ((n + kWdN - 1) / kWdN);
-    const bool al = kp % 16 == 0 && aligned16(a_packed);
+    const bool al = kp % 16 == 0 && aligned16(p.a);
     const auto launch_w2 = [&]() -> int {
         const uint64_t tiles = ((m + kWdM - 1) / kWdM) * ((n + kW2N - 1) / kW2N);
         const uint64_t per = (tiles + kXcds - 1) / kXcds;
@@ -3934,11 +3921,50 @@ static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const 
         if (per * kXcds > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
         launch_mfma(al, vec, dim3((uint32_t)(per * kXcds)), s, p);
     } else {
-        const uint64_t blocks = (mn + kTmBlock - 1) / kTmBlock;
-        if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+        const uint64_t blocks = std::min<uint64_t>((m * n + kTmBlock - 1) / kTmBlock, 1ull << 23);
         hipLaunchKernelGGL(ternary_i8_generic_kernel, dim3((uint32_t)blocks), dim3(kTmBlock), 0, s, p);
     }
     return launch_status();
+}
+
+// The int8 matmul with the output in either layout (trans: c[n, m]) and an
+// optional bias per weight row.
+static int ternary_i8_run(const uint8_t* a_packed, const float* a_scales, const int8_t* q, const float* q_scales,
+                          const float* bias, float* c, uint64_t m, uint64_t n, uint64_t k, bool trans,
+                          hipStream_t s) {
+    if (m == 0 || n == 0) return KORE_HIP_OK;
+    if (!c || !a_scales || !q_scales) return KORE_HIP_ERR_NULL_PTR;
+    if (k > 0 && (!a_packed || !q)) return KORE_HIP_ERR_NULL_PTR;
+    // |sum| <= 127 * k must stay exact in int32 and every index in 32 bits.
+    if (m > 0x7fffffffull || n > 0x7fffffffull || k > (1ull << 24)) return KORE_HIP_ERR_OVERFLOW;
+    uint64_t mn, nk;
+    if (!mul_ok(m, n, &mn) || mn >= kTernOut || !mul_ok(n, k, &nk) || nk > kMaxElements)
+        return KORE_HIP_ERR_OVERFLOW;
+    const uint64_t kp = (k + 4) / 5;
+    // c is written while the inputs are read: it must not overlap any of them.
+    {
+        const char* c0 = reinterpret_cast<const char*>(c);
+        const char* c1 = c0 + mn * sizeof(float);
+        const struct { const void* p; uint64_t bytes; } ins[] = {
+            {a_packed, m * kp}, {q, nk}, {a_scales, m * sizeof(float)}, {q_scales, n * sizeof(float)},
+            {bias, bias ? m * sizeof(float) : 0u}};
+        for (const auto& in : ins) {
+            const char* i0 = reinterpret_cast<const char*>(in.p);
+            if (in.p && in.bytes && i0 < c1 && c0 < i0 + in.bytes) return KORE_HIP_ERR_ALIAS;
+        }
+    }
+    const uint64_t rows = n <= (uint64_t)kW2N ? kTernRows : m;
+    for (uint64_t r0 = 0; r0 < m; r0 += rows) {
+        for (uint64_t c0 = 0; c0 < n; c0 += kTernCols) {
+            const TernArgs p{k > 0 ? a_packed + r0 * kp : a_packed, a_scales + r0, k > 0 ? q + c0 * k : q, q_scales + c0,
+                             c + (trans ? c0 * m + r0 : r0 * n + c0), (uint32_t)std::min(rows, m - r0),
+                             (uint32_t)std::min(kTernCols, n - c0), (uint32_t)k, (uint32_t)kp,
+                             bias ? bias + r0 : nullptr, trans ? 1u : 0u, (uint32_t)(trans ? m : n)};
+            const int st = ternary_i8_launch(p, s);
+            if (st != KORE_HIP_OK) return st;
+        }
+    }
+    return KORE_HIP_OK;
 }
 
 extern "C" int kore_hip_ternary_matmul_i8(const uint8_t* a_packed, const float* a_scales, const int8_t* q,

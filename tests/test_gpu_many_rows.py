@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
-from inputs import assert_bitexact, assert_close, normal
+from inputs import assert_bitexact, assert_close, int8_codes, normal, raw_packed
 
 pytestmark = pytest.mark.gpu
 
@@ -149,3 +149,44 @@ def test_rms_norm_backward_many_rows():
     want_dx, want_dg = oracle.rms_norm_backward(ds, xs, g, 1e-5)  # the other rows' dy is 0
     assert_close(rows_of(dx, at), want_dx, rtol=1e-4, atol=1e-5, what="dx")
     assert_close(dgb.to_host(np.float32)[:cols], want_dg, rtol=1e-5, atol=1e-5, what="dgamma")
+
+
+def ternary_rows(m, n, k):
+    """Sampled weight rows with bytes, scales and bias of their own among rows of zero trits, scale 1 and bias 0."""
+    torch.cuda.empty_cache()
+    need = m * ((k + 4) // 5 + 8 + 4 * n)
+    if torch.cuda.mem_get_info()[0] < need + (4 << 30):
+        pytest.skip(f"needs {need >> 30} GiB of device memory")
+    at = sample(m)
+    a = torch.full((m, (k + 4) // 5), 121, dtype=torch.uint8, device="cuda:0")
+    sa, bias = torch.ones(m, device="cuda:0"), torch.zeros(m, device="cuda:0")
+    packed, scales, add = raw_packed(len(at), k, k), normal((len(at),), 11, 1.0, 0.1), normal((len(at),), 12)
+    put(a, at, packed), put(sa.view(m, 1), at, scales[:, None]), put(bias.view(m, 1), at, add[:, None])
+    c = torch.full((m * n,), 7.0, device="cuda:0")
+    bufs = [HipBuffer.from_tensor(t.view(-1)) for t in (a, sa, bias, c)]
+    return at, packed, scales, add, c, bufs
+
+
+def check_ternary(c, m, n, at, want, add, matmul, layer):
+    matmul()
+    assert_bitexact(rows_of(c.view(m, n), at), want, "c[m, n]")
+    if not want.any():
+        assert torch.count_nonzero(c) == 0, "c[m, n] of no columns"
+    c.fill_(7.0)
+    layer()
+    assert_bitexact(rows_of(c.view(n, m).T, at), want + add[:, None], "layer")
+
+
+# Just past 2^32 threads: 16 a weight row for one code, 4 for two with K not a multiple of 8, one an output for K = 0.
+# Then bands of 256 x 128 and 128 x 128 tiles, the last one short, and 256 x 192 and 256 x 256 tiles, which have none.
+@pytest.mark.parametrize("m,n,k", [((1 << 28) + 5, 1, 8), ((1 << 30) + 5, 2, 17), ((1 << 26) + 3, 64, 0),
+                                   ((1 << 24) + 5, 70, 16), ((1 << 24) + 261, 130, 1296), ((1 << 24) + 5, 200, 4176),
+                                   ((1 << 24) + 133, 70, 17)])
+def test_ternary_i8_many_rows(m, n, k):
+    print(f"ternary i8 m={m} n={n} k={k}", flush=True)
+    at, packed, scales, add, c, (ab, sab, bb, cb) = ternary_rows(m, n, k)
+    q, sq = int8_codes(n, k, 13), np.abs(normal((n,), 14, 0.02, 0.005))
+    qb, sqb = HipBuffer.from_host(DEV, q), HipBuffer.from_host(DEV, sq)
+    want = oracle.ternary_matmul_i8(packed, scales, q, sq, len(at), n, k)
+    check_ternary(c, m, n, at, want, add, lambda: rocm.rocm_ternary_matmul_i8(DEV, ab, sab, qb, sqb, m, n, k, out=cb),
+                  lambda: rocm.rocm_bit_linear_i8(DEV, ab, sab, qb, sqb, bb, m, n, k, out=cb))

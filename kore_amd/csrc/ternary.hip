@@ -3980,6 +3980,40 @@ extern "C" int kore_hip_bit_linear_i8(const uint8_t* a_packed, const float* a_sc
                           (hipStream_t)stream);
 }
 
+// The f32-activation matmul of one band of weight rows.
+static int ternary_f32_launch(const TernF32Args& p, bool tm, hipStream_t s) {
+    const uint64_t m = p.m, n = p.n, k = p.k, kp = p.kp;
+    int ct = 64;
+    while (ct > 1 && (uint64_t)(ct / 2) >= n) ct /= 2;  // smallest power of two >= n (<= 64)
+    // Five columns and more: the matrix cores, or the row-broadcast kernel (any
+    // row alignment) in 16-, 32- or 64-column tiles.
+    if (n >= kRowsMinCols) {
+        const F32Form form = tm ? f32_layer_form(m, n, k, kp)
+                                : f32_use_mf4(m, n, k, kp)  ? F32Form::Mf4
+                                : f32_use_mfma(m, n, k) ? F32Form::Mfma
+                                                        : F32Form::Rows;
+        if (form == F32Form::Mf4) return tm ? launch_f32_mf4<true>(m, n, s, p) : launch_f32_mf4<false>(m, n, s, p);
+        if (form == F32Form::Mfma) return tm ? launch_f32_mfma<true>(m, n, s, p) : launch_f32_mfma<false>(m, n, s, p);
+        if (ct <= 16) return tm ? launch_f32_rows<16, true>(m, n, s, p) : launch_f32_rows<16, false>(m, n, s, p);
+        if (ct == 32) return tm ? launch_f32_rows<32, true>(m, n, s, p) : launch_f32_rows<32, false>(m, n, s, p);
+        return tm ? launch_f32_rows<64, true>(m, n, s, p) : launch_f32_rows<64, false>(m, n, s, p);
+    }
+    // One to four columns: the fold-wave kernel; the per-lane kernel for K = 0
+    // and for matrices of fewer than 20 packed bytes (the fold-wave kernel's
+    // 8-byte windows).
+    if (k > 0 && m * kp >= 20) {
+        const dim3 gp((uint32_t)((m + kWave - 1) / kWave));
+        if (n == 1) hipLaunchKernelGGL(ternary_f32_pipe_kernel<1>, gp, dim3((kPfDec + 1) * kWave), 0, s, p);
+        else if (n == 2) hipLaunchKernelGGL(ternary_f32_pipe_kernel<2>, gp, dim3((kPfDec + 2) * kWave), 0, s, p);
+        else hipLaunchKernelGGL(ternary_f32_pipe_kernel<4>, gp, dim3((kPfDec + 4) * kWave), 0, s, p);
+        return launch_status();
+    }
+    const dim3 g((uint32_t)((m + 4 * (kWave / ct) - 1) / (4 * (kWave / ct))));  // 4 waves of 64 / ct rows
+    if (kp % 16 == 0 && aligned16(p.a)) launch_f32_seq<true>(ct, g, s, p);
+    else launch_f32_seq<false>(ct, g, s, p);
+    return launch_status();
+}
+
 // The f32-activation matmul with b either [K, N] or token-major [N, K]
 // (tm), the output in either layout (trans: c[n, m]) and an optional bias.
 static int ternary_f32_run(const uint8_t* a_packed, const float* a_scales, const float* b, const float* bias,
@@ -4010,58 +4044,23 @@ static int ternary_f32_run(const uint8_t* a_packed, const float* a_scales, const
     if (tm && k > (1ull << 23)) return KORE_HIP_ERR_OVERFLOW;
     TernF32Args p{a_packed, a_scales, b, c, (uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)kp,
                   tm ? 1u : n, tm ? k : 1u, bias, trans ? 1u : 0u, m};
-    int ct = 64;
-    while (ct > 1 && (uint64_t)(ct / 2) >= n) ct /= 2;  // smallest power of two >= n (<= 64)
-    // Five columns and more: the row-broadcast kernel (any row alignment) in
-    // 16-, 32- or 64-column tiles, over row ranges of less than 2 GiB of
-    // packed weights each (its buffer offsets are 31-bit).
-    if (n >= kRowsMinCols) {
-        const uint64_t span = kp ? std::min<uint64_t>(m, 0x7fffffffull / kp) : m;  // rows per launch
-        for (uint64_t r0 = 0; r0 < m; r0 += span) {
-            TernF32Args q = p;
-            q.a += r0 * kp;
-            q.sa += r0;
-            q.m = (uint32_t)std::min<uint64_t>(span, m - r0);
-            q.c += trans ? r0 : r0 * n;  // c[n, m]: columns r0 .. of every row, row stride m
-            if (bias) q.bias += r0;
-            const F32Form form = tm ? f32_layer_form(q.m, n, k, kp)
-                                    : f32_use_mf4(q.m, n, k, kp)  ? F32Form::Mf4
-                                    : f32_use_mfma(q.m, n, k) ? F32Form::Mfma
-                                                              : F32Form::Rows;
-            if (form == F32Form::Mf4) {
-                const int st = tm ? launch_f32_mf4<true>(q.m, n, s, q) : launch_f32_mf4<false>(q.m, n, s, q);
-                if (st != KORE_HIP_OK) return st;
-                continue;
-            }
-            if (form == F32Form::Mfma) {
-                const int st = tm ? launch_f32_mfma<true>(q.m, n, s, q) : launch_f32_mfma<false>(q.m, n, s, q);
-                if (st != KORE_HIP_OK) return st;
-                continue;
-            }
-            const int st = tm ? (ct <= 16 ? launch_f32_rows<16, true>(q.m, n, s, q)
-                                 : ct == 32 ? launch_f32_rows<32, true>(q.m, n, s, q)
-                                            : launch_f32_rows<64, true>(q.m, n, s, q))
-                              : (ct <= 16 ? launch_f32_rows<16, false>(q.m, n, s, q)
-                                 : ct == 32 ? launch_f32_rows<32, false>(q.m, n, s, q)
-                                            : launch_f32_rows<64, false>(q.m, n, s, q));
-            if (st != KORE_HIP_OK) return st;
-        }
-        return KORE_HIP_OK;
+    // Bands of at most kTernRows rows (see there; a thread an output for K = 0),
+    // and of less than 2 GiB of packed weights for the kernels of five columns
+    // and more (their buffer offsets are 31-bit).
+    uint64_t span = std::min(m, kTernRows);
+    if (kp && n >= kRowsMinCols) span = std::min<uint64_t>(span, 0x7fffffffull / kp);
+    if (!kp) span = std::min<uint64_t>(span, std::max<uint64_t>((1ull << 31) / n, 1));
+    for (uint64_t r0 = 0; r0 < m; r0 += span) {
+        TernF32Args q = p;
+        if (k > 0) q.a += r0 * kp;
+        q.sa += r0;
+        q.m = (uint32_t)std::min<uint64_t>(span, m - r0);
+        q.c += trans ? r0 : r0 * n;  // c[n, m]: columns r0 .. of every row, row stride m
+        if (bias) q.bias += r0;
+        const int st = ternary_f32_launch(q, tm, s);
+        if (st != KORE_HIP_OK) return st;
     }
-    // One to four columns: the fold-wave kernel; the per-lane kernel for K = 0
-    // and for matrices of fewer than 20 packed bytes (the fold-wave kernel's
-    // 8-byte windows).
-    if (k > 0 && mkp >= 20) {
-        const dim3 gp((uint32_t)((m + kWave - 1) / kWave));
-        if (n == 1) hipLaunchKernelGGL(ternary_f32_pipe_kernel<1>, gp, dim3((kPfDec + 1) * kWave), 0, s, p);
-        else if (n == 2) hipLaunchKernelGGL(ternary_f32_pipe_kernel<2>, gp, dim3((kPfDec + 2) * kWave), 0, s, p);
-        else hipLaunchKernelGGL(ternary_f32_pipe_kernel<4>, gp, dim3((kPfDec + 4) * kWave), 0, s, p);
-        return launch_status();
-    }
-    const dim3 g((uint32_t)((m + 4 * (kWave / ct) - 1) / (4 * (kWave / ct))));  // 4 waves of 64 / ct rows
-    if (kp % 16 == 0 && aligned16(a_packed)) launch_f32_seq<true>(ct, g, s, p);
-    else launch_f32_seq<false>(ct, g, s, p);
-    return launch_status();
+    return KORE_HIP_OK;
 }
 
 extern "C" int kore_hip_ternary_matmul_f32(const uint8_t* a_packed, const float* a_scales, const float* b, float* c,

@@ -190,3 +190,15 @@ def test_ternary_i8_many_rows(m, n, k):
     want = oracle.ternary_matmul_i8(packed, scales, q, sq, len(at), n, k)
     check_ternary(c, m, n, at, want, add, lambda: rocm.rocm_ternary_matmul_i8(DEV, ab, sab, qb, sqb, m, n, k, out=cb),
                   lambda: rocm.rocm_bit_linear_i8(DEV, ab, sab, qb, sqb, bb, m, n, k, out=cb))
+
+
+# Just past 2^32 threads: 7 a weight row for one column, 8 for five with K = 0; then bands of the 16 x 16 kernel.
+@pytest.mark.parametrize("m,n,k", [((1 << 30) + 5, 1, 7), ((1 << 29) + 5, 5, 0), ((1 << 24) + 67, 20, 6)])
+def test_ternary_f32_many_rows(m, n, k):
+    print(f"ternary f32 m={m} n={n} k={k}", flush=True)
+    at, packed, scales, add, c, (ab, sab, bb, cb) = ternary_rows(m, n, k)
+    b = normal((k, n), 15)
+    b0, b1 = HipBuffer.from_host(DEV, b), HipBuffer.from_host(DEV, np.ascontiguousarray(b.T))
+    want = oracle.ternary_matmul(packed, scales, b, len(at), n, k)
+    check_ternary(c, m, n, at, want, add, lambda: rocm.rocm_ternary_matmul_f32(DEV, ab, sab, b0, m, n, k, out=cb),
+                  lambda: rocm.rocm_bit_linear_f32(DEV, ab, sab, b1, bb, m, n, k, out=cb))

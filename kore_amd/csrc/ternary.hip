@@ -4092,15 +4092,24 @@ extern "C" int kore_hip_pack_weights_ternary(const float* w, uint64_t m, uint64_
             if (w && mk && o.p && o.bytes && o0 < w1 && w0 < o0 + o.bytes) return KORE_HIP_ERR_ALIAS;
         }
     }
-    const uint64_t blocks = (m + kPackWaves - 1) / kPackWaves;
-    if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-    const dim3 g((uint32_t)blocks), blk(kPackWaves * kWave);
-    hipStream_t s = (hipStream_t)stream;
     const uint64_t slices = ((k + 19) / 20 + kWave - 1) / kWave;  // 64-chunk slices of 20 floats per row
+    if ((m + kPackWaves - 1) / kPackWaves > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+    // a workgroup a row: m < 2^31 blocks, as ever
+    if (m > 0x7fffffffull && k % 4 == 0 && aligned16(w) && slices > 2 && slices <= 8 * kPackWaves)
+        return KORE_HIP_ERR_OVERFLOW;
+    // A launch holds fewer than 2^32 threads (a larger grid wraps without an
+    // error, and rows are left out), at up to 256 threads a row.
+    constexpr uint64_t kBand = 1ull << 23;
+    for (; m > kBand; w += kBand * k, packed += kBand * kp, scales += kBand, m -= kBand) {
+        const int st = kore_hip_pack_weights_ternary(w, kBand, k, threshold, packed, scales, stream);
+        if (st != KORE_HIP_OK) return st;
+    }
+    const dim3 g((uint32_t)((m + kPackWaves - 1) / kPackWaves)), blk(kPackWaves * kWave);
+    hipStream_t s = (hipStream_t)stream;
     // Two slices: a workgroup of two waves per row, one slice each (measured
     // 6912 x 2560 15.65 -> 15.17 us against one wave per row); one slice: a
     // wave per row.
-    if (k > 0 && k % 4 == 0 && aligned16(w) && slices == 2 && m <= 0x7fffffffull) {
+    if (k > 0 && k % 4 == 0 && aligned16(w) && slices == 2) {
         hipLaunchKernelGGL((ternary_pack_vec_kernel<1, true, 2>), dim3((uint32_t)m), dim3(2 * kWave), 0, s, w, m,
                            (uint32_t)k, threshold, packed, scales);
         return launch_status();
@@ -4109,8 +4118,7 @@ extern "C" int kore_hip_pack_weights_ternary(const float* w, uint64_t m, uint64_
         if (slices <= 1) hipLaunchKernelGGL((ternary_pack_vec_kernel<1, false>), g, blk, 0, s, w, m, (uint32_t)k, threshold, packed, scales);
         else hipLaunchKernelGGL((ternary_pack_vec_kernel<2, false>), g, blk, 0, s, w, m, (uint32_t)k, threshold, packed, scales);
     } else if (k > 0 && k % 4 == 0 && aligned16(w) && slices <= 8 * kPackWaves) {
-        // long rows: a workgroup per row (m < 2^31 blocks)
-        if (m > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+        // long rows: a workgroup per row
         const dim3 gr((uint32_t)m);
         const uint64_t per_wave = (slices + kPackWaves - 1) / kPackWaves;
         if (per_wave <= 1) hipLaunchKernelGGL((ternary_pack_vec_kernel<1, true>), gr, blk, 0, s, w, m, (uint32_t)k, threshold, packed, scales);

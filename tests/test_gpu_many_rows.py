@@ -202,3 +202,17 @@ def test_ternary_f32_many_rows(m, n, k):
     want = oracle.ternary_matmul(packed, scales, b, len(at), n, k)
     check_ternary(c, m, n, at, want, add, lambda: rocm.rocm_ternary_matmul_f32(DEV, ab, sab, b0, m, n, k, out=cb),
                   lambda: rocm.rocm_bit_linear_f32(DEV, ab, sab, b1, bb, m, n, k, out=cb))
+
+
+# 64 threads a row of up to 1280 columns, whole float4 or not, and 256 of more than 2560.
+@pytest.mark.parametrize("m,k", [((1 << 26) + 5, 4), ((1 << 26) + 5, 3), ((1 << 24) + 5, 2564)])
+def test_pack_weights_many_rows(m, k):
+    print(f"pack m={m} k={k}", flush=True)
+    kp = (k + 4) // 5
+    t, at = big(m, k + (kp + 7) // 4), sample(m)
+    w = t.view(-1)[:m * k].view(m, k).zero_()
+    x = fill(w, at, 16)
+    p, sc = rocm.rocm_pack_weights_ternary(DEV, HipBuffer.from_tensor(w), m, k, 0.5)
+    want_p, want_s = oracle.pack_weights_ternary(x, 0.5)
+    assert_bitexact(rows_of(p.tensor(torch.uint8)[:m * kp].view(m, kp), at), want_p, "packed")
+    assert_bitexact(rows_of(sc.tensor(torch.float32)[:m].view(m, 1), at)[:, 0], want_s, "scales")

@@ -367,11 +367,11 @@ static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols) {
 // Rows of the generic path where the workspace plan does not run: a workgroup a
 // row and a thread a dgamma column, against the long path's two launches that
 // few rows leave waiting on 16 waves' barriers (us, generic against long path):
-// 16 x 257 5.9 against 9.2, 48 9.9 against 9.4; 64 x 1001 12.3 against 13.8, 80
-// 14.3 against 13.8; 32 x 3001 10.4 against 11.0, 48 12.4 against 11.1; 8 x 4100
+// 16 x 257 5.9 against 9.2, 48 9.9 against 9.4; 40 x 700 9.0 against 9.2, 48 x 1021
+// 10.6 against 10.0; 32 x 3001 10.4 against 11.0, 48 12.4 against 11.1; 8 x 4100
 // 8.5 against 8.9, 16 9.5 against 9.1; 2 x 7000 10.6 against 9.7.
 static uint64_t bwd_generic_rows(uint64_t cols) {
-    return cols <= 512 ? 44 : cols <= 1024 ? 72 : cols <= 4096 ? 36 : cols <= 5120 ? 8 : 1;
+    return cols <= 1024 ? 44 : cols <= 4096 ? 36 : cols <= 5120 ? 8 : 1;
 }
 
 template <int NCHW, int S>
@@ -386,7 +386,10 @@ static void launch_rows(const BwArgs& a, hipStream_t s) {
 // 4096 x 8192 85.5 us (4.7 TB/s; one workgroup per row and one thread per
 // dgamma column before: 1740), 4096 x 8191 108 (1753), 8000 x 2049 57 (2770),
 // 2048 x 14336 82 (966); with 512 workgroups of 8 waves 90, 110, 62 and 96,
-// 256 of 8 86, 117, 67 and 82, 128 of 16 110, 134, 76 and 96.  Rows of whole
+// 256 of 8 86, 117, 67 and 82, 128 of 16 110, 134, 76 and 96.  Ragged rows of
+// 513-1024 columns take two waves of 2 float4, as one of 4 has more registers in
+// use than four waves a SIMD leave it and spills (100 x 1001 13.9 -> 10.0, 4096 x
+// 1021 28.4 -> 24.0, 16384 x 1001 58.4 -> 54.6, 16384 x 515 44.4 -> 39.4).  Whole
 // float4 up to 4096 columns keep the workspace plan (8192 x 4096 74 us, 5.4
 // TB/s: no row is done twice).
 constexpr int kBwLongWaves = 16;
@@ -515,7 +518,7 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         // partial rows wait in dx's last P rows until the second launch has
         // reduced them and computes those rows' dx; 2 P <= rows, the inv and
         // coeff it needs being the workspace's first 2 P floats.
-        const uint64_t slots = (uint32_t)kBwLongWaves / split;
+        const uint64_t slots = (uint32_t)kBwLongWaves / (cols4 > 128 && cols4 <= 256 ? 2u : split);
         uint64_t rpb = (rows + kBwLongBlocks - 1) / kBwLongBlocks;
         if (rpb < 2) rpb = 2;
         rpb = (rpb + slots - 1) / slots * slots;
@@ -527,7 +530,7 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         a.part = grad_x + a.dx_rows * cols;
         if (cols4 <= 64) launch_long<1, 1>(a, !aligned, s);
         else if (cols4 <= 128) launch_long<2, 1>(a, !aligned, s);
-        else if (cols4 <= 256) launch_long<4, 1>(a, !aligned, s);
+        else if (cols4 <= 256) launch_long<2, 2>(a, !aligned, s);
         else if (cols4 <= 512) launch_long<4, 2>(a, !aligned, s);
         else if (cols4 <= 1024) launch_long<4, 4>(a, !aligned, s);
         else if (cols4 <= 1536) launch_long<3, 8>(a, !aligned, s);

@@ -42,8 +42,8 @@ def inside(t, start: int, n: int) -> np.ndarray:
 # row more than the generic path takes and odd numbers of rows; 16385 is the generic path's, as are the first rows of each
 # range up to 5120 columns.  Rows: fewer than, and not a multiple of, a workgroup's.
 @pytest.mark.parametrize("rows,cols,offset", [
-    (1, 1, 0), (3, 5, 1), (45, 5, 1), (9, 255, 2), (44, 255, 2), (45, 255, 2), (601, 258, 3), (7, 513, 0), (73, 513, 0),
-    (72, 1021, 1), (75, 1021, 1), (513, 1030, 2), (36, 2049, 0), (37, 2049, 0), (6, 3071, 3), (39, 3071, 3),
+    (1, 1, 0), (3, 5, 1), (45, 5, 1), (9, 255, 2), (44, 255, 2), (45, 255, 2), (601, 258, 3), (7, 513, 0), (44, 513, 0), (45, 513, 0), (73, 513, 0),
+    (44, 1024, 1), (45, 1024, 1), (45, 769, 3), (46, 767, 2), (72, 1021, 1), (75, 1021, 1), (513, 1030, 2), (36, 2049, 0), (37, 2049, 0), (6, 3071, 3), (39, 3071, 3),
     (1100, 4095, 1), (4, 4096, 1), (37, 4096, 1), (3, 4097, 0), (9, 4097, 0), (8, 4100, 0), (9, 4100, 0), (8, 5120, 1),
     (2, 5121, 0), (515, 6143, 2), (2, 6144, 0), (3, 6145, 1), (520, 8192, 0), (2, 8191, 0), (3, 8193, 3), (2, 12288, 0),
     (2, 12291, 1), (259, 16384, 0), (2, 16383, 2), (2, 16385, 0)])

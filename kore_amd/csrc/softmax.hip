@@ -257,10 +257,11 @@ __global__ __launch_bounds__(BS, NCH < 16 ? 1 : K == SmKind::Bwd ? 3 : 4) void s
 // registers that the first chunks' loads then take over.
 // Bound by HBM: 8 bytes a float.  2048 x 128256: 767 us in the loop kernel's
 // three passes, 382 here (5.5 TB/s); x 50257 421 -> 157, x 20000 98 -> 56; 64 x
-// 128256 103 -> 19.  Ragged 16368 x 1023 in the wave kernel 60.5 -> 25.8 us,
-// its backward 49.4 -> 38.4 (whole float4, 16384 x 1024: 22.7 and 31.3).
+// 128256 103 -> 19.
 constexpr int kLongThreads = 1024;
-constexpr int kLongRegs = 24;   // float4 a thread: 96 of the 128 VGPRs that 16 waves leave
+// float4 a thread: 96 of the 128 VGPRs that 16 waves leave (the causal kernels and
+// the ragged cross-entropy one spill 4-7 VGPRs besides)
+constexpr int kLongRegs = 24;
 constexpr int kLongLds = 9;     // float4 a thread: 144 of the 160 KB
 constexpr uint64_t kLongCols = 4ull * kLongThreads * (kLongRegs + kLongLds);
 
@@ -574,8 +575,12 @@ static void softmax_dispatch(const SmArgs& a, hipStream_t s) {
     }
     else if (cols4 <= 1024) {
         switch (mid_form<K, Ragged>(a.rows, cols4)) {
-        case MidForm::Wave: return launch_wave<K, 16, Ragged>(a, s);
-        case MidForm::Group256: return launch_block<K, 4, Ragged, 256>(a, s);
+        case MidForm::Wave:  // not for ragged backward rows
+            if constexpr (!kBwd || !Ragged) return launch_wave<K, 16, Ragged>(a, s);
+            [[fallthrough]];
+        case MidForm::Group256:  // not for whole ones
+            if constexpr (!kBwd || Ragged) return launch_block<K, 4, Ragged, 256>(a, s);
+            [[fallthrough]];
         case MidForm::Group512: return launch_block<K, 2, Ragged, 512>(a, s);
         }
     }

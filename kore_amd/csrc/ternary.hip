@@ -3439,7 +3439,8 @@ static void launch_mfma(bool aligned_a, bool aligned_b, dim3 grid, hipStream_t s
 // 256 (m) x 128 (n) output tile, wave w its weight rows [64 w, 64 w + 64)
 // against the tile's 128 code rows: 2 x 4 MFMA tiles of 32 x 32 (128 int32
 // accumulators per lane), 128 VGPRs + 128 AGPRs, so that each SIMD runs one
-// wave of each of two workgroups.  A v_mfma_i32_32x32x32_i8 issues every 32
+// wave of each of two workgroups (with unaligned packed rows and a transposed
+// output four of them are spilled).  A v_mfma_i32_32x32x32_i8 issues every 32
 // cycles, but the vector and LDS instructions a wave issues between its own
 // MFMAs (the trit decode, operand reads, code loads) delay its next one
 // (measured: one wave per SIMD with three VALU and one LDS read per MFMA
@@ -3880,12 +3881,12 @@ static int ternary_i8_launch(const TernArgs& p, hipStream_t s) {
     };
     // Past the skinny kernel's range and below the wide one's, and for one tile
     // column whatever the rows (128256 x 100 x 2560 48.8 us against 78.9 in 256 x
-    // 192 tiles, x 6912 120 against 173): 256 x 128 tiles, up to about one a CU, their K loop two to three times the 128 x 128 kernel's
-    // rate (measured, graph replays: 6912 x 800 x 2560 39.4 -> 30.2 us, 2560 x
-    // 1600 x 6912 87.3 -> 70.4, 5376 x 1000 x 896 25.3 -> 19.1, 4096 x 1200 x
-    // 4096 57.8 -> 45.5, 2048 x 3000 x 2048 37.7 -> 28.3).
-    // (up to 128 rows fill half of such a tile at most: 64 x 33000 x 2560 38 us in
-    // 128 x 128 tiles, 41 here)
+    // 192 tiles, x 6912 120 against 173): 256 x 128 tiles, their K loop two to
+    // three times the 128 x 128 kernel's rate (measured, graph replays: 6912 x 800
+    // x 2560 39.4 -> 30.2 us, 2560 x 1600 x 6912 87.3 -> 70.4, 5376 x 1000 x 896
+    // 25.3 -> 19.1, 4096 x 1200 x 4096 57.8 -> 45.5, 2048 x 3000 x 2048 37.7 ->
+    // 28.3).  Not for up to 128 rows, which fill half of such a tile at most (64 x
+    // 33000 x 2560 38 us in 128 x 128 tiles, 41 here).
     if (vec && nk < (1ull << 31) && m > (uint64_t)kTmM && (wide_tiles < kWdMinTiles || n <= (uint64_t)kW2N))
         return launch_w2();
     if (vec && wide_tiles >= kWdMinTiles && nk < (1ull << 31)) {

@@ -185,8 +185,14 @@ void rms_bwd_rows_kernel(BwArgs a) {
             dv[k] = dn[k];
         }
     }
-    // Row slots' partials added in j order through LDS (gamma is done with),
-    // then one partial row.
+    // One partial row: a single row slot's as it is, several added in j order
+    // through LDS (gamma is done with).
+    float* prow = a.part + (uint64_t)blockIdx.x * cols;
+    if (kSlots == 1) {
+#pragma unroll
+        for (int k = 0; k < NCHW; ++k) st_row4<Ragged, false>(prow, col4(k), cols, acc[k]);
+        return;
+    }
     __syncthreads();
 #pragma unroll 1
     for (int jj = 0; jj < kSlots; ++jj) {
@@ -199,7 +205,6 @@ void rms_bwd_rows_kernel(BwArgs a) {
         }
         __syncthreads();
     }
-    float* prow = a.part + (uint64_t)blockIdx.x * cols;
     for (uint32_t f = threadIdx.x; f < cols4; f += kThreads) st_row4<Ragged, false>(prow, f, cols, gam[f]);
 }
 
@@ -223,9 +228,12 @@ __device__ __forceinline__ void reduce_partials(const BwArgs& a, int c, int slot
 #pragma unroll
             for (int u = 0; u < kRedBatch; ++u) {
                 const uint64_t p = p0 + (uint64_t)u * kRedSlots;
-                v[u] = p < a.partials
-                           ? ld_row4<Ragged, false>(a.part + p * a.cols, (uint32_t)col, (uint32_t)a.cols)
-                           : zero;
+                if (Ragged)
+                    v[u] = p < a.partials
+                               ? ld_row4<true, false>(a.part + p * a.cols, (uint32_t)col, (uint32_t)a.cols)
+                               : zero;
+                else
+                    v[u] = p < a.partials ? reinterpret_cast<const f32x4*>(a.part)[p * cols4 + col] : zero;
             }
 #pragma unroll
             for (int u = 0; u < kRedBatch; ++u) {

@@ -691,8 +691,8 @@ __global__ __launch_bounds__(kWave * WPB) void row_norm_kernel(NormArgs args) {
     }
 }
 
-// Scalar path for rows of more than 16384 columns: one thread per row, the
-// reference loop verbatim.
+// One thread per row, the reference loop verbatim: rows of more than 16384
+// columns, and short ones (see thread_a_row).
 template <NormOut Out>
 __global__ __launch_bounds__(64) void row_norm_scalar_kernel(NormArgs args) {
     const uint64_t row = (uint64_t)blockIdx.x * 64 + threadIdx.x;
@@ -799,6 +799,26 @@ static int launch_sl4(NormArgs a, uint32_t nch, RowForm form, hipStream_t s) {
 // four rows per wave at lower occupancy, and than splitting a row over two
 // waves that meet through block barriers (4096 x 2560 pre-quant 14.4 vs
 // 16.4 us).
+// Short rows, of which a wave a row leaves most lanes idle.  A thread a row against
+// a wave a row, graph replays, us: RMSNorm 1000000 x 1 5.8 against 312, 200000 x 3
+// 3.5 against 67, x 8 10.4 against 74, x 16 46 against 74; 64 x 4 2.35 against 3.15,
+// 1000 x 7 3.2 against 3.6.  From 8 columns (pre-quant 4) the rows have to fill the
+// chip, and the row counts where the two meet lie on a line (ragged 3500 x 10 4.0
+// against 4.5, but 1000 x 8 3.8 against 3.3; 10000 x 17 6.0 against 7.4, 20000 x 28 9.5
+// against 11.7, but 16000 x 32 11.4 against 9.8; whole rows, which a wave reads with
+// fewer instructions, later: 3500 x 8 3.9 against 3.7).  Past 20 columns they have to
+// stay in the caches, as a wave's lanes read 64 rows at a time (200000 x 24 102
+// against 76, pre-quant 60 against 98; 250000 x 17 63 against 103); whole rows past
+// 16 never gain (120000 x 32 79 against 48).
+template <NormOut Out>
+static bool thread_a_row(uint64_t rows, uint64_t cols, bool whole) {
+    constexpr bool kCodes = Out == NormOut::I8;
+    if (cols <= (kCodes ? 3u : 7u)) return true;
+    if (rows < 512 || cols > (whole ? 16u : 32u)) return false;
+    if (whole ? rows + 3600 < 1000 * cols : rows + 1600 < 600 * cols) return false;
+    return cols <= 20 || rows * cols <= (kCodes ? 1ull << 23 : 1ull << 22);
+}
+
 template <NormOut Out>
 static int norm_launch(NormArgs a, hipStream_t s) {
     if (a.rows == 0) return KORE_HIP_OK;
@@ -810,21 +830,18 @@ static int norm_launch(NormArgs a, hipStream_t s) {
     uint64_t elems;
     if (!mul_ok(a.rows, a.cols, &elems) || elems > kMaxElements) return KORE_HIP_ERR_OVERFLOW;
     const uint32_t nch = (uint32_t)(((uint64_t)a.cols + 255) / 256);
-    const bool vec = nch <= 64;
     bool whole = a.cols % 4 == 0 && aligned16(a.x) && aligned16(a.w);
     if (Out == NormOut::F32) whole = whole && aligned16(a.y);
     else if (Out == NormOut::SiluGate) whole = whole && aligned16(a.y) && aligned16(a.z);
     else whole = whole && (reinterpret_cast<uintptr_t>(a.q) & 3u) == 0;
-    if (!vec) {
-        uint64_t blocks = (a.rows + 63) / 64;
-        if (blocks > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
-        hipLaunchKernelGGL(row_norm_scalar_kernel<Out>, dim3((uint32_t)blocks), dim3(64), 0, s, a);
-        return launch_status();
-    }
-    if (whole && a.rows > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+    if (whole && nch <= 64 && a.rows > 0x7fffffffull) return KORE_HIP_ERR_OVERFLOW;
+    const bool scalar = nch > 64 || thread_a_row<Out>(a.rows, a.cols, whole);
+    const uint64_t band = scalar ? 1ull << 30 : kLaunchRows;
     for (uint64_t left = a.rows; left > 0;) {
-        a.rows = left < kLaunchRows ? left : kLaunchRows;
-        const int st = launch_sl4<Out>(a, nch, whole ? RowForm::Part : RowForm::Ragged, s);
+        a.rows = left < band ? left : band;
+        if (scalar)
+            hipLaunchKernelGGL(row_norm_scalar_kernel<Out>, dim3((uint32_t)((a.rows + 63) / 64)), dim3(64), 0, s, a);
+        const int st = scalar ? launch_status() : launch_sl4<Out>(a, nch, whole ? RowForm::Part : RowForm::Ragged, s);
         if (st != KORE_HIP_OK) return st;
         left -= a.rows;
         const uint64_t n = a.rows * a.cols;

@@ -75,10 +75,9 @@ def test_softmax_backward_many_rows(rows, cols):
     rocm.rocm_softmax_backward_f32(DEV, b, b, rows, cols, b)
     assert_close(rows_of(t, at), oracle.softmax_backward(y, y), rtol=1e-5 + cols * U32, atol=1e-6, what="backward")
 
-# Just past 2^32 threads at a wave a row; odd bands start a ragged row anywhere.
-@pytest.mark.parametrize("cols", [1, 3])
-def test_norm_family_many_rows(cols):
-    rows = (1 << 26) + 3
+# Just past 2^32 threads at a wave a row, and at a thread a row; odd bands start a ragged row anywhere.
+@pytest.mark.parametrize("rows,cols", [((1 << 26) + 3, 17), ((1 << 26) + 3, 3), ((1 << 32) + 3, 1)])
+def test_norm_family_many_rows(rows, cols):
     print(f"norm family rows={rows} cols={cols}", flush=True)
     t, at = big(rows, cols), sample(rows)
     w = normal((cols,), 4, 1.0, 0.02)

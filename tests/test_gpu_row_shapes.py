@@ -40,12 +40,13 @@ def inside(t, start: int, n: int) -> np.ndarray:
 
 # One float4 per lane and wave more or less around 256, 512, 1024, 4096, 6144, 8192, 12288 and 16384 columns, each with a
 # row more than the generic path takes and odd numbers of rows; 16385 is the generic path's, as are the first rows of each
-# range up to 5120 columns.  Rows: fewer than, and not a multiple of, a workgroup's.
+# range (a few of any length, more odd than even ones).  Rows: fewer than, and not a multiple of, a workgroup's.
 @pytest.mark.parametrize("rows,cols,offset", [
     (1, 1, 0), (3, 5, 1), (45, 5, 1), (9, 255, 2), (44, 255, 2), (45, 255, 2), (601, 258, 3), (7, 513, 0), (44, 513, 0), (45, 513, 0), (73, 513, 0),
     (44, 1024, 1), (45, 1024, 1), (45, 769, 3), (46, 767, 2), (72, 1021, 1), (75, 1021, 1), (513, 1030, 2), (36, 2049, 0), (37, 2049, 0), (6, 3071, 3), (39, 3071, 3),
     (1100, 4095, 1), (4, 4096, 1), (37, 4096, 1), (3, 4097, 0), (9, 4097, 0), (8, 4100, 0), (9, 4100, 0), (8, 5120, 1),
-    (2, 5121, 0), (515, 6143, 2), (2, 6144, 0), (3, 6145, 1), (520, 8192, 0), (2, 8191, 0), (3, 8193, 3), (2, 12288, 0),
+    (2, 5121, 0), (18, 4100, 1), (19, 4100, 1), (10, 5120, 0), (11, 5120, 0), (9, 6144, 0), (11, 6144, 0), (18, 8189, 2),
+    (19, 8189, 2), (20, 8192, 1), (4, 8196, 0), (9, 12285, 3), (11, 12285, 3), (515, 6143, 2), (2, 6144, 0), (3, 6145, 1), (520, 8192, 0), (2, 8191, 0), (3, 8193, 3), (2, 12288, 0),
     (2, 12291, 1), (259, 16384, 0), (2, 16383, 2), (2, 16385, 0)])
 def test_rms_norm_backward_long_and_ragged(rows, cols, offset):
     print(f"rms_norm_backward rows={rows} cols={cols} offset={offset}", flush=True)
@@ -174,8 +175,11 @@ def test_softmax_long_and_ragged_nonfinite_rows(cols):
 
 # ------------------------------------------------- RMSNorm, pre-quant, gate
 # Bit-exact for every plan: one wave a row to 3072 columns, two to 4096, four to 16384, each at its first and last
-# length, whole, partly filled (a wave without any column) and ragged; 16385 is the scalar kernel's.
-NORM_LENGTHS = [(3, 1, 1), (5, 6, 3), (300, 255, 2), (7, 1021, 1), (9, 1537, 0), (260, 2561, 3), (300, 3071, 0),
+# length, whole, partly filled (a wave without any column) and ragged; 16385 is the scalar kernel's, as are the shortest rows and
+# many of up to 32 columns.
+NORM_LENGTHS = [(3, 1, 1), (5, 6, 3), (65, 3, 1), (70, 4, 0), (66, 7, 2), (511, 4, 0), (512, 4, 0), (4400, 8, 0),
+                (4399, 8, 0), (3200, 8, 1), (3199, 9, 1), (12400, 16, 0), (12399, 16, 0), (8600, 17, 3), (17600, 32, 1),
+                (17600, 32, 0), (20000, 33, 2), (300, 255, 2), (7, 1021, 1), (9, 1537, 0), (260, 2561, 3), (300, 3071, 0),
                 (5, 3072, 0), (300, 3073, 0), (3, 3076, 0), (2, 4095, 2), (3, 4096, 1), (300, 4097, 0), (2, 4100, 0), (5, 5119, 1), (270, 5120, 0), (3, 6144, 0),
                 (300, 6912, 0), (3, 6915, 2), (2, 7168, 0), (4, 7172, 0), (300, 8192, 0), (3, 8191, 3), (2, 8193, 0),
                 (2, 9000, 0), (3, 10240, 0), (2, 12285, 1), (3, 12288, 0), (259, 14336, 0), (2, 16383, 2),

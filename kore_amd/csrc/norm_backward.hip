@@ -375,11 +375,18 @@ static uint64_t bwd_ws_floats(uint64_t rows, uint64_t cols) {
 // Rows of the generic path where the workspace plan does not run: a workgroup a
 // row and a thread a dgamma column, against the long path's two launches that
 // few rows leave waiting on 16 waves' barriers (us, generic against long path):
-// 16 x 257 5.9 against 9.2, 48 9.9 against 9.4; 40 x 700 9.0 against 9.2, 48 x 1021
-// 10.6 against 10.0; 32 x 3001 10.4 against 11.0, 48 12.4 against 11.1; 8 x 4100
-// 8.5 against 8.9, 16 9.5 against 9.1; 2 x 7000 10.6 against 9.7.
-static uint64_t bwd_generic_rows(uint64_t cols) {
-    return cols <= 1024 ? 44 : cols <= 4096 ? 36 : cols <= 5120 ? 8 : 1;
+// 40 x 700 9.4 against 9.9, 48 x 1021 10.6 against 10.0; 40 x 4095 12.9 against
+// 12.9, 49 x 2049 12.3 against 11.5; ragged 16 x 6912 12.3 against 12.9, 24 x 6144
+// 12.6 against 10.5, 20 x 8192 14.2 against 13.8; whole 8 x 5120 9.4 against 9.9, 16
+// 10.4 against 10.1, 2 x 8192 11.8 against 11.0; ragged 2 x 12001 15.8 against 14.2.
+// An odd row more than the partial rows leave room for takes every workgroup
+// another turn: whole 3 x 6144 9.9 against 10.7, 15 11.3 against 10.6, 9 x 8192 12.5
+// against 12.8; ragged 5 x 12000 16.0 against 16.4, 15 x 12001 17.4 against 16.3.
+static uint64_t bwd_generic_rows(uint64_t rows, uint64_t cols, bool aligned) {
+    if (cols <= 4096) return 44;
+    if (!aligned && cols <= 8192) return 18;
+    if (cols <= 5120) return 10;
+    return rows % 2 == 1 && cols <= (aligned ? 8192u : 12288u) ? 9 : 1;
 }
 
 template <int NCHW, int S>
@@ -521,7 +528,7 @@ static int rms_bwd_run(const float* grad_out, const float* x, const float* gamma
         else launch_rows<4, 4>(a, s);
         hipLaunchKernelGGL(rms_bwd_reduce_kernel, dim3((uint32_t)((cols4 + kRedCols - 1) / kRedCols)),
                            dim3(kRedCols * kRedSlots), 0, s, a);
-    } else if (cols <= 16384 && rows > bwd_generic_rows(cols)) {
+    } else if (cols <= 16384 && rows > bwd_generic_rows(rows, cols, aligned)) {
         // The workspace of these shapes holds one float per row, so the P
         // partial rows wait in dx's last P rows until the second launch has
         // reduced them and computes those rows' dx; 2 P <= rows, the inv and

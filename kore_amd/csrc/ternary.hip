@@ -3698,7 +3698,6 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) sam[i] = p.sa[min(mw + 32 * i + r, p.m - 1u)];
         const uint32_t mc = mw + 4 * (lane & 15);
-        const bool vec_out = (p.ld & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
         f32x4 bias4 = {0.f, 0.f, 0.f, 0.f};
         if (p.bias) {
 #pragma unroll
@@ -3723,8 +3722,8 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
                 v = v * sqn;
                 if (p.bias) v = v + bias4;
                 float* crow = p.c + (uint64_t)n * p.ld;
-                if (vec_out && mc + 3 < p.m) {
-                    __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(crow + mc));
+                if (mc + 3 < p.m) {
+                    __builtin_nontemporal_store((f32x4_a4)v, reinterpret_cast<f32x4_a4*>(crow + mc));
                 } else {
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
@@ -3739,7 +3738,6 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) sqn[j] = p.sq[min(n0 + 32 * j + r, p.n - 1u)];
     float* slab = reinterpret_cast<float*>(wlds) + wave * 32 * kW2EpPitch;
-    const bool vec_out = (p.ld & 3u) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15u) == 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const uint32_t mb = m0 + 64 * wave + 32 * i;
@@ -3760,8 +3758,8 @@ __global__ __launch_bounds__(256, 2) void ternary_i8_w2_kernel(TernArgs p) {
             if (p.bias) v = v + p.bias[m];
             float* crow = p.c + (uint64_t)m * p.ld;
             const uint32_t nc = n0 + col;
-            if (vec_out && nc + 3 < p.n) {
-                __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(crow + nc));
+            if (nc + 3 < p.n) {
+                __builtin_nontemporal_store((f32x4_a4)v, reinterpret_cast<f32x4_a4*>(crow + nc));
             } else {
 #pragma unroll
                 for (int u = 0; u < 4; ++u)

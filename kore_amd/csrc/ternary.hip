@@ -1042,9 +1042,9 @@ static int launch_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
     return launch_status();
 }
 
-// Small-n path (one or two code rows, k % 8 == 0, 8-byte aligned codes): a group of waves
+// Small-n path (one code row, few more at times, k % 8 == 0, 8-byte aligned codes): a group of waves
 // owns 4 weight rows and every lane a 40-column window of them (8 packed
-// bytes per row), decoded through the LDS table and reused for both code
+// bytes per row), decoded through the LDS table and reused for up to 4 code
 // rows: 10 v_dot4_i32_i8 per row and code row, then exact integer
 // wave sums (DPP) and the same epilogue.  K is walked in chunks of 2560
 // columns (512 packed bytes) shared by the group's waves.  Bound by the
@@ -1052,13 +1052,21 @@ static int launch_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
 // would waste most of their columns.
 constexpr int kGvRows = 4;     // weight rows per wave group
 constexpr int kGvChunk = 2560; // columns per lane-window sweep (64 lanes x 40)
-// One code row; two of them for few weight rows and long K, and below the skinny
-// kernel's 16 columns.  Measured against the skinny kernel, graph replays: 2560 x
-// 2 x 2560 4.2 against 4.5 us, x 6912 6.8 against 8.5, but x 1024 4.7 against 4.0,
-// and 6912 x 2 x 2560 5.2 against 4.7, x 6912 9.2 against 7.5; 2560 x 4 x 6912 9.0
-// against 8.1.
+// One code row; more of them where the weight rows are few, K is long enough to
+// leave the skinny kernel's waves several blocks each, and the chunks are filled.
+// Measured against the skinny kernel, graph replays, us: two codes 2560 x 2560 4.2
+// against 4.5, 4800 x 6912 7.7 against 8.6, 8000 x 5120 6.3 against 6.8, x 9000 9.1
+// against 10.3, but 2560 x 1024 4.7 against 4.0, 8000 x 4096 7.5 against 6.9, x 6912
+// 10.2 against 8.6; three 1000 x 6912 6.7 against 8.3, 300 x 5120 5.8 against 6.4,
+// but x 4104 7.5 against 6.5; four 2560 x 6912 9.0 against 8.1.  Below the skinny
+// kernel's 16 columns the 128 x 128 kernel is the other one: 6912 x 3 x 8 7.3 against
+// 13.7, x 8 13.3 against 13.7, 100000 x 3 42 against 26.
 static bool small_n_wins(uint64_t m, uint64_t n, uint64_t k) {
-    return n == 1 || (n == 2 && ((m <= 4096 && k > 2048) || k < 16));
+    if (n == 1) return true;
+    if (k < 16) return n == 2 || (n <= 8 && m <= 8192);
+    if (n == 2 && k > 2048)
+        return m <= 5120 || (m <= 8192 && (k <= 2560 || (k > 4096 && k <= 5120) || k > 7680));
+    return n <= 4 && m <= 1024 && k > 4608;
 }
 
 __device__ __forceinline__ int32_t wave_sum_i32(int32_t v) {
@@ -3856,10 +3864,12 @@ static int ternary_i8_launch(const TernArgs& p, hipStream_t s) {
         const bool al8 = kp % 8 == 0 && (reinterpret_cast<uintptr_t>(p.a) & 7u) == 0;
         if (al8) {
             if (n <= 1) launch_gemv<1, true>(p, m, k, s);
-            else launch_gemv<2, true>(p, m, k, s);
+            else if (n <= 2) launch_gemv<2, true>(p, m, k, s);
+            else launch_gemv<4, true>(p, m, k, s);
         } else {
             if (n <= 1) launch_gemv<1, false>(p, m, k, s);
-            else launch_gemv<2, false>(p, m, k, s);
+            else if (n <= 2) launch_gemv<2, false>(p, m, k, s);
+            else launch_gemv<4, false>(p, m, k, s);
         }
         return launch_status();
     }

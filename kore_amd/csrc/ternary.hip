@@ -1057,16 +1057,16 @@ constexpr int kGvChunk = 2560; // columns per lane-window sweep (64 lanes x 40)
 // Measured against the skinny kernel, graph replays, us: two codes 2560 x 2560 4.2
 // against 4.5, 4800 x 6912 7.7 against 8.6, 8000 x 5120 6.3 against 6.8, x 9000 9.1
 // against 10.3, but 2560 x 1024 4.7 against 4.0, 8000 x 4096 7.5 against 6.9, x 6912
-// 10.2 against 8.6; three 1000 x 6912 6.7 against 8.3, 300 x 5120 5.8 against 6.4,
-// but x 4104 7.5 against 6.5; four 2560 x 6912 9.0 against 8.1.  Below the skinny
+// 10.2 against 8.6, while 18673 x 2560 is 6.9 against 7.8; three 1000 x 6912 6.7 against 8.3, 300 x 5120 5.8 against 6.4,
+// but x 4104 7.5 against 6.5; 1188 x 4 x 8848 9.2 against 10.6; four 2560 x 6912 9.0 against 8.1.  Below the skinny
 // kernel's 16 columns the 128 x 128 kernel is the other one: 6912 x 3 x 8 7.3 against
 // 13.7, x 8 13.3 against 13.7, 100000 x 3 42 against 26.
 static bool small_n_wins(uint64_t m, uint64_t n, uint64_t k) {
     if (n == 1) return true;
     if (k < 16) return n == 2 || (n <= 8 && m <= 8192);
     if (n == 2 && k > 2048)
-        return m <= 5120 || (m <= 8192 && (k <= 2560 || (k > 4096 && k <= 5120) || k > 7680));
-    return n <= 4 && m <= 1024 && k > 4608;
+        return m <= 5120 || (k <= 2560 && m <= 49152) || (m <= 8192 && ((k > 4096 && k <= 5120) || k > 7680));
+    return n <= 4 && k > 4608 && m <= (k > 7680 ? 2048u : 1024u);
 }
 
 __device__ __forceinline__ int32_t wave_sum_i32(int32_t v) {
@@ -3830,12 +3830,17 @@ using namespace kore;
 // 25 against 67, but x 6912 117 against 114; 50257 x 64 x 2560 32 against 28; up to
 // 512 columns from 40960: 50257 x 33 x 160 9.0 against 12.6), and 65-128 codes
 // from 28672 (32768 x 65 x 512 13.8 against 18.8, x 2560 27.4 against 30.2, but x
-// 6912 69 against 60; 24576 x 65 x 2560 27.3 against 25.1).
+// 6912 69 against 60; 24576 x 65 x 2560 27.3 against 25.1).  Few K steps leave its
+// waves little but the stores, so there it goes at 128 tiles (4096 x 1000 x 144 11.7
+// against 17.0, 6912 x 300 x 320 11.3 against 13.9, x 960 16.0 against 16.6, x 1280
+// 18.6 against 17.5; 2048 x 1024 x 144 10.4 against 9.8).
 constexpr uint64_t kSkLongK = 5120;
 static bool skinny_wins(uint64_t m, uint64_t n, uint64_t k, bool vec) {
     if (n <= 32) return true;
     if (vec && k <= kSkLongK && n <= 128 && m > (n > 64 ? 28672u : k <= 512 ? 40960u : 57344u)) return false;
-    return n <= 64 || ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN) <= 256;
+    if (n <= 64) return true;
+    const uint64_t tiles = ((m + kTmM - 1) / kTmM) * ((n + kTmN - 1) / kTmN);
+    return tiles <= (vec && k <= 960 && m > (uint64_t)kTmM ? 128 : 256);
 }
 
 static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
@@ -3843,7 +3848,12 @@ static int ternary_i8_skinny(const TernArgs& p, bool aligned_a, hipStream_t s) {
     // 32 x 32 outputs a workgroup of 8 waves while that is up to two a CU (more
     // of them, shorter; 2560 x 45 x 6912 8.8 us against 11.7 with 32 x 64, 3712
     // x 100 x 2375 10.0 against 12.6 with 64 x 64);
-    if (m32 * n32 <= 2 * kCus) return launch_skinny<1, 1, 8>(p, aligned_a, s);
+    if (m32 * n32 <= 2 * kCus) {
+        // (two workgroups a CU and more than two blocks a wave: 32 x 64, 6912 x 33 x
+        // 3696 8.7 against 9.3, x 4096 8.8 against 9.3)
+        if (n32 == 2 && m32 * n32 > kCus && p.k > 2560) return launch_skinny<1, 2, 8>(p, aligned_a, s);
+        return launch_skinny<1, 1, 8>(p, aligned_a, s);
+    }
     if (n64 == 1 && (n32 == 1 || p.k <= kSkLongK)) {
         // then one to two code tiles of 32, each with 32 weight rows and 4 waves
         // (24576 x 32 x 2560 9.8 against 11.2 with 8; 14336 x 64 x 512 6.1 against

@@ -31,10 +31,11 @@ def at(arr: np.ndarray, offset: int) -> HipBuffer:
 FORMS = [(5, 1, 15, 0, 0), (5, 1, 16, 0, 0), (33, 1, 17, 1, 1), (7, 2, 8, 0, 0), (64, 2, 2048, 0, 0), (64, 2, 2056, 0, 0),
          (5120, 2, 2064, 0, 0), (5121, 2, 2064, 0, 0), (5121, 2, 2568, 0, 0), (8192, 2, 4104, 0, 1), (8193, 2, 4104, 0, 0),
          (5121, 2, 7680, 0, 0), (5121, 2, 7688, 0, 3), (1024, 4, 4616, 0, 0), (1025, 4, 4616, 0, 0), (1023, 3, 4616, 0, 1),
-         (9, 4, 9000, 0, 2), (64, 3, 4608, 0, 0), (8192, 7, 8, 0, 0), (8193, 8, 8, 0, 0), (31, 3, 8, 0, 1),
+         (9, 4, 9000, 0, 2), (2048, 4, 7688, 0, 0), (2049, 3, 7688, 0, 0), (64, 3, 4608, 0, 0), (8192, 7, 8, 0, 0), (8193, 8, 8, 0, 0), (31, 3, 8, 0, 1),
          (7, 2, 2563, 3, 2), (300, 3, 2560, 0, 0), (129, 8, 2568, 0, 0), (31, 32, 31, 5, 3),
          (32, 33, 159, 0, 0), (65, 33, 160, 0, 0), (64, 31, 161, 9, 1), (97, 40, 1001, 7, 0), (6657, 45, 175, 15, 3),
-         (8192, 64, 320, 0, 0), (8193, 64, 320, 0, 0), (16384, 40, 163, 3, 1), (16385, 64, 176, 0, 0), (8200, 45, 1040, 0, 1),
+         (8192, 64, 320, 0, 0), (8193, 64, 320, 0, 0), (4128, 45, 2576, 0, 1), (8192, 64, 2561, 3, 0), (8224, 64, 2576, 0, 0), (49152, 2, 2056, 0, 0),
+         (49153, 2, 2056, 0, 1), (16384, 40, 163, 3, 1), (16385, 64, 176, 0, 0), (8200, 45, 1040, 0, 1),
          (16385, 9, 161, 0, 0), (65504, 5, 33, 1, 0), (65505, 32, 48, 0, 2), (40960, 33, 48, 0, 0), (40961, 33, 48, 0, 0),
          (57344, 33, 528, 0, 0), (57345, 33, 528, 0, 0), (57345, 40, 33, 2, 1), (8224, 33, 5136, 0, 0), (28672, 65, 32, 0, 0), (28673, 65, 32, 0, 3), (28673, 70, 37, 1, 0),
          (4096, 65, 163, 0, 0), (8200, 65, 336, 0, 0), (8192, 100, 164, 2, 1), (1024, 1000, 177, 0, 0),
@@ -60,7 +61,7 @@ def test_ternary_i8_forms(m, n, k, oq, oa):
 # 256 x 128 tiles from just past the skinny kernel's range: one and several K steps, more of them than the
 # two-workgroup form takes on larger outputs, ragged in every dimension, packed rows at each byte offset; one tile column
 # where there are 144 tiles of 256 x 256 too.
-@pytest.mark.parametrize("m,n,k,oa", [(4100, 1025, 16, 0), (4097, 1030, 176, 1), (2600, 1700, 2736, 0), (2570, 1665, 4112, 3),
+@pytest.mark.parametrize("m,n,k,oa", [(4100, 1025, 16, 0), (2048, 1025, 960, 0), (2048, 1024, 960, 1), (2049, 1023, 960, 0), (2049, 1024, 976, 0), (4097, 1030, 176, 1), (2600, 1700, 2736, 0), (2570, 1665, 4112, 3),
                                       (4101, 1026, 176, 0), (4102, 1027, 336, 2), (4103, 1028, 16, 0),
                                       (6912, 601, 2560, 0), (129, 33000, 336, 2), (128, 33000, 176, 0), (36900, 65, 1296, 1),
                                       (36900, 128, 16, 0)])

@@ -19,7 +19,7 @@
  *     matmuls read and write unaligned rows through their vector kernels;
  *     element-wise ops, RoPE and the gather take a scalar path for unaligned
  *     pointers, with identical results.  One thread per row, column or output
- *     remains for norm rows of more than 16384 columns and short ones (up to 32
+ *     remains for norm rows of more than 16384 columns and short ones (up to 48
  *     columns), for the RMSNorm backward's grad_gamma with more than 16384
  *     columns or few rows, and for a ternary matmul whose output is not 4-byte
  *     aligned or whose K is 0.

@@ -805,18 +805,22 @@ static int launch_sl4(NormArgs a, uint32_t nch, RowForm form, hipStream_t s) {
 // 1000 x 7 3.2 against 3.6.  From 8 columns (pre-quant 4) the rows have to fill the
 // chip, and the row counts where the two meet lie on a line (ragged 3500 x 10 4.0
 // against 4.5, but 1000 x 8 3.8 against 3.3; 10000 x 17 6.0 against 7.4, 20000 x 28 9.5
-// against 11.7, but 16000 x 32 11.4 against 9.8; whole rows, which a wave reads with
-// fewer instructions, later: 3500 x 8 3.9 against 3.7).  Past 20 columns they have to
-// stay in the caches, as a wave's lanes read 64 rows at a time (200000 x 24 102
-// against 76, pre-quant 60 against 98; 250000 x 17 63 against 103); whole rows past
-// 16 never gain (120000 x 32 79 against 48).
+// against 11.7, 30000 x 42 15 against 18, but 16000 x 42 13 against 11; whole rows,
+// which a wave reads with fewer instructions, later: 3500 x 8 3.9 against 3.7).  Past
+// 20 columns they have to stay in the caches, as a wave's lanes read 64 rows at a
+// time (250000 x 17 63 against 103, but 200000 x 24 102 against 76; 60000 x 42 28
+// against 32, 80000 x 33 49 against 39; pre-quant 200000 x 24 60 against 98, 80000 x
+// 38 43 against 45, x 42 49 against 45; gate 45000 x 33 24 against 28, 60000 x 33 39
+// against 35); ragged rows past 48 (gate 32) and whole ones past 16 never gain
+// (45000 x 50 25 against 25; 120000 x 32 79 against 48).
 template <NormOut Out>
 static bool thread_a_row(uint64_t rows, uint64_t cols, bool whole) {
     constexpr bool kCodes = Out == NormOut::I8;
     if (cols <= (kCodes ? 3u : 7u)) return true;
-    if (rows < 512 || cols > (whole ? 16u : 32u)) return false;
+    constexpr bool kGate = Out == NormOut::SiluGate;
+    if (rows < 512 || cols > (whole ? 16u : kGate ? 32u : 48u)) return false;
     if (whole ? rows + 3600 < 1000 * cols : rows + 1600 < 600 * cols) return false;
-    return cols <= 20 || rows * cols <= (kCodes ? 1ull << 23 : 1ull << 22);
+    return cols <= 20 || rows * cols <= (kGate ? 3u << 19 : !kCodes ? 5u << 19 : cols <= 32 ? 1u << 23 : 3u << 20);
 }
 
 template <NormOut Out>

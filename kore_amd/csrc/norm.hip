@@ -810,8 +810,8 @@ static int launch_sl4(NormArgs a, uint32_t nch, RowForm form, hipStream_t s) {
 // 20 columns they have to stay in the caches, as a wave's lanes read 64 rows at a
 // time (250000 x 17 63 against 103, but 200000 x 24 102 against 76; 60000 x 42 28
 // against 32, 80000 x 33 49 against 39; pre-quant 200000 x 24 60 against 98, 80000 x
-// 38 43 against 45, x 42 49 against 45; gate 45000 x 33 24 against 28, 60000 x 33 39
-// against 35); ragged rows past 48 (gate 32) and whole ones past 16 never gain
+// 38 43 against 45, x 42 49 against 45; gate 120000 x 21 44 against 63, 60000 x 31 33
+// against 36, 80000 x 31 no faster); ragged rows past 48 (gate 32) and whole ones past 16 never gain
 // (45000 x 50 25 against 25; 120000 x 32 79 against 48).
 template <NormOut Out>
 static bool thread_a_row(uint64_t rows, uint64_t cols, bool whole) {
@@ -820,7 +820,8 @@ static bool thread_a_row(uint64_t rows, uint64_t cols, bool whole) {
     constexpr bool kGate = Out == NormOut::SiluGate;
     if (rows < 512 || cols > (whole ? 16u : kGate ? 32u : 48u)) return false;
     if (whole ? rows + 3600 < 1000 * cols : rows + 1600 < 600 * cols) return false;
-    return cols <= 20 || rows * cols <= (kGate ? 3u << 19 : !kCodes ? 5u << 19 : cols <= 32 ? 1u << 23 : 3u << 20);
+    if (cols <= 24) return cols <= 20 || rows * cols <= (kCodes ? 1u << 23 : 3u << 20);
+    return rows <= (kCodes && cols <= 38 ? 98304u : 65536u);
 }
 
 template <NormOut Out>

@@ -179,8 +179,8 @@ def test_softmax_long_and_ragged_nonfinite_rows(cols):
 # many of up to 48 columns.
 NORM_LENGTHS = [(3, 1, 1), (5, 6, 3), (65, 3, 1), (70, 4, 0), (66, 7, 2), (511, 4, 0), (512, 4, 0), (4400, 8, 0),
                 (4399, 8, 0), (3200, 8, 1), (3199, 9, 1), (12400, 16, 0), (12399, 16, 0), (8600, 17, 3), (17600, 32, 1),
-                (17600, 32, 0), (18200, 33, 2), (18199, 33, 2), (26000, 46, 1), (28000, 49, 3), (54700, 48, 1),
-                (66000, 24, 3), (300, 255, 2), (7, 1021, 1), (9, 1537, 0), (260, 2561, 3), (300, 3071, 0),
+                (17600, 32, 0), (18200, 33, 2), (18199, 33, 2), (26000, 46, 1), (28000, 49, 3), (65536, 25, 1),
+                (65537, 25, 1), (98304, 25, 2), (98305, 25, 2), (140000, 24, 3), (300, 255, 2), (7, 1021, 1), (9, 1537, 0), (260, 2561, 3), (300, 3071, 0),
                 (5, 3072, 0), (300, 3073, 0), (3, 3076, 0), (2, 4095, 2), (3, 4096, 1), (300, 4097, 0), (2, 4100, 0), (5, 5119, 1), (270, 5120, 0), (3, 6144, 0),
                 (300, 6912, 0), (3, 6915, 2), (2, 7168, 0), (4, 7172, 0), (300, 8192, 0), (3, 8191, 3), (2, 8193, 0),
                 (2, 9000, 0), (3, 10240, 0), (2, 12285, 1), (3, 12288, 0), (259, 14336, 0), (2, 16383, 2),
